@@ -503,13 +503,25 @@ int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int 
  * then with trp[ntiles+1], tcp[ntiles+1], tcols[tcp[ntiles]], lcol[nnz]. */
 int nmg_tiling_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int max_nodes, int64_t *ntiles,
                     int *max_used, int64_t *trp, int64_t *tcp, int32_t *tcols, uint16_t *lcol);
+/* The node tiles of a node pattern (nb rows, columns < nb) as the LDS-staged
+ * products of nmgpu_tiles.hip use them, computed on the host only (no
+ * reference counterpart; no device use): tiles of at most `rows` rows (a
+ * multiple of 16) and `cap` nodes, `waves` wavefronts per tile, quads stored
+ * singly (pack 1) or in pairs (2).  sizes[6]: tiles (0: the pattern does not
+ * fit), quads, list entries, slices per tile, longest list, partial sums of a
+ * tile.  Then with units[8*waves*tiles] (list, nodes, row0, own, q0, nq,
+ * slice, part | parts << 8 | slot << 16), lists, lrow[16*slices],
+ * eidx[64*quads] and perm[64*quads]; null pointers are skipped. */
+int nmg_node_tiles_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int rows, int cap, int waves, int pack,
+                        int64_t *sizes, int32_t *units, int32_t *lists, uint16_t *lrow, uint16_t *eidx, int32_t *perm);
 /* Autotuner (no reference counterpart): times the product layouts of mat for
  * K columns on the device (lanes per row; rows per wavefront; LDS tiles with
  * capacities on a geometric ladder up to 64 KB, workgroups of 1024 or 256
  * threads; for K = 1 also row groups) and keeps the fastest.  kind: 0
  * lanes-per-row, 1 rows per wavefront, 2 tiled, 3 row groups, 4 wide,
  * 5 tiled wide (4 and 5: scalar mass, K >= 2), 6 pipelined lanes-per-row
- * (3x3 blocks, K = 1); rows: lanes per row (kinds 0, 4, 5), rows per
+ * (3x3 blocks, K = 1), 7 the default route (node tiles, or the row kernels
+ * for small matrices); rows: lanes per row (kinds 0, 4, 5), rows per
  * wavefront (1, 2), groups per wavefront (3) or rows per lane group (6);
  * cap: tile node capacity (kinds 2, 5) or lanes per group (6); threads:
  * tile workgroup size (kind 2). */

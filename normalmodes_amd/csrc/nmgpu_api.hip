@@ -138,6 +138,12 @@ void DevMat::release() {
   dfree(bcol);
   dfree(bval);
   dfree(bval32);
+  for (TileSet& t : tset) {
+    t.use.store(nullptr);
+    t.plan.reset();
+    dfree(t.val);
+    dfree(t.val32);
+  }
 }
 DevMat::~DevMat() { release(); }
 
@@ -409,6 +415,7 @@ DevMat* clone_devmat(const DevMat& S, hipStream_t s) {
     if (S.tiling[i])
       build_tiling(*M, 1 << i, S.tiling[i]->cap, S.tiling[i]->rows_per_wave, S.tiling[i]->block, S.tiling[i]->wide);
   if (S.rgroups) build_row_groups(*M, S.rgroups->per_wave);
+  for (int i = 0; i < 2; ++i) M->tset[i].plan = S.tset[i].plan;  // in use once build_tiles has filled the values
   return M.release();
 }
 
@@ -2348,6 +2355,7 @@ int nmg_set_amv_dad(nmg_handle h, nmg_handle matA, const double* d) {
     dd.ensure(S->n);
     NMG_HIP(hipMemcpyAsync(dd.p, d, sizeof(double) * S->n, hipMemcpyHostToDevice, S->s));
     scale_devmat(*C, dd.p, dd.p, 1.0, S->s);
+    build_tiles(*C, S->s);
     NMG_HIP(hipStreamSynchronize(S->s));
     S->adad = std::move(C);
     S->amat = nullptr;
@@ -2376,6 +2384,7 @@ int nmg_set_amv_fs(nmg_handle h, nmg_handle matAd, nmg_handle matE, nmg_handle m
       NMG_CHECK(std::isfinite(d[i]) && d[i] > 0.0, NMG_EINVAL, "scaling vector must be positive");
     for (int64_t i = 0; i < np; ++i)
       NMG_CHECK(std::isfinite(dp[i]) && dp[i] > 0.0, NMG_EINVAL, "pressure scaling vector must be positive");
+    build_tiles(*F->Ad, S->s);
     F->n = n;
     F->np = np;
     F->d.ensure(n);
@@ -2480,6 +2489,7 @@ int nmg_setup_chebiter(double lmin, double lmax, int deg, nmg_handle mat, nmg_ha
               "chebiter needs 0 < lmin < lmax (an SPD matrix)");
     NMG_CHECK(deg >= 1 && deg <= 100000, NMG_EINVAL, "chebiter degree must be >= 1");
     NMG_CHECK(M->nrow == M->ncol, NMG_EINVAL, "chebiter needs a square matrix");
+    build_tiles(*M, default_stream());
     Cheb* C = new Cheb();
     C->mat = M;
     C->lmin = lmin;
@@ -3135,6 +3145,17 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   // another width leaves it as it is)
   build_tiling(M, K, 0, 1);
   M.wide[idx] = 0;
+  M.block_map[idx] = 0;
+  if (K == 1) {
+    M.single_blocked = false;
+    M.pipe = 0;
+    M.group = 0;
+    build_row_groups(M, 0);
+  }
+  build_tiles(M, s);
+  if (M.tset[0].use.load())
+    consider(time_launches(s, reps, [&] { K == 1 ? k_spmv(M, x.p, y.p, s, fp32) : k_block_spmv(K, M, x.p, y.p, s, fp32); }),
+             7, 0, 0, 0, 0);
   if (M.layout == L_MASS3 && K >= 2 && K <= 16) {
     for (int G : {4, 8, 16, 32}) {
       M.wide[idx] = G;
@@ -3198,7 +3219,9 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   // apply the winner
   build_tiling(M, K, 0, 1);
   M.block_map[idx] = 0;
-  if (best.kind == 0) {
+  if (best.kind == 7) {
+    // no explicit layout: the node tiles
+  } else if (best.kind == 0) {
     M.group = best.group;
   } else if (best.kind == 6) {
     M.group = best.group;
@@ -3313,6 +3336,32 @@ int nmg_tiling_host(int64_t nb, const int64_t* rowptr, const int32_t* col, int m
     if (tcp) std::memcpy(tcp, H.tcp.data(), sizeof(int64_t) * H.tcp.size());
     if (tcols) std::memcpy(tcols, H.tcols.data(), sizeof(int32_t) * H.tcols.size());
     if (lcol) std::memcpy(lcol, H.lcol.data(), sizeof(uint16_t) * H.lcol.size());
+  });
+}
+
+int nmg_node_tiles_host(int64_t nb, const int64_t* rowptr, const int32_t* col, int rows, int cap, int waves, int pack,
+                        int64_t* sizes, int32_t* units, int32_t* lists, uint16_t* lrow, uint16_t* eidx, int32_t* perm) {
+  return guarded([&] {
+    NMG_CHECK(nb > 0 && rowptr && col && sizes, NMG_EINVAL, "null pattern");
+    NMG_CHECK(rows > 0 && rows % kSliceRows == 0 && cap > 0 && waves > 0 && (pack == 1 || pack == 2), NMG_EINVAL,
+              "rows must be a multiple of 16, cap and waves positive, pack 1 or 2");
+    HostTiles H;
+    const bool ok = tile_layout(nb, rowptr, col, rows, cap, waves, pack, H);
+    sizes[0] = ok ? H.ntiles : 0;
+    sizes[1] = ok ? H.quads : 0;
+    sizes[2] = ok ? (int64_t)H.tcols.size() : 0;
+    sizes[3] = ok ? H.spt : 0;
+    sizes[4] = ok ? H.max_nodes : 0;
+    sizes[5] = ok ? H.max_extra : 0;
+    if (!ok) return;
+    auto out = [](auto* to, const auto& v) {
+      if (to) std::memcpy(to, v.data(), sizeof(v[0]) * v.size());
+    };
+    if (units) std::memcpy(units, H.un.data(), sizeof(TileUnit) * H.un.size());
+    out(lists, H.tcols);
+    out(lrow, H.lrow);
+    out(eidx, H.eidx);
+    out(perm, H.perm);
   });
 }
 

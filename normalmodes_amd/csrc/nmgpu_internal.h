@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -66,6 +67,43 @@ struct RowGroups {
   ~RowGroups();
 };
 
+// Node tiles of a square BSR3 / MASS3 matrix (nmgpu_tiles.hip).
+constexpr int kSliceRows = 16;  // rows of a slice, four lanes each
+// one wavefront's share of a tile: the tile's node list and rows, and a run of
+// quads (four entries of each row) of one slice
+struct TileUnit {
+  int list, nodes;  // first list entry, entries
+  int row0, own;    // first row of the tile, its place in the list (own rows are consecutive there)
+  int q0, nq;       // first quad, quads
+  int slice;        // -1: none
+  int part;         // part | parts << 8 | slot of the slice's first partial sum << 16
+};
+struct HostTiles {
+  int64_t ntiles = 0, quads = 0;
+  int spt = 0, max_nodes = 0, max_extra = 0;
+  std::vector<TileUnit> un;          // per tile and wavefront
+  std::vector<int32_t> tcols;        // node lists, ascending
+  std::vector<uint16_t> lrow, eidx;  // row of each slice place within its tile (0xffff: none); entries' list places
+  std::vector<int32_t> perm;         // entry of each slot (-1: padding)
+};
+struct TilePlan {
+  int64_t ntiles = 0, quads = 0;
+  int max_nodes = 0, max_extra = 0;
+  TileUnit* un = nullptr;
+  int32_t* tcols = nullptr;
+  uint16_t* lrow = nullptr;
+  uint16_t* eidx = nullptr;
+  int32_t* perm = nullptr;
+  ~TilePlan();
+};
+
+struct TileSet {
+  std::shared_ptr<const TilePlan> plan;        // the pattern, shared by copies of a matrix
+  std::atomic<const TilePlan*> use{nullptr};   // set once the values are in place
+  double* val = nullptr;                       // values in the tiles' order, and their FP32 copy
+  float* val32 = nullptr;
+};
+
 // Process-wide source of layout generations (unique across matrices, so a
 // matrix freed and re-created at the same address never repeats one).
 inline uint64_t next_layout_gen() {
@@ -116,6 +154,17 @@ struct DevMat {
     if (layout == L_CSR) return nnz;
     if (layout == L_MASS3) return nbnz;
     return tiled_vals ? 9 * ((nbnz + 63) / 64 * 64) : 9 * nbnz;
+  }
+  // node tiles (nmgpu_tiles.hip): [0] for up to 48 staged bytes per node, [1]
+  // for more (unset when both are cut alike)
+  TileSet tset[2];
+  // whether K-column products take the node tiles: a layout set or tuned
+  // explicitly for that width comes first
+  bool tile_use(int K) const {
+    if (K == 1 && (group > 0 || pipe > 0 || rgroups || single_blocked)) return false;
+    for (int i = 0; i < 7; ++i)
+      if ((1 << i) == K) return block_map[i] == 0 && !tiling[i] && wide[i] == 0;
+    return false;
   }
   std::vector<int64_t> h_browptr;  // host copy of the node pattern (tiling)
   std::vector<int32_t> h_bcol;
@@ -176,6 +225,21 @@ void scale_devmat(DevMat& M, const double* dl, const double* dr, double sign, hi
 void diag_devmat(const DevMat& M, double* d, hipStream_t s);
 // refresh float copies of the values
 void make_fp32(DevMat& M, hipStream_t s);
+
+// node tiles (nmgpu_tiles.hip): host layout, plan and values; the products
+// return false when M takes another route
+bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int cap, int waves, int pack,
+                 HostTiles& H);
+void build_tiles(DevMat& M, hipStream_t s);
+// (re)writes the FP32 tile values, and with fp64 (or when new) the FP64 ones
+void fill_tile_values(DevMat& M, hipStream_t s, bool fp64);
+bool k_tile_spmv(int K, const DevMat& M, const double* x, double* y, hipStream_t s, bool fp32);
+bool k_tile_cheb_step(int K, const DevMat& M, const double* b, const double* xk, double* xm, double w, double ith,
+                      hipStream_t s, bool fp32);
+bool k_tile_cheb_step32(int K, const DevMat& M, const float* b, const float* xk, float* xm, double w, double ith,
+                        hipStream_t s, bool fp32);
+bool k_tile_filter_step(int K, const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
+                        const double* mu, double mu0, double t, double cc, bool first, hipStream_t s, bool fp32);
 
 // ---------------------------------------------------------------------------
 // kernel launchers (nmgpu_kernels.hip); all asynchronous on stream s

@@ -14,31 +14,13 @@
 // Chebyshev B-solve and of the polynomial filter are fused into the same pass.
 #include <hip/hip_cooperative_groups.h>
 
+#include "nmgpu_device.h"
 #include "nmgpu_internal.h"
 
 namespace nmg {
 
 constexpr int kBlock = 256;
 constexpr int kDotBlocks = 512;
-constexpr int kXcd = 8;  // accelerator complex dies (XCDs) of an MI355X
-
-// Kernel flags of the sparse products: bit 0 XCD-contiguous workgroup order,
-// bit 1 non-temporal (streaming) loads of the matrix values and indices.
-// Workgroup b of a launch runs on XCD b % 8 (round-robin dispatch).  With
-// bit 0 set the logical block index gives each XCD one contiguous range,
-// so neighbouring node rows -- which gather the same x entries -- share one
-// XCD's L2 instead of being spread over eight.  A bijection of [0, grid).
-__device__ __forceinline__ int64_t xcd_block(int flags) {
-  const int64_t b = blockIdx.x;
-  if (!(flags & 1)) return b;
-  const int64_t n = gridDim.x, q = n / kXcd, r = n % kXcd;
-  const int64_t x = b % kXcd, i = b / kXcd;
-  return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
-}
-// position of value q of BSR3 entry k (planes, or tiles of 64 entries)
-__device__ __forceinline__ int64_t bidx(int64_t k, int q, int64_t nbnz, int flags) {
-  return (flags & 4) ? ((k >> 6) * 576 + (int64_t)q * 64 + (k & 63)) : ((int64_t)q * nbnz + k);
-}
 // matrix loads: streamed once per product, so with bit 1 they are issued as
 // non-temporal loads that do not displace the gathered x from the caches
 template <class T>
@@ -509,12 +491,14 @@ static void dispatch(const DevMat& M, const double* x, Epi epi, hipStream_t s, b
 }
 
 void k_spmv(const DevMat& M, const double* x, double* y, hipStream_t s, bool fp32) {
+  if (k_tile_spmv(1, M, x, y, s, fp32)) return;
   if (M.single_blocked && !M.rgroups) return k_block_spmv(1, M, x, y, s, fp32);
   dispatch(M, x, EpiStore{y}, s, fp32);
 }
 
 void k_cheb_step(const DevMat& M, const double* b, const double* xk, double* xm, double w,
                  double ith, hipStream_t s, bool fp32) {
+  if (k_tile_cheb_step(1, M, b, xk, xm, w, ith, s, fp32)) return;
   if (M.single_blocked && !M.rgroups) return k_block_cheb_step(1, M, b, xk, xm, w, ith, s, fp32);
   dispatch(M, xk, EpiCheb{b, xk, xm, w, ith}, s, fp32);
 }
@@ -958,6 +942,7 @@ void scale_devmat(DevMat& M, const double* dl, const double* dr, double sign, hi
   }
   NMG_HIP(hipGetLastError());
   if (M.val32 || M.bval32) make_fp32(M, s);
+  fill_tile_values(M, s, true);
 }
 
 __global__ void csr_diag_k(int64_t nrow, const int64_t* rp, const int32_t* ci, const double* v, double* d) {
@@ -1021,6 +1006,7 @@ void make_fp32(DevMat& M, hipStream_t s) {
     hipLaunchKernelGGL(to_f32_k, dim3(grid_for(nv)), dim3(kBlock), 0, s, nv, M.bval, M.bval32);
   }
   NMG_HIP(hipGetLastError());
+  fill_tile_values(M, s, false);
 }
 
 }  // namespace nmg
@@ -1441,20 +1427,24 @@ static void dispatch_block(const DevMat& M, const XT* x, Epi epi, hipStream_t s,
 
 void k_filter_step(const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
                    double t, double cc, double mu, bool first, hipStream_t s, bool fp32) {
+  if (k_tile_filter_step(1, A, x, vk, vkm, y, nullptr, mu, t, cc, first, s, fp32)) return;
   dispatch(A, x, EpiFilter{vk, vkm, y, t, cc, mu, first ? 1 : 0}, s, fp32);
 }
 
 void k_block_spmv(int K, const DevMat& M, const double* x, double* y, hipStream_t s, bool fp32) {
+  if (k_tile_spmv(K, M, x, y, s, fp32)) return;
   NMG_BLOCK_SWITCH(K, (dispatch_block<KK>(M, x, BEpiStore<KK>{y}, s, fp32)));
 }
 
 void k_block_cheb_step(int K, const DevMat& M, const double* b, const double* xk, double* xm, double w,
                        double ith, hipStream_t s, bool fp32) {
+  if (k_tile_cheb_step(K, M, b, xk, xm, w, ith, s, fp32)) return;
   NMG_BLOCK_SWITCH(K, (dispatch_block<KK>(M, xk, BEpiCheb<KK>{b, xk, xm, w, ith}, s, fp32)));
 }
 
 void k_block_cheb_step32(int K, const DevMat& M, const float* b, const float* xk, float* xm, double w,
                          double ith, hipStream_t s, bool fp32) {
+  if (k_tile_cheb_step32(K, M, b, xk, xm, w, ith, s, fp32)) return;
   NMG_BLOCK_SWITCH(K, (dispatch_block<KK>(M, xk, BEpiCheb32<KK>{b, xk, xm, w, ith}, s, fp32)));
 }
 
@@ -1501,6 +1491,7 @@ void k_f32_to_f64(int64_t n, const float* x, double* y, hipStream_t s) {
 
 void k_block_filter_step(int K, const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
                          const double* mu, double t, double cc, bool first, hipStream_t s, bool fp32) {
+  if (k_tile_filter_step(K, A, x, vk, vkm, y, mu, 0.0, t, cc, first, s, fp32)) return;
   NMG_BLOCK_SWITCH(K, (dispatch_block<KK>(A, x, BEpiFilter<KK>{vk, vkm, y, mu, t, cc, first ? 1 : 0}, s, fp32)));
 }
 

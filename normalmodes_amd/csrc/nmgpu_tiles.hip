@@ -1,0 +1,711 @@
+// Node tiles: the products of the scalar-mass (MASS3) and 3x3-block (BSR3)
+// layouts with x staged in LDS and no reduction across a wavefront's rows.
+//
+// What bounds these products: every entry gathers the 3K values of its node,
+// 24K bytes against the 12 (MASS3) or 76 (BSR3) bytes of the entry itself.
+// Row kernels take them from the caches, 28 times per node; at 1.9M DoF that
+// traffic, at 6.5-7 TB/s, was the whole time of the k-column steps.  Here a
+// workgroup owns a tile of consecutive node rows (the numbering is spatially
+// local), reads each node it references once into LDS (3-4 times its own rows
+// instead of 28) and forms the rows from there.
+//
+// Rows of a tile are sorted by length and cut into slices of 16; four lanes
+// share a row.  A "quad" is the next four entries of each of the 16 rows: lane
+// 4r + e loads entry e of row r, values and 16-bit list places in unit stride
+// without row offsets, and hands them to the row's other lanes by DPP.  With
+// K >= 4 each of the four lanes owns one column (groups of four columns per
+// workgroup), so sums stay in their lane; with K = 2 and 1 the four lanes are
+// 2 columns x 2 and 1 x 4 entries, and one or two DPP additions close a row.
+// The row kernels' butterflies cost 24 LDS permutes per row at K = 4.
+//
+// Long slices (the vertex rows of P2 meshes hold 65 entries, edge rows 19-27)
+// are split over several wavefronts with partial sums in LDS added in a fixed
+// order, so that no wavefront carries more than about six quads: with one
+// wavefront per slice the longest one set the time of the tile.
+//
+// Measured (FP64 fused Chebyshev step, us; row kernels as the autotuner left
+// them in brackets; one MI355X):
+//   DoF        K = 1         K = 2         K = 4         K = 8         K = 16
+//   51.5k    4.1 (4.6)     4.7 (5.7)     5.7 (8.2)     8.3 (12.5)   15.6 (21.9)
+//   439k    14.7 (19.8)   17.0 (24.5)   24.4 (39.5)   38.0 (84.5)   79.8 (161)
+//   1.90M   52.3 (65.5)   67.7 (276)     107 (184)     213 (541)     460 (956)
+// (the 1.9M-DoF figures in brackets at K = 2, 8, 16 are the untuned ones).  At
+// 1.9M DoF the step moves 487 MB at K = 4 (counted): 4.5 TB/s, against 5.6 TB/s
+// of a copy of that size.  Loads wider than 8 bytes, lists read once per
+// wavefront and 64 registers (two workgroups of 16 wavefronts per CU) each
+// counted: with 8 wavefronts or spills the same step took 2-4 times as long.  A
+// persistent form with the next tile's x in registers was no faster (137 us at
+// K = 4), nor was an epilogue through LDS with contiguous stores (143 us).
+#include <algorithm>
+#include <initializer_list>
+#include <memory>
+#include <mutex>
+#include <numeric>
+#include <type_traits>
+#include <vector>
+
+#include "nmgpu_device.h"
+#include "nmgpu_internal.h"
+
+namespace nmg {
+
+TilePlan::~TilePlan() {
+  for (void* p : {(void*)un, (void*)tcols, (void*)lrow, (void*)eidx, (void*)perm})
+    if (p) (void)hipFree(p);
+}
+
+template <class T>
+static T* to_device(const std::vector<T>& v) {
+  T* p = nullptr;
+  NMG_HIP(hipMalloc(&p, sizeof(T) * std::max<size_t>(v.size(), 1)));
+  const hipError_t e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void)hipFree(p);
+    NMG_HIP(e);
+  }
+  return p;
+}
+
+bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int cap, int waves, int pack,
+                 HostTiles& H) {
+  const int spt = rows / kSliceRows;
+  if (spt < 1 || spt > waves) return false;  // one wavefront at least per slice
+  const int64_t nblk = (nb + rows - 1) / rows;
+  int64_t longest = 0;
+  for (int64_t r = 0; r < nb; ++r) longest = std::max(longest, rp[r + 1] - rp[r]);
+  if (longest + 1 > cap || cap > 65535 || rp[nb] > (int64_t)1 << 28 || nb > (int64_t)1 << 28) return false;
+  // cut every aligned run of `rows` rows where its node list would pass cap
+  struct Cut {
+    int64_t r0, r1;
+    std::vector<int32_t> nodes;
+  };
+  std::vector<std::vector<Cut>> blk(nblk);
+#pragma omp parallel
+  {
+    std::vector<int64_t> stamp(nb, -1);
+    std::vector<int32_t> fresh;
+    int64_t id = 0;
+#pragma omp for schedule(dynamic, 16)
+    for (int64_t b = 0; b < nblk; ++b) {
+      const int64_t end = std::min(nb, (b + 1) * rows);
+      Cut cur{b * rows, b * rows, {}};
+      for (int64_t r = b * rows; r < end;) {
+        fresh.clear();
+        auto see = [&](int32_t c) {
+          if (stamp[c] != id) {
+            stamp[c] = id;
+            fresh.push_back(c);
+          }
+        };
+        for (int64_t k = rp[r]; k < rp[r + 1]; ++k) see(ci[k]);
+        see((int32_t)r);  // the row's own x, for the epilogue
+        if ((int64_t)(cur.nodes.size() + fresh.size()) > cap) {
+          std::sort(cur.nodes.begin(), cur.nodes.end());
+          blk[b].push_back(std::move(cur));
+          cur = Cut{r, r, {}};
+          ++id;
+          continue;  // the row opens the next tile
+        }
+        cur.nodes.insert(cur.nodes.end(), fresh.begin(), fresh.end());
+        cur.r1 = ++r;
+      }
+      std::sort(cur.nodes.begin(), cur.nodes.end());
+      blk[b].push_back(std::move(cur));
+      ++id;
+    }
+  }
+  std::vector<const Cut*> cut;
+  for (auto& v : blk)
+    for (auto& c : v) cut.push_back(&c);
+  const int64_t nt = (int64_t)cut.size();
+  H.ntiles = nt;
+  H.spt = spt;
+  H.lrow.assign(nt * spt * kSliceRows, 0xffff);
+  std::vector<int64_t> first(nt + 1, 0);
+  H.max_nodes = 0;
+  for (int64_t t = 0; t < nt; ++t) {
+    first[t + 1] = first[t] + (int64_t)cut[t]->nodes.size();
+    H.max_nodes = std::max(H.max_nodes, (int)cut[t]->nodes.size());
+  }
+  H.tcols.resize(first[nt]);
+  std::vector<int2> sd(nt * spt, int2{0, 0});  // per slice {first quad, quads}
+  // rows of a tile in order of falling length, 16 to a slice
+#pragma omp parallel for schedule(dynamic, 16)
+  for (int64_t t = 0; t < nt; ++t) {
+    const Cut& c = *cut[t];
+    std::copy(c.nodes.begin(), c.nodes.end(), H.tcols.begin() + first[t]);
+    std::vector<int32_t> ord(c.r1 - c.r0);
+    std::iota(ord.begin(), ord.end(), (int32_t)c.r0);
+    std::stable_sort(ord.begin(), ord.end(),
+                     [&](int32_t a, int32_t b) { return rp[a + 1] - rp[a] > rp[b + 1] - rp[b]; });
+    for (size_t i = 0; i < ord.size(); ++i) {
+      const int64_t s = t * spt + (int64_t)(i / kSliceRows);
+      H.lrow[s * kSliceRows + i % kSliceRows] = (uint16_t)(ord[i] - c.r0);
+      if (i % kSliceRows == 0) {
+        const int nq = (int)((rp[ord[i] + 1] - rp[ord[i]] + 3) / 4);
+        sd[s].y = (nq + pack - 1) / pack * pack;
+      }
+    }
+  }
+  int64_t q = 0;
+  for (auto& s : sd) {
+    s.x = (int)q;
+    q += s.y;
+  }
+  if (q * 64 > (int64_t)1 << 30) return false;
+  H.quads = q;
+  // work units: the slices of a tile cut into runs of at most m quads, m the
+  // smallest that needs no more units than a workgroup has wavefronts; the
+  // runs of one slice after its first leave partial sums
+  H.un.assign(nt * waves, TileUnit{0, 1, 0, 0, 0, 0, -1, 0});
+  H.max_extra = 0;
+  for (int64_t t = 0; t < nt; ++t) {
+    const Cut& c = *cut[t];
+    const int own = (int)(std::lower_bound(c.nodes.begin(), c.nodes.end(), (int32_t)c.r0) - c.nodes.begin());
+    const int ns = (int)((c.r1 - c.r0 + kSliceRows - 1) / kSliceRows);
+    auto units = [&](int m) {
+      int n = 0;
+      for (int i = 0; i < ns; ++i) n += std::max(1, (sd[t * spt + i].y + m - 1) / m);
+      return n;
+    };
+    int m = pack;
+    while (units(m) > waves) m += pack;
+    int u = 0, extra = 0;
+    for (int w = 0; w < waves; ++w) {
+      H.un[t * waves + w].list = (int)first[t];
+      H.un[t * waves + w].nodes = (int)c.nodes.size();
+      H.un[t * waves + w].row0 = (int)c.r0;
+      H.un[t * waves + w].own = own;
+    }
+    for (int i = 0; i < ns; ++i) {
+      const int2 d = sd[t * spt + i];
+      const int np = std::max(1, (d.y + m - 1) / m);
+      for (int p = 0; p < np; ++p) {
+        TileUnit& w = H.un[t * waves + u++];
+        w.q0 = d.x + p * m;
+        w.nq = std::min(m, d.y - p * m);
+        w.slice = (int)(t * spt + i);
+        w.part = p | np << 8 | extra << 16;
+      }
+      extra += np - 1;
+    }
+    H.max_extra = std::max(H.max_extra, extra);
+  }
+  H.eidx.assign(q * 64, 0);
+  H.perm.assign(q * 64, -1);
+  // Entries of a row in an order that spreads the simultaneous LDS reads of
+  // four neighbouring rows over the banks: row i of a slice takes at place e
+  // an entry whose node's place in the list is (e + i) mod 4, while it has one
+#pragma omp parallel
+  {
+    std::vector<uint16_t> local(nb, 0);
+    std::vector<int64_t> by[4];
+#pragma omp for schedule(dynamic, 16)
+    for (int64_t t = 0; t < nt; ++t) {
+      const Cut& c = *cut[t];
+      for (size_t i = 0; i < c.nodes.size(); ++i) local[c.nodes[i]] = (uint16_t)i;
+      for (int64_t s = t * spt; s < (t + 1) * spt; ++s)
+        for (int j = 0; j < kSliceRows; ++j) {
+          if (H.lrow[s * kSliceRows + j] == 0xffff) continue;
+          const int64_t r = c.r0 + H.lrow[s * kSliceRows + j];
+          for (auto& b : by) b.clear();
+          for (int64_t k = rp[r + 1] - 1; k >= rp[r]; --k) by[local[ci[k]] & 3].push_back(k);
+          for (int64_t e = 0; e < rp[r + 1] - rp[r]; ++e) {
+            int cl = (int)((e + j) & 3);
+            if (by[cl].empty())
+              for (int b = 0; b < 4; ++b)
+                if (by[b].size() > by[cl].size()) cl = b;
+            const int64_t k = by[cl].back();
+            by[cl].pop_back();
+            const int64_t slot = (sd[s].x + e / 4) * 64 + j * 4 + e % 4;
+            H.eidx[slot] = local[ci[k]];
+            H.perm[slot] = (int32_t)k;
+          }
+        }
+    }
+  }
+  if (pack == 2)  // the two indices of a pair of quads side by side
+    for (int64_t p = 0; p < q / 2; ++p) {
+      uint16_t t[128];
+      for (int l = 0; l < 64; ++l) {
+        t[2 * l] = H.eidx[p * 128 + l];
+        t[2 * l + 1] = H.eidx[p * 128 + 64 + l];
+      }
+      std::copy(t, t + 128, H.eidx.begin() + p * 128);
+    }
+  return true;
+}
+
+// Value slots: MASS3 pairs of quads, [pair][lane][2]; BSR3 [quad], the nine
+// values of each lane as 16-byte planes and one plane of the ninth value.
+template <class T>
+__global__ void tile_values_k(int64_t nslot, int nv, int64_t nbnz, const int32_t* __restrict__ perm,
+                              const double* __restrict__ bval, T* __restrict__ out, int flags) {
+  constexpr int PW = 16 / (int)sizeof(T);
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nslot; i += (int64_t)gridDim.x * 256) {
+    const int32_t k = perm[i];
+    const int64_t quad = i >> 6, lane = i & 63;
+    if (nv == 1) {
+      out[(quad >> 1) * 128 + lane * 2 + (quad & 1)] = k < 0 ? (T)0 : (T)bval[k];
+    } else {
+      for (int q = 0; q < 9; ++q)
+        out[quad * 576 + (q < 8 ? (q / PW) * 64 * PW + lane * PW + q % PW : 512 + lane)] =
+            k < 0 ? (T)0 : (T)bval[bidx(k, q, nbnz, flags)];
+    }
+  }
+}
+
+void fill_tile_values(DevMat& M, hipStream_t s, bool fp64) {
+  const int nv = M.layout == L_BSR3 ? 9 : 1;
+  for (TileSet& T : M.tset) {
+    if (!T.plan) continue;
+    const int64_t nslot = T.plan->quads * 64;
+    const size_t cnt = (size_t)std::max<int64_t>(nslot * nv, 1);
+    const unsigned grid = (unsigned)std::min<int64_t>(std::max<int64_t>((nslot + 255) / 256, 1), 16384);
+    if (fp64 || !T.val) {
+      if (!T.val) NMG_HIP(hipMalloc(&T.val, sizeof(double) * cnt));
+      hipLaunchKernelGGL((tile_values_k<double>), dim3(grid), dim3(256), 0, s, nslot, nv, M.nbnz, T.plan->perm, M.bval,
+                         T.val, kflags(M));
+    }
+    if (M.bval32) {
+      if (!T.val32) NMG_HIP(hipMalloc(&T.val32, sizeof(float) * cnt));
+      hipLaunchKernelGGL((tile_values_k<float>), dim3(grid), dim3(256), 0, s, nslot, nv, M.nbnz, T.plan->perm, M.bval,
+                         T.val32, kflags(M));
+    }
+    NMG_HIP(hipGetLastError());
+  }
+}
+
+// Rows of a tile.  Large matrices: as many as two workgroups per CU leave LDS
+// for -- 192 rows of up to 1400 nodes while a node takes at most 48 bytes (K <=
+// 2; FP32 vectors), 128 rows of up to 700 nodes at 96 bytes (K >= 4): at 1.9M
+// DoF K = 1 took 52 us with 192 rows against 65 with 128, K = 4 took 107 us
+// with 128 rows against 129 with 192 (one workgroup per CU); 96 rows for the
+// stiffness (K = 4: 360 us against 369 with 128).  Small ones: one tile per CU
+// (51.5k DoF, K = 4: 5.7 us with 80 rows, 6.3 with 48, 6.6 with 128).
+static int tile_rows(const DevMat& M, int most) {
+  const int64_t r = (M.nb + 256 * kSliceRows - 1) / (256 * kSliceRows) * kSliceRows;
+  return (int)std::min<int64_t>(r, most);
+}
+
+void build_tiles(DevMat& M, hipStream_t s) {
+  static std::mutex mu;  // two solvers may set up on one matrix at once
+  std::lock_guard<std::mutex> lk(mu);
+  if (M.layout == L_CSR || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return;
+  if (M.tset[0].use.load()) return;
+  const bool bsr = M.layout == L_BSR3;
+  const int small = tile_rows(M, bsr ? 96 : 128), large = tile_rows(M, bsr ? 96 : 192);
+  for (int i = 0; i < (small == large ? 1 : 2); ++i) {
+    TileSet& T = M.tset[i];
+    if (!T.plan) {  // else: the pattern of the matrix this one was copied from
+      HostTiles H;
+      const bool wide = i == 0 && small != large;
+      if (!tile_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), wide ? large : small, wide ? 1400 : 700,
+                       bsr ? 8 : 16, bsr ? 1 : 2, H))
+        break;
+      auto P = std::make_shared<TilePlan>();
+      P->ntiles = H.ntiles;
+      P->max_nodes = H.max_nodes;
+      P->max_extra = H.max_extra;
+      P->quads = H.quads;
+      P->un = to_device(H.un);
+      P->tcols = to_device(H.tcols);
+      P->lrow = to_device(H.lrow);
+      P->eidx = to_device(H.eidx);
+      P->perm = to_device(H.perm);
+      T.plan = P;
+    }
+  }
+  M.touch();
+  fill_tile_values(M, s, false);
+  NMG_HIP(hipStreamSynchronize(s));
+  for (int i = 1; i >= 0; --i)
+    if (M.tset[i].plan) M.tset[i].use.store(M.tset[i].plan.get());
+}
+
+// The tiles for a K-column product on vectors of `size`-byte values, or null
+// for the row kernels: a layout set or tuned explicitly for that width, and
+// matrices too small to pay for the list -> x -> LDS chain of a tile (measured
+// against the row kernels, us: scalar mass 556 nodes K = 1 3.5 : 3.4, K = 4
+// 4.5 : 3.9, K = 8 4.6 : 5.0; 3545 nodes K = 1 3.1 : 4.0, K = 4 4.6 : 5.3;
+// stiffness K = 1 17 180 nodes 9.8 : 8.9, 146k nodes 65 : 73; K = 4 3545 nodes
+// 5.1 : 7.3).
+static const TileSet* tile_set(const DevMat& M, int K, int size) {
+  if (M.layout == L_CSR || !M.tile_use(K)) return nullptr;
+  const int64_t least = M.layout == L_BSR3 ? (K == 1 ? 65536 : 1024) : (K >= 8 ? 1 : 2048);
+  if (M.nb < least) return nullptr;
+  const int i = M.tset[1].use.load() && std::min(K, 4) * size > 16 ? 1 : 0;
+  return M.tset[i].use.load() ? &M.tset[i] : nullptr;
+}
+
+struct TileView {
+  const TileUnit* un;
+  const int32_t* tcols;
+  const uint16_t* lrow;
+  const uint16_t* eidx;
+};
+
+// element l of p, with the 32-bit byte offset the scalar-base address form takes
+template <class T>
+__device__ __forceinline__ T* at(T* p, uint32_t l) {
+  using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+  return reinterpret_cast<T*>(reinterpret_cast<C*>(p) + l * (uint32_t)sizeof(T));
+}
+
+// Epilogues on the value at offset o + l of the block vectors (o uniform over
+// the wavefront, column c): s is the product there and own the staged x.
+struct TEpiStore {
+  double* y;
+  struct Pre {};
+  __device__ __forceinline__ void load(int64_t, uint32_t, int, Pre&) const {}
+  __device__ __forceinline__ void store(int64_t o, uint32_t l, int, double s, double, const Pre&) const {
+    *at(y + o, l) = s;
+  }
+};
+template <class XT>
+struct TEpiCheb {
+  const XT* b;
+  XT* xm;
+  double w, ith;
+  struct Pre {
+    double b, xm;
+  };
+  __device__ __forceinline__ void load(int64_t o, uint32_t l, int, Pre& p) const {
+    p.b = (double)*at(b + o, l);
+    p.xm = (double)*at((const XT*)xm + o, l);
+  }
+  __device__ __forceinline__ void store(int64_t o, uint32_t l, int, double s, double own, const Pre& p) const {
+    *at(xm + o, l) = (XT)(p.xm + w * (own - p.xm + (p.b - s) * ith));
+  }
+};
+struct TEpiFilter {
+  const double* vk;
+  double* vkm;
+  double* y;
+  const double* mu;  // per column, or null for mu0
+  double mu0, t, cc;
+  int first;
+  struct Pre {
+    double vk, vkm, y;
+  };
+  __device__ __forceinline__ void load(int64_t o, uint32_t l, int, Pre& p) const {
+    p.vk = *at(vk + o, l);
+    p.vkm = first ? 0.0 : *at((const double*)vkm + o, l);
+    p.y = *at((const double*)y + o, l);
+  }
+  __device__ __forceinline__ void store(int64_t o, uint32_t l, int c, double s, double, const Pre& p) const {
+    const double v = t * (s - cc * p.vk) - p.vkm;
+    *at(vkm + o, l) = v;
+    *at(y + o, l) = p.y + (mu ? mu[c] : mu0) * v;
+  }
+};
+
+// lane permutation within groups of four (DPP quad_perm)
+template <int CTRL>
+__device__ __forceinline__ int quad(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double quad(double v) {
+  const int lo = quad<CTRL>((int)__double2loint(v)), hi = quad<CTRL>((int)__double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad(float v) {
+  return __int_as_float(quad<CTRL>(__float_as_int(v)));
+}
+
+
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void lds_load16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(uintptr_t)g,
+                                   (__attribute__((address_space(3))) void*)(uint32_t)(uintptr_t)l, 16, 0, 0);
+}
+
+// the values and list places of one lane: a pair of quads (MASS3) or one (BSR3)
+template <bool BSR, class VT>
+struct Entry;
+template <>
+struct Entry<false, double> {
+  d2 v;
+  uint32_t id;
+  __device__ __forceinline__ void load(const double* val, const uint16_t* e, int64_t i, int lane) {
+    v = *at(reinterpret_cast<const d2*>(val + i * 128), lane);
+    id = *at(reinterpret_cast<const uint32_t*>(e + i * 128), lane);
+  }
+};
+template <>
+struct Entry<false, float> {
+  f2 v;
+  uint32_t id;
+  __device__ __forceinline__ void load(const float* val, const uint16_t* e, int64_t i, int lane) {
+    v = *at(reinterpret_cast<const f2*>(val + i * 128), lane);
+    id = *at(reinterpret_cast<const uint32_t*>(e + i * 128), lane);
+  }
+};
+template <>
+struct Entry<true, double> {
+  d2 w[4];
+  double w8;
+  int id;
+  __device__ __forceinline__ void load(const double* val, const uint16_t* e, int64_t i, int lane) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = *at(reinterpret_cast<const d2*>(val + i * 576 + k * 128), lane);
+    w8 = *at(val + i * 576 + 512, lane);
+    id = *at(e + i * 64, lane);
+  }
+  __device__ __forceinline__ void get(double* m) const {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m[k] = w[k / 2][k % 2];
+    m[8] = w8;
+  }
+};
+template <>
+struct Entry<true, float> {
+  f4 w[2];
+  float w8;
+  int id;
+  __device__ __forceinline__ void load(const float* val, const uint16_t* e, int64_t i, int lane) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) w[k] = *at(reinterpret_cast<const f4*>(val + i * 576 + k * 256), lane);
+    w8 = *at(val + i * 576 + 512, lane);
+    id = *at(e + i * 64, lane);
+  }
+  __device__ __forceinline__ void get(float* m) const {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m[k] = w[k / 4][k % 4];
+    m[8] = w8;
+  }
+};
+
+template <int KG, bool BSR, class VT, class XT, class Epi>
+__global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
+    TileView T, const VT* __restrict__ val, const XT* __restrict__ x, int K, int lgroups, int part_off, Epi epi,
+    int flags) {
+  extern __shared__ double2 tile_lds[];
+  char* const xs = reinterpret_cast<char*>(tile_lds);
+  double* const partial = reinterpret_cast<double*>(xs + part_off);
+  constexpr int NW = BSR ? 8 : 16, TB = 64 * NW;
+  constexpr int NV = BSR ? 9 : 1;
+  constexpr int QP = BSR ? 1 : 2;            // quads of an Entry
+  constexpr int QD = BSR ? 2 : 3;            // entries in flight per lane
+  constexpr int SEG = KG * (int)sizeof(XT);  // bytes of one component's columns
+  constexpr int NB = 3 * SEG;                // bytes of a node in LDS
+  constexpr int UB = SEG >= 16 ? 16 : SEG;   // staged unit
+  constexpr int NU = NB / UB, SU = SEG / UB;
+  constexpr int SB = NU == 3 ? 3 : 5;        // units per lane and list load
+  constexpr int NP = KG == 4 ? 3 : (KG == 2 ? 2 : 1);  // components a lane writes
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qr = lane & 3;
+  const int col = KG == 4 ? qr : (KG == 2 ? (qr & 1) : 0);
+  auto comp = [&](int p) { return KG == 4 ? p : (KG == 2 ? (qr >> 1) + 2 * p : qr); };
+  const int lb = (int)xcd_block(flags);
+  const int c0 = (lb & ((1 << lgroups) - 1)) * KG;
+  const TileUnit un = T.un[(int64_t)(lb >> lgroups) * NW + wave];
+
+  int lr = 0xffff;  // this lane's row within the tile
+  if (un.slice >= 0) lr = (int)T.lrow[(int64_t)un.slice * kSliceRows + (lane >> 2)];
+  Entry<BSR, VT> en[QD];
+  const int64_t e0 = un.q0 / QP;
+  const int ne = un.nq / QP;
+#pragma unroll
+  for (int u = 0; u < QD; ++u)
+    if (u < ne) en[u].load(val, T.eidx, e0 + u, lane);
+  // stage x: each wavefront a run of the tile's units, the list read once per
+  // SB units and handed to the lanes across the wavefront
+  {
+    const int total = un.nodes * NU;
+    const int per = (total + TB * SB - 1) / (TB * SB) * (64 * SB);
+    for (int b0 = wave * per; b0 < (wave + 1) * per && b0 < total; b0 += 64 * SB) {
+      const int n0 = b0 / NU;
+      const int ln = T.tcols[un.list + min(n0 + lane, un.nodes - 1)];
+      uint32_t src[SB];
+#pragma unroll
+      for (int u = 0; u < SB; ++u) {
+        const int t = min(b0 + u * 64 + lane, total - 1);
+        const int n = t / NU, part = t - n * NU;
+        const int node = __builtin_amdgcn_ds_bpermute((n - n0) * 4, ln);
+        src[u] = (uint32_t)(3 * node + part / SU) * (uint32_t)K + (part % SU) * (UB / (int)sizeof(XT));
+      }
+      if constexpr (UB == 16) {
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+          if (b0 + u * 64 < total) lds_load16(at(x + c0, src[u]), xs + (size_t)(b0 + u * 64) * 16);
+      } else {
+        using U = std::conditional_t<UB == 8, double, float>;
+        U v[SB];
+#pragma unroll
+        for (int u = 0; u < SB; ++u) v[u] = *reinterpret_cast<const U*>(at(x + c0, src[u]));
+#pragma unroll
+        for (int u = 0; u < SB; ++u)
+          if (b0 + u * 64 + lane < total) reinterpret_cast<U*>(xs)[b0 + u * 64 + lane] = v[u];
+      }
+    }
+  }
+  const int part = un.part & 255, np = (un.part >> 8) & 255, slot = un.part >> 16;
+  const int64_t o = 3 * (int64_t)un.row0 * K + c0;
+  const uint32_t l0 = (uint32_t)(3 * lr * K + col);
+  const bool wr = part == 0 && lr != 0xffff;
+  typename Epi::Pre pre[NP];
+  if (wr) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (comp(p) < 3) epi.load(o, l0 + comp(p) * K, c0 + col, pre[p]);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  double y[3] = {0.0, 0.0, 0.0};
+  auto madd = [&](const VT* m, const char* xn) {
+    double xv[3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) xv[p] = (double)*reinterpret_cast<const XT*>(xn + p * SEG);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      if constexpr (BSR) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) y[p] += (double)m[3 * p + j] * xv[j];
+      } else {
+        y[p] += (double)m[0] * xv[p];
+      }
+    }
+  };
+  const char* const xc = xs + col * (int)sizeof(XT);
+  auto step = [&](const VT* m, int id) {
+    const int off = id * NB;
+    auto one = [&](auto ctrl) {
+      constexpr int C = decltype(ctrl)::value;
+      VT a[NV];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) a[v] = quad<C>(m[v]);
+      madd(a, xc + quad<C>(off));
+    };
+    if constexpr (KG == 1) {
+      madd(m, xc + off);
+    } else if constexpr (KG == 2) {
+      one(std::integral_constant<int, 0x50>{});
+      one(std::integral_constant<int, 0xfa>{});
+    } else {
+      one(std::integral_constant<int, 0x00>{});
+      one(std::integral_constant<int, 0x55>{});
+      one(std::integral_constant<int, 0xaa>{});
+      one(std::integral_constant<int, 0xff>{});
+    }
+  };
+  // the sums of one quad before the reads of the next: left alone the compiler
+  // gathers several quads' reads first and spills
+  auto keep = [&] { asm volatile("" : "+v"(y[0]), "+v"(y[1]), "+v"(y[2])); };
+  for (int q = 0; q < ne; q += QD) {
+#pragma unroll
+    for (int u = 0; u < QD; ++u)
+      if (q + u < ne) {
+        if constexpr (BSR) {
+          VT m[9];
+          en[u].get(m);
+          step(m, en[u].id);
+          keep();
+        } else {
+          const VT m0 = en[u].v[0], m1 = en[u].v[1];
+          step(&m0, (int)(en[u].id & 0xffff));
+          keep();
+          step(&m1, (int)(en[u].id >> 16));
+          keep();
+        }
+        if (q + QD + u < ne) en[u].load(val, T.eidx, e0 + q + QD + u, lane);
+      }
+  }
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      y[p] += quad<0xb1>(y[p]);
+      y[p] += quad<0x4e>(y[p]);
+    }
+  } else if constexpr (KG == 2) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) y[p] += quad<0x4e>(y[p]);
+  }
+  double sum[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) sum[p] = comp(p) == 0 ? y[0] : (comp(p) == 1 ? y[1] : y[2]);
+  if (part_off > 0) {  // some slice of the matrix is split
+    if (part > 0) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) partial[((slot + part - 1) * NP + p) * 64 + lane] = sum[p];
+    }
+    __syncthreads();
+    if (part == 0)
+      for (int i = 0; i < np - 1; ++i)
+#pragma unroll
+        for (int p = 0; p < NP; ++p) sum[p] += partial[((slot + i) * NP + p) * 64 + lane];
+  }
+  if (wr) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (comp(p) < 3) {
+        const double own = (double)*reinterpret_cast<const XT*>(xc + (un.own + lr) * NB + comp(p) * SEG);
+        epi.store(o, l0 + comp(p) * K, c0 + col, sum[p], own, pre[p]);
+      }
+  }
+}
+
+template <int KG, bool BSR, class VT, class XT, class Epi>
+static void launch_tile(const DevMat& M, const TilePlan& P, const VT* v, const XT* x, int K, Epi epi, hipStream_t s) {
+  int lg = 0;
+  while ((KG << lg) < K) ++lg;
+  const TileView T{P.un, P.tcols, P.lrow, P.eidx};
+  constexpr int NP = KG == 4 ? 3 : (KG == 2 ? 2 : 1);
+  size_t lds = ((size_t)P.max_nodes * 3 * KG * sizeof(XT) + 1023) / 1024 * 1024;
+  int part_off = 0;  // no slice is split
+  if (P.max_extra > 0) {
+    part_off = (int)lds;
+    lds += (size_t)P.max_extra * 64 * NP * sizeof(double);
+  }
+  hipLaunchKernelGGL((node_tile_k<KG, BSR, VT, XT, Epi>), dim3((unsigned)(P.ntiles << lg)), dim3(BSR ? 512 : 1024),
+                     lds, s, T, v, x, K, lg, part_off, epi, kflags(M));
+  NMG_HIP(hipGetLastError());
+}
+
+template <bool BSR, class XT, class Epi>
+static bool tile_product(const DevMat& M, const XT* x, int K, Epi epi, hipStream_t s, bool fp32,
+                         std::initializer_list<const void*> others) {
+  if (M.layout != (BSR ? L_BSR3 : L_MASS3)) return false;
+  const TileSet* T = tile_set(M, K, sizeof(XT));
+  if (!T) return false;
+  // 32-bit offsets into x, and 16-byte loads (8 at K = 2 in FP32) of its columns
+  if ((uint64_t)M.nrow * K * sizeof(XT) >= (uint64_t)1 << 32) return false;
+  uintptr_t a = (uintptr_t)x;
+  for (const void* p : others) a |= (uintptr_t)p;
+  if (a % std::min<size_t>(16, std::min(K, 4) * sizeof(XT))) return false;
+  auto go = [&](auto* v) {
+    if (K == 1) launch_tile<1, BSR>(M, *T->plan, v, x, K, epi, s);
+    else if (K == 2) launch_tile<2, BSR>(M, *T->plan, v, x, K, epi, s);
+    else launch_tile<4, BSR>(M, *T->plan, v, x, K, epi, s);
+  };
+  if (fp32 && T->val32) go((const float*)T->val32);
+  else go((const double*)T->val);
+  return true;
+}
+
+bool k_tile_spmv(int K, const DevMat& M, const double* x, double* y, hipStream_t s, bool fp32) {
+  return tile_product<false>(M, x, K, TEpiStore{y}, s, fp32, {y}) ||
+         tile_product<true>(M, x, K, TEpiStore{y}, s, fp32, {y});
+}
+bool k_tile_cheb_step(int K, const DevMat& M, const double* b, const double* xk, double* xm, double w, double ith,
+                      hipStream_t s, bool fp32) {
+  return tile_product<false>(M, xk, K, TEpiCheb<double>{b, xm, w, ith}, s, fp32, {b, xm});
+}
+bool k_tile_cheb_step32(int K, const DevMat& M, const float* b, const float* xk, float* xm, double w, double ith,
+                        hipStream_t s, bool fp32) {
+  return tile_product<false>(M, xk, K, TEpiCheb<float>{b, xm, w, ith}, s, fp32, {b, xm});
+}
+bool k_tile_filter_step(int K, const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
+                        const double* mu, double mu0, double t, double cc, bool first, hipStream_t s, bool fp32) {
+  return tile_product<true>(A, x, K, TEpiFilter{vk, vkm, y, mu, mu0, t, cc, first ? 1 : 0}, s, fp32, {vk, vkm, y});
+}
+
+}  // namespace nmg

@@ -582,7 +582,7 @@ def csr_autotune(mat: Handle, K: int, reps: int = 10, fp32: bool = False):
                                    ctypes.byref(s), ctypes.byref(kind), ctypes.byref(rows), ctypes.byref(cap),
                                    ctypes.byref(thr)))
     return dict(seconds=s.value, kind=["lanes_per_row", "rows_per_wave", "tiled", "row_groups", "wide", "tiled_wide",
-                                      "pipelined_rows"][kind.value],
+                                      "pipelined_rows", "node_tiles"][kind.value],
                 rows=rows.value, cap=cap.value, threads=thr.value)
 
 

@@ -1,0 +1,207 @@
+"""Node tiles: the host layout on the CPU (every entry once, sums as the
+kernel forms them) and the products on the GPU against scipy, at tile edges,
+empty and long rows, every column count, value and vector type."""
+import ctypes
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from normalmodes_amd import pevsl as pv
+
+_i64p, _i32p, _u16p = (ctypes.POINTER(t) for t in (ctypes.c_int64, ctypes.c_int32, ctypes.c_uint16))
+
+
+def _pattern(nb, seed, band=60, long_row=0):
+    """A ragged node pattern: 0 to 30 local columns per row, some rows without
+    a diagonal, a few far columns, optionally one row of `long_row` columns."""
+    rng = np.random.default_rng(seed)
+    rows, cols = [], []
+    for r in range(nb):
+        n = int(rng.integers(0, 31)) if r % 7 else 0
+        c = np.clip(r + rng.integers(-band, band + 1, n), 0, nb - 1)
+        if r % 11 == 0:
+            c = np.append(c, rng.integers(0, nb, 2))
+        if r % 3:
+            c = np.append(c, r)
+        if long_row and r == nb // 2:
+            c = np.append(c, rng.choice(nb, min(long_row, nb), replace=False))
+        c = np.unique(c)
+        rows.append(np.full(c.size, r))
+        cols.append(c)
+    rows, cols = np.concatenate(rows), np.concatenate(cols)
+    M = sp.csr_matrix((rng.standard_normal(rows.size), (rows, cols)), shape=(nb, nb))
+    M.sort_indices()
+    return M
+
+
+def _layout(M, rows, cap, waves, pack):
+    rp, ci = M.indptr.astype(np.int64), M.indices.astype(np.int32)
+    sz = np.zeros(6, dtype=np.int64)
+
+    def call(*out):
+        p = [None if o is None else o.ctypes.data_as(t)
+             for o, t in zip(out, (_i32p, _i32p, _u16p, _u16p, _i32p))]
+        pv._check(pv._lib().nmg_node_tiles_host(
+            ctypes.c_int64(M.shape[0]), rp.ctypes.data_as(_i64p), ci.ctypes.data_as(_i32p), ctypes.c_int(rows),
+            ctypes.c_int(cap), ctypes.c_int(waves), ctypes.c_int(pack), sz.ctypes.data_as(_i64p), *p))
+
+    call(None, None, None, None, None)
+    nt, quads, nl, spt, mx, ex = (int(v) for v in sz)
+    if nt == 0:
+        return None
+    units = np.zeros((nt, waves, 8), dtype=np.int32)
+    lists = np.zeros(nl, dtype=np.int32)
+    lrow = np.zeros((nt * spt, 16), dtype=np.uint16)
+    eidx, perm = np.zeros(64 * quads, dtype=np.uint16), np.zeros(64 * quads, dtype=np.int32)
+    call(units, lists, lrow, eidx, perm)
+    return dict(units=units, lists=lists, lrow=lrow, eidx=eidx, perm=perm, spt=spt, max_nodes=mx, max_extra=ex)
+
+
+def _product(M, L, x, pack):
+    """y = M x in the tiles' order: per unit, quads of four entries of 16 rows,
+    x through the tile's list; later parts of a slice added to its first."""
+    y = np.full((M.shape[0], x.shape[1]), np.nan)
+    seen = np.zeros(M.nnz, dtype=int)
+    for tile in L["units"]:
+        for w, (lst, nodes, row0, own, q0, nq, sl, part) in enumerate(tile):
+            if sl < 0:
+                continue
+            xs = x[L["lists"][lst:lst + nodes]]
+            part, parts, slot = part & 255, (part >> 8) & 255, part >> 16
+            assert part < parts and slot + parts - 1 <= L["max_extra"] and nodes <= L["max_nodes"]
+            acc = np.zeros((16, x.shape[1]))
+            for q in range(q0, q0 + nq):
+                for j in range(16):
+                    for e in range(4):
+                        k = L["perm"][64 * q + 4 * j + e]
+                        if k < 0:
+                            continue
+                        at = 64 * q + 4 * j + e if pack == 1 else 128 * (q // 2) + 2 * (4 * j + e) + q % 2
+                        acc[j] += M.data[k] * xs[L["eidx"][at]]
+                        seen[k] += 1
+            rows = L["lrow"][sl].astype(int)
+            for j in np.flatnonzero(rows != 0xffff):
+                r = row0 + rows[j]
+                assert L["lists"][lst + own + rows[j]] == r      # the row's own x
+                y[r] = acc[j] if part == 0 else y[r] + acc[j]
+    assert (seen == 1).all()
+    return y
+
+
+@pytest.mark.parametrize("nb,rows,cap,waves,pack,long_row", [
+    (1, 16, 100, 16, 2, 0), (15, 16, 100, 8, 1, 0), (16, 16, 100, 16, 1, 0), (17, 16, 100, 16, 2, 0),
+    (300, 128, 700, 16, 2, 0), (300, 96, 150, 8, 1, 0), (130, 128, 700, 8, 1, 90), (257, 192, 260, 16, 2, 250),
+    (260, 48, 120, 16, 2, 0)])
+def test_layout_forms_the_product(nb, rows, cap, waves, pack, long_row):
+    M = _pattern(nb, nb + rows, long_row=long_row)
+    L = _layout(M, rows, cap, waves, pack)
+    x = np.random.default_rng(1).standard_normal((nb, 2))
+    # both sides sum at most 300 terms: (300 + 3) eps of the absolute sum
+    bound = 303 * np.finfo(float).eps * (abs(M) @ abs(x)) + 1e-300
+    assert (abs(_product(M, L, x, pack) - M @ x) <= bound).all()
+
+
+def test_layout_refuses_what_a_tile_cannot_hold():
+    M = _pattern(200, 3, long_row=150)
+    assert _layout(M, 64, 100, 16, 2) is None          # one row references more than 100 nodes
+    assert _layout(M, 256, 700, 8, 1) is None          # more slices than wavefronts
+    assert _layout(M, 64, 160, 16, 2) is not None
+
+
+def _handles(M, kind, seed):
+    """The DoF matrix of a node pattern: mass (x) I3, or random 3x3 blocks."""
+    if kind == "mass":
+        D = sp.kron(M, sp.identity(3), format="csr")
+    else:
+        rng = np.random.default_rng(seed)
+        D = sp.bsr_matrix((rng.standard_normal((M.nnz, 3, 3)), M.indices, M.indptr), shape=(3 * M.shape[0],) * 2)
+        D = D.tocsr()
+    D.sort_indices()
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    assert pv.csr_info(m)["layout"] == ("mass3" if kind == "mass" else "bsr3")
+    return D, m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,nb,long_row", [
+    ("mass", 2048, 0), ("mass", 2049, 0), ("mass", 6000, 300), ("mass", 40000, 0), ("mass", 3000, 1500), ("mass", 40, 0),
+    ("bsr", 1024, 0), ("bsr", 1025, 300), ("bsr", 30000, 0), ("bsr", 66000, 0)])
+def test_products(kind, nb, long_row):
+    """A x (or B x) on 1 to 64 columns, FP64 and FP32 values; the filter's fused
+    step through it on the same matrix as A~ of a diagonal-mass pencil."""
+    M = _pattern(nb, nb, long_row=long_row)
+    D, m = _handles(M, kind, 5)
+    n = D.shape[0]
+    h = ch = None
+    try:
+        ch = pv.pevsl_setup_chebiter(0.5, 1.5, 1, m)        # lays the tiles out
+        h = pv.pevsl_start(0)
+        pv.pevsl_setprobsizes(h, n, n, -1)
+        pv.pevsl_setbmv(h, m)
+        pv.pevsl_setbsol_chebiter(h, 2, ch)
+        pv.pevsl_setamv(h, m)
+        rng = np.random.default_rng(2)
+        aD = abs(D)
+        most = int(np.diff(D.indptr).max())
+        eps = np.finfo(float).eps
+        for K in (1, 2, 4, 8, 16, 32, 64):
+            X = rng.standard_normal((K, n))
+            tol = 2 * (most + 3) * eps * (aD @ abs(X).T).T + 1e-300
+            assert (abs(pv.apply_block(h, 1, X) - (D @ X.T).T) <= tol).all(), K
+        pv.pevsl_set_precision(h, pv.FP32_FILTER)
+        for K in (1, 4):  # FP32 values: one rounding of 2^-24 per entry
+            X = rng.standard_normal((K, n))
+            tol = (2 * (most + 3) * eps + 2.0 ** -24) * (aD @ abs(X).T).T + 1e-300
+            assert (abs(pv.apply_block(h, 0, X) - (D @ X.T).T) <= tol).all(), K
+    finally:
+        if h:
+            pv.pevsl_finish(h)
+        if ch:
+            pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nb,long_row", [(2048, 0), (6001, 300), (36000, 0)])
+def test_chebyshev_steps(nb, long_row):
+    """The fused step on a mass pattern: `deg` steps against the recurrence in
+    numpy, FP64 and FP32 iterates, 1 to 16 columns."""
+    M = _pattern(nb, nb + 1, long_row=long_row)
+    M = M * 0.02 + sp.identity(nb) * 2.0                    # well conditioned, not symmetric
+    M.sort_indices()
+    D, m = _handles(M.tocsr(), "mass", 5)
+    n, deg, lo, hi = D.shape[0], 5, 1.0, 3.0
+    h = ch = None
+    try:
+        ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+        h = pv.pevsl_start(0)
+        pv.pevsl_setprobsizes(h, n, n, -1)
+        pv.pevsl_setbmv(h, m)
+        pv.pevsl_setbsol_chebiter(h, 2, ch)
+        pv.pevsl_setamv(h, m)
+        pv.pevsl_set_geneig(h)
+        th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
+
+        def ref(b):
+            xm, xk, w = np.zeros_like(b), b / th, 2.0
+            for _ in range(deg):
+                w = 1.0 / (1.0 - w / (4.0 * sg * sg))
+                xm, xk = xk, xm + w * (xk - xm + (b - D @ xk) / th)
+            return xk
+
+        rng = np.random.default_rng(4)
+        for prec, rel in ((pv.FP64, 1e-13), (pv.FP32_FILTER, 1e-6), (pv.FP32_BSOLVE, 4e-6)):
+            if prec != pv.FP64:
+                pv.pevsl_set_precision(h, prec)
+            for K in (1, 2, 4, 8, 16):
+                X = rng.standard_normal((K, n))
+                want = ref(X.T).T
+                got = pv.apply_block(h, 2, X)
+                assert np.linalg.norm(got - want) <= rel * np.linalg.norm(want), (prec, K)
+    finally:
+        if h:
+            pv.pevsl_finish(h)
+        if ch:
+            pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
