@@ -391,6 +391,7 @@ DevMat* clone_devmat(const DevMat& S, hipStream_t s) {
   M->group = S.group;
   for (int i = 0; i < 7; ++i) M->block_map[i] = S.block_map[i];
   for (int i = 0; i < 7; ++i) M->wide[i] = S.wide[i];
+  for (int i = 0; i < 7; ++i) M->tuned[i] = S.tuned[i];
   auto cp = [&](auto* src, auto*& dst, size_t count) {
     using T = std::remove_pointer_t<std::remove_reference_t<decltype(dst)>>;
     if (!src) return;
@@ -459,6 +460,10 @@ struct Cheb {
   // Chebyshev solve of degree inner_deg with FP32 values and FP32 iterates
   // on the FP64 residual b - B~x of the sum so far, added in FP64
   int refine = 0, inner_deg = 0;
+  // one-launch solve of a small system (null: the matrix does not fit), with
+  // the step weights w_1 .. w_deg on the device
+  std::shared_ptr<const SmallPlan> small;
+  DVec wts;
   FVec own32;           // inner work (3 n K floats) when the caller brings none
   PersistPlan plan[2];  // FP64 / FP32 values
   bool planned[2] = {false, false};
@@ -756,6 +761,14 @@ static Solver::GraphKey graph_key(const Solver& S, const Cheb& C, int K, int par
 //   x_1 = b/th,  x_{k+1} = x_{k-1} + w_{k+1}(x_k - x_{k-1} + (b - B x_k)/th),
 //   w_1 = 2, w_{k+1} = 1/(1 - w_k/(4 s^2)), th = (lmax+lmin)/2, s = th/de.
 // The result lands in `out`; `tmp` is a second buffer.
+// The whole solve of K columns in one launch where the matrix is small enough
+// (nmgpu_small.hip) and no layout was set explicitly for that width.
+static bool small_solve(const Cheb& C, int K, const double* b, double* out, hipStream_t s, bool fp32) {
+  if (!C.small || !C.mat->small_use(K)) return false;
+  k_cheb_small(*C.small, *C.mat, K, C.deg, 2.0 / (C.lmax + C.lmin), C.wts.p, b, out, s, fp32);
+  return true;
+}
+
 // The Chebyshev semi-iteration as one fused launch per step: x_1 = b/th,
 // x_0 = 0 (cleared here), x_{k+1} from the fused product + update; the
 // iterates alternate between out and tmp so that the last lands in out.
@@ -840,8 +853,18 @@ static void cheb_solve(Cheb& C, const double* b, double* out, double* tmp, hipSt
     }
     return;
   }
-  // in a sampled solve one step launch (the middle one) is bracketed
   const bool pr = probe && probe->armed();
+  if (C.small && C.mat->small_use(1)) {  // a sampled solve is bracketed whole
+    if (pr) probe->before(s);
+    small_solve(C, 1, b, out, s, fp32);
+    if (pr) probe->after(s);
+    if (probe) {
+      probe->bytes = step_bytes * C.deg;
+      probe->launches = 1;
+    }
+    return;
+  }
+  // in a sampled solve one step launch (the middle one) is bracketed
   cheb_steps(C, b, out, tmp, s, fp32, pr ? probe : nullptr);
   if (probe) {
     probe->bytes = step_bytes;
@@ -1393,11 +1416,21 @@ static void block_cheb(Cheb& C, int K, const double* b, double* out, double* tmp
     }
     return;
   }
+  const bool pr = probe && probe->armed();
+  if (C.small && C.mat->small_use(K)) {  // a sampled solve is bracketed whole
+    if (pr) probe->before(s);
+    small_solve(C, K, b, out, s, fp32);
+    if (pr) probe->after(s);
+    if (probe) {
+      probe->bytes = step_bytes * C.deg;
+      probe->launches = 1;
+    }
+    return;
+  }
   double* xk = (C.deg % 2 == 0) ? out : tmp;
   double* xm = (C.deg % 2 == 0) ? tmp : out;
   k_scale_copy(nk, 1.0 / th, b, xk, s);
   k_fill(nk, 0.0, xm, s);
-  const bool pr = probe && probe->armed();
   const int mid = (C.deg + 1) / 2;
   double w = 2.0;
   for (int k = 1; k <= C.deg; ++k) {
@@ -2490,12 +2523,21 @@ int nmg_setup_chebiter(double lmin, double lmax, int deg, nmg_handle mat, nmg_ha
     NMG_CHECK(deg >= 1 && deg <= 100000, NMG_EINVAL, "chebiter degree must be >= 1");
     NMG_CHECK(M->nrow == M->ncol, NMG_EINVAL, "chebiter needs a square matrix");
     build_tiles(*M, default_stream());
-    Cheb* C = new Cheb();
+    std::unique_ptr<Cheb> C(new Cheb());
     C->mat = M;
     C->lmin = lmin;
     C->lmax = lmax;
     C->deg = deg;
-    *cheb = reg(C, K_CHEB);
+    C->small = plan_small(*M);
+    if (C->small) {
+      std::vector<double> w(deg);
+      const double sg = (lmax + lmin) / (lmax - lmin);
+      double wk = 2.0;
+      for (int k = 0; k < deg; ++k) w[k] = wk = 1.0 / (1.0 - wk / (4.0 * sg * sg));
+      C->wts.ensure(deg);
+      NMG_HIP(hipMemcpy(C->wts.p, w.data(), sizeof(double) * deg, hipMemcpyHostToDevice));
+    }
+    *cheb = reg(C.release(), K_CHEB);
   });
 }
 
@@ -2558,7 +2600,8 @@ int nmg_chebiter_noalloc(int type, const double* b, double* x, nmg_handle cheb, 
     NMG_CHECK(n <= kScratchDoubles, NMG_EINVAL,
               "nmg_chebiter_noalloc: the matrix has more rows than the scratch array holds (4194304)");
     double* tmp = scratch_on_current_device();
-    cheb_steps(*C, b, x, tmp, static_cast<hipStream_t>(stream), false, nullptr);
+    if (!small_solve(*C, 1, b, x, static_cast<hipStream_t>(stream), false))
+      cheb_steps(*C, b, x, tmp, static_cast<hipStream_t>(stream), false, nullptr);
     NMG_HIP(hipGetLastError());
     C->ncalls++;
     C->nmatvec += C->deg;
@@ -3061,6 +3104,7 @@ int nmg_set_stream_loads(nmg_handle mat, int on) {
 int nmg_set_kernel_map(nmg_handle mat, int group, int K, int rows_per_wave) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
+    M->set_by_hand(K > 0 ? K : 1);
     NMG_CHECK(group == 0 || group == 8 || group == 16 || group == 32 || group == 64, NMG_EINVAL,
               "group must be 0, 8, 16, 32 or 64");
     M->group = group;
@@ -3219,6 +3263,7 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   // apply the winner
   build_tiling(M, K, 0, 1);
   M.block_map[idx] = 0;
+  M.tuned[idx] = true;
   if (best.kind == 7) {
     // no explicit layout: the node tiles
   } else if (best.kind == 0) {
@@ -3368,6 +3413,7 @@ int nmg_node_tiles_host(int64_t nb, const int64_t* rowptr, const int32_t* col, i
 int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int threads) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
+    M->set_by_hand(K);
     NMG_CHECK(rows_per_wave >= 1 && rows_per_wave <= 8 && K * rows_per_wave <= 64, NMG_EINVAL,
               "bad rows per wavefront");
     NMG_CHECK(max_nodes <= tile_cap_limit(K), NMG_EINVAL, "tile exceeds 64 KB of LDS");
@@ -3384,6 +3430,7 @@ int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int 
 int nmg_set_tiled_wide(nmg_handle mat, int K, int max_nodes, int lanes) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
+    M->set_by_hand(K);
     NMG_CHECK(K == 2 || K == 4 || K == 8 || K == 16, NMG_EINVAL, "K must be 2, 4, 8 or 16");
     NMG_CHECK(max_nodes * 24 * K <= 64 * 1024, NMG_EINVAL, "tile exceeds 64 KB of LDS");
     build_tiling(*M, K, max_nodes, 1, 1024, max_nodes > 0 ? lanes : 0);
@@ -3395,6 +3442,7 @@ int nmg_set_tiled_wide(nmg_handle mat, int K, int max_nodes, int lanes) {
 int nmg_set_wide(nmg_handle mat, int K, int lanes) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
+    M->set_by_hand(K);
     int idx = -1;
     for (int i = 1; i < 5; ++i)
       if ((1 << i) == K) idx = i;
@@ -3410,6 +3458,7 @@ int nmg_set_wide(nmg_handle mat, int K, int lanes) {
 int nmg_set_row_pipeline(nmg_handle mat, int lanes, int rows) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
+    M->set_by_hand(1);
     NMG_CHECK(rows == 0 || rows == 2 || rows == 4 || rows == 8, NMG_EINVAL, "rows per lane group must be 0, 2, 4 or 8");
     NMG_CHECK(rows == 0 || lanes == 16 || lanes == 32 || lanes == 64, NMG_EINVAL, "lanes per group must be 16, 32 or 64");
     NMG_CHECK(rows == 0 || M->layout == L_BSR3, NMG_EINVAL, "pipelined rows apply to 3x3-block matrices");
@@ -3426,6 +3475,7 @@ int nmg_set_row_pipeline(nmg_handle mat, int lanes, int rows) {
 int nmg_set_row_groups(nmg_handle mat, int per_wave) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
+    M->set_by_hand(1);
     NMG_CHECK(per_wave == 0 || per_wave == 1 || per_wave == 2 || per_wave == 4 || per_wave == 8, NMG_EINVAL,
               "groups per wavefront must be 0, 1, 2, 4 or 8");
     NMG_CHECK(per_wave == 0 || M->layout != L_CSR, NMG_EINVAL, "row groups apply to the blocked layouts");

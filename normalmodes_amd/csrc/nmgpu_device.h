@@ -27,4 +27,20 @@ __device__ __forceinline__ int64_t bidx(int64_t k, int q, int64_t nbnz, int flag
   return (flags & 4) ? ((k >> 6) * 576 + (int64_t)q * 64 + (k & 63)) : ((int64_t)q * nbnz + k);
 }
 
+// lane permutation by DPP: within groups of four (quad_perm), or mirrored in
+// rows of 8 (0x141) or 16 (0x140) lanes
+template <int CTRL>
+__device__ __forceinline__ int quad(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double quad(double v) {
+  const int lo = quad<CTRL>((int)__double2loint(v)), hi = quad<CTRL>((int)__double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad(float v) {
+  return __int_as_float(quad<CTRL>(__float_as_int(v)));
+}
+
 }  // namespace nmg

@@ -104,6 +104,24 @@ struct TileSet {
   float* val32 = nullptr;
 };
 
+// One-launch Chebyshev solves of small scalar-mass systems (nmgpu_small.hip):
+// per wavefront the bits of the quads that end a slice (then those that end one
+// of 16 lanes per row), the rows of its slices (0xffff: none), and each slot's node and matrix entry (-1: padding).
+struct HostSmall {
+  int quads = 0, slices = 0;  // per wavefront
+  std::vector<uint32_t> ends;
+  std::vector<uint16_t> rows, eidx;
+  std::vector<int32_t> perm;
+};
+struct SmallPlan {
+  int quads = 0, slices = 0;
+  uint32_t* head = nullptr;
+  uint16_t* rows = nullptr;
+  uint16_t* eidx = nullptr;
+  int32_t* perm = nullptr;
+  ~SmallPlan();
+};
+
 // Process-wide source of layout generations (unique across matrices, so a
 // matrix freed and re-created at the same address never repeats one).
 inline uint64_t next_layout_gen() {
@@ -164,6 +182,18 @@ struct DevMat {
     if (K == 1 && (group > 0 || pipe > 0 || rgroups || single_blocked)) return false;
     for (int i = 0; i < 7; ++i)
       if ((1 << i) == K) return block_map[i] == 0 && !tiling[i] && wide[i] == 0;
+    return false;
+  }
+  // layouts of the autotuner's choosing (per K = 1 .. 64): the one-launch solve
+  // of a small system comes before them, but not before one set by hand
+  bool tuned[7] = {false, false, false, false, false, false, false};
+  void set_by_hand(int K) {
+    for (int i = 0; i < 7; ++i)
+      if ((1 << i) == K) tuned[i] = false;
+  }
+  bool small_use(int K) const {
+    for (int i = 0; i < 7; ++i)
+      if ((1 << i) == K) return tuned[i] || tile_use(K);
     return false;
   }
   std::vector<int64_t> h_browptr;  // host copy of the node pattern (tiling)
@@ -240,6 +270,13 @@ bool k_tile_cheb_step32(int K, const DevMat& M, const float* b, const float* xk,
                         hipStream_t s, bool fp32);
 bool k_tile_filter_step(int K, const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
                         const double* mu, double mu0, double t, double cc, bool first, hipStream_t s, bool fp32);
+
+// one-launch solves of small systems: null when M does not fit; x ~ M^-1 b on K
+// interleaved columns by deg steps with the weights wts[deg] (device)
+bool small_layout(int64_t nb, const int64_t* rp, const int32_t* ci, HostSmall& H);
+std::shared_ptr<const SmallPlan> plan_small(const DevMat& M);
+void k_cheb_small(const SmallPlan& P, const DevMat& M, int K, int deg, double ith, const double* wts, const double* b,
+                  double* out, hipStream_t s, bool fp32);
 
 // ---------------------------------------------------------------------------
 // kernel launchers (nmgpu_kernels.hip); all asynchronous on stream s

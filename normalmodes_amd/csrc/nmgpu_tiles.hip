@@ -400,22 +400,6 @@ struct TEpiFilter {
   }
 };
 
-// lane permutation within groups of four (DPP quad_perm)
-template <int CTRL>
-__device__ __forceinline__ int quad(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ __forceinline__ double quad(double v) {
-  const int lo = quad<CTRL>((int)__double2loint(v)), hi = quad<CTRL>((int)__double2hiint(v));
-  return __hiloint2double(hi, lo);
-}
-template <int CTRL>
-__device__ __forceinline__ float quad(float v) {
-  return __int_as_float(quad<CTRL>(__float_as_int(v)));
-}
-
-
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));

@@ -1,0 +1,83 @@
+"""One-launch Chebyshev solves of small scalar-mass systems: against the
+recurrence in numpy and against the step-by-step kernels (a layout set by hand
+turns the one-launch form off), at one node, empty and long rows, the sizes
+around its limits, 1 to 64 columns, FP64 and FP32 values."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from normalmodes_amd import pevsl as pv
+
+pytestmark = pytest.mark.gpu
+
+
+def _mass(nb, per_row, seed, long_row=0):
+    rng = np.random.default_rng(seed)
+    rows, cols = [], []
+    for r in range(nb):
+        n = 0 if r % 9 == 4 else int(rng.integers(0, per_row + 1))
+        c = np.unique(rng.integers(0, nb, n + (long_row if r == nb // 3 else 0)))
+        rows.append(np.full(c.size, r))
+        cols.append(c)
+    rows, cols = np.concatenate(rows), np.concatenate(cols)
+    M = sp.csr_matrix((0.4 / max(per_row, 1) * rng.standard_normal(rows.size), (rows, cols)), shape=(nb, nb))
+    M = (M + sp.diags(np.where(np.arange(nb) % 9 == 4, 0.0, 2.0))).tocsr()
+    M.eliminate_zeros()
+    M.sort_indices()
+    return M
+
+
+# (nodes, entries per row): one slot per wavefront, a whole and a broken slice,
+# both sides of each register size (8, 16, 24, 32 quads) and sizes too large
+@pytest.mark.parametrize("nb,per_row,long_row", [
+    (1, 1, 0), (15, 6, 0), (16, 6, 0), (17, 6, 0), (555, 28, 0), (614, 15, 0), (700, 40, 400), (1100, 28, 0),
+    (2300, 12, 0), (4096, 3, 0), (4097, 3, 0), (3000, 40, 0)])
+def test_small_solve(nb, per_row, long_row):
+    M = _mass(nb, per_row, nb, long_row)
+    D = sp.kron(M, sp.identity(3), format="csr")
+    D.sort_indices()
+    n, lo, hi = D.shape[0], 1.0, 3.0
+    th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
+
+    def ref(b, deg):
+        xm, xk, w = np.zeros_like(b), b / th, 2.0
+        for _ in range(deg):
+            w = 1.0 / (1.0 - w / (4.0 * sg * sg))
+            xm, xk = xk, xm + w * (xk - xm + (b - D @ xk) / th)
+        return xk
+
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    rng = np.random.default_rng(2)
+    handles = []
+    try:
+        if pv.csr_info(m)["layout"] != "mass3":
+            pytest.skip("the pattern reads as 3x3 blocks")
+        for deg in (1, 2, 9):
+            ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+            handles.append((pv.pevsl_chebiter_free, ch))
+            h = pv.pevsl_start(0)
+            handles.insert(0, (pv.pevsl_finish, h))
+            pv.pevsl_setprobsizes(h, n, n, -1)
+            pv.pevsl_setbmv(h, m)
+            pv.pevsl_setbsol_chebiter(h, 2, ch)
+            pv.pevsl_setamv(h, m)
+            pv.pevsl_set_geneig(h)
+            for K in (1, 2, 4, 16, 64):
+                X = rng.standard_normal((K, n))
+                want = ref(X.T, deg).T
+                got = pv.apply_block(h, 2, X)
+                assert np.linalg.norm(got - want) <= 1e-13 * np.linalg.norm(want), (deg, K)
+            x = rng.standard_normal(n)
+            one = pv.pevsl_chebiter(2, x, ch)
+            assert np.linalg.norm(one - ref(x, deg)) <= 1e-13 * np.linalg.norm(one)
+            pv.set_kernel_map(m, 32)                       # by hand: step by step
+            step = pv.pevsl_chebiter(2, x, ch)
+            pv.set_kernel_map(m, 0)
+            assert np.linalg.norm(one - step) <= 1e-14 * deg * np.linalg.norm(step)
+            pv.pevsl_set_precision(h, pv.FP32_FILTER)      # FP32 values: 2^-24 each, grown by the recurrence
+            got = pv.apply_block(h, 2, X)
+            assert np.linalg.norm(got - want) <= 2.0 ** -22 * np.linalg.norm(want)
+    finally:
+        for f, v in handles:
+            f(v)
+        pv.csr_free(m)
