@@ -514,8 +514,9 @@ int nmg_tiling_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int m
  * eidx[64*quads] and perm[64*quads]; null pointers are skipped. */
 int nmg_node_tiles_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int rows, int cap, int waves, int pack,
                         int64_t *sizes, int32_t *units, int32_t *lists, uint16_t *lrow, uint16_t *eidx, int32_t *perm);
-/* Autotuner (no reference counterpart): times the product layouts of mat for
- * K columns on the device (lanes per row; rows per wavefront; LDS tiles with
+/* Autotuner (no reference counterpart): times the layouts of mat for K columns
+ * on the device, as the fused Chebyshev step of a scalar mass, the fused filter
+ * step of 3x3 blocks or the product of a rectangular matrix (lanes per row; rows per wavefront; LDS tiles with
  * capacities on a geometric ladder up to 64 KB, workgroups of 1024 or 256
  * threads; for K = 1 also row groups) and keeps the fastest.  kind: 0
  * lanes-per-row, 1 rows per wavefront, 2 tiled, 3 row groups, 4 wide,

@@ -3152,6 +3152,15 @@ static double time_launches(hipStream_t s, int reps, F&& f) {
   return ms * 1e-3 / reps;
 }
 
+// the tuner's timing: at least `reps` launches and 0.3 ms of them, the better
+// of two runs (a run of 10 launches of a 3 us kernel mostly times its events)
+template <class F>
+static double time_candidate(hipStream_t s, int reps, F&& f) {
+  const double t = time_launches(s, reps, f);
+  const int n = (int)std::min(200.0, 3e-4 / std::max(t, 1e-7));
+  return n <= reps ? t : std::min(time_launches(s, n, f), time_launches(s, n, f));
+}
+
 struct TuneResult {
   double seconds = 1e30;
   int kind = 0;  // 0 lanes-per-row (K = 1), 1 untiled block, 2 tiled block, 3 row groups (K = 1),
@@ -3167,10 +3176,36 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   int idx = 0;
   while ((1 << idx) != K) ++idx;
   const int64_t nk = M.nrow * K;
-  DVec x, y;
-  x.ensure(nk);
+  DVec x, y, z, w, mu;
+  x.ensure(M.ncol * K);
   y.ensure(nk);
-  k_fill(nk, 1.0, x.p, s);
+  z.ensure(nk);
+  w.ensure(nk);
+  mu.ensure(K);
+  k_fill(M.ncol * K, 1.0, x.p, s);
+  k_fill(nk, 0.5, y.p, s);
+  k_fill(nk, 0.5, z.p, s);
+  k_fill(nk, 0.0, w.p, s);
+  k_fill(K, 0.1, mu.p, s);
+  // What is timed is what the solver runs: the fused Chebyshev step of a scalar
+  // mass, the fused filter step of 3x3 blocks (the plain product only of
+  // rectangular matrices).  Plain products misjudge layouts whose epilogue
+  // operands are loaded row by row: at 10.6k DoF one that won as a product took
+  // 7.2 us as a Chebyshev step, against 4.0 for the row kernels.
+  const bool square = M.nrow == M.ncol, mass = M.layout == L_MASS3;
+  double *a = x.p, *b = y.p;
+  auto op = [&] {
+    if (!square) {
+      K == 1 ? k_spmv(M, x.p, y.p, s, fp32) : k_block_spmv(K, M, x.p, y.p, s, fp32);
+    } else if (mass) {
+      K == 1 ? k_cheb_step(M, z.p, a, b, 1.0, 0.1, s, fp32) : k_block_cheb_step(K, M, z.p, a, b, 1.0, 0.1, s, fp32);
+      std::swap(a, b);
+    } else if (K == 1) {
+      k_filter_step(M, x.p, z.p, y.p, w.p, 1.0, 1.0, 0.1, true, s, fp32);
+    } else {
+      k_block_filter_step(K, M, x.p, z.p, y.p, w.p, mu.p, 1.0, 1.0, true, s, fp32);
+    }
+  };
   // The wide layouts (kinds 4 and 5: one entry per lane, the K columns in
   // registers) are chosen only when they win by 3%. Timed alone they can tie
   // the row layouts within noise, but beside a second stream's products they
@@ -3179,7 +3214,9 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   TuneResult best;
   double best_score = 1e30;
   auto consider = [&](double t, int kind, int group, int rows, int cap, int64_t nt, int block = 1024) {
-    const double score = (kind == 4 || kind == 5) ? 1.03 * t : t;
+    // and every layout has to beat the default route by 3%: noise otherwise
+    // decides between launches of 3 us
+    const double score = (kind == 4 || kind == 5) ? 1.03 * t : (kind == 7 ? 0.97 * t : t);
     if (score < best_score) {
       best_score = score;
       best = TuneResult{t, kind, group, rows, cap, nt, block};
@@ -3197,13 +3234,13 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
     build_row_groups(M, 0);
   }
   build_tiles(M, s);
-  if (M.tset[0].use.load())
-    consider(time_launches(s, reps, [&] { K == 1 ? k_spmv(M, x.p, y.p, s, fp32) : k_block_spmv(K, M, x.p, y.p, s, fp32); }),
-             7, 0, 0, 0, 0);
-  if (M.layout == L_MASS3 && K >= 2 && K <= 16) {
+  // 7: no layout set -- the node tiles or, for small matrices, the row kernels
+  const bool tiles = tiles_taken(M, K);
+  consider(time_candidate(s, reps, op), 7, 0, 0, 0, 0);
+  if (!tiles && M.layout == L_MASS3 && K >= 2 && K <= 16) {
     for (int G : {4, 8, 16, 32}) {
       M.wide[idx] = G;
-      consider(time_launches(s, reps, [&] { k_block_spmv(K, M, x.p, y.p, s, fp32); }), 4, 0, G, 0, 0);
+      consider(time_candidate(s, reps, op), 4, 0, G, 0, 0);
     }
     M.wide[idx] = 0;
   }
@@ -3212,33 +3249,41 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
     M.pipe = 0;
     for (int pw : {1, 2, 4, 8}) {
       build_row_groups(M, pw);
-      consider(time_launches(s, reps, [&] { k_spmv(M, x.p, y.p, s, fp32); }), 3, 0, pw, 0, 0);
+      consider(time_candidate(s, reps, op), 3, 0, pw, 0, 0);
     }
     build_row_groups(M, 0);
     for (int g : {8, 16, 32, 64}) {
       M.group = g;
-      consider(time_launches(s, reps, [&] { k_spmv(M, x.p, y.p, s, fp32); }), 0, g, 1, 0, 0);
+      consider(time_candidate(s, reps, op), 0, g, 1, 0, 0);
     }
     if (M.layout == L_BSR3)
       for (int g : {16, 32, 64})
         for (int pr : {2, 4, 8}) {
           M.group = g;
           M.pipe = pr;
-          consider(time_launches(s, reps, [&] { k_spmv(M, x.p, y.p, s, fp32); }), 6, g, pr, 0, 0);
+          consider(time_candidate(s, reps, op), 6, g, pr, 0, 0);
         }
     M.pipe = 0;
     M.group = 0;
   }
+  // the k-column kernels on one column: products and Chebyshev steps only, so
+  // not for 3x3 blocks
+  const bool blocked = K > 1 || mass;
+  if (K == 1) M.single_blocked = blocked;
   for (int R : {1, 2, 4, 8}) {
-    if (K * R > 64) continue;
+    if (K * R > 64 || !blocked) continue;
     M.block_map[idx] = R;
-    consider(time_launches(s, reps, [&] { k_block_spmv(K, M, x.p, y.p, s, fp32); }), 1, 0, R, 0, 0);
+    consider(time_candidate(s, reps, op), 1, 0, R, 0, 0);
   }
-  // tiled layouts: tile capacities on a geometric ladder from the longest
-  // row (a tile must hold one row) up to 64 KB of LDS per workgroup
+  // Where the node tiles are the default the LDS tiles and the wide layouts are
+  // not built: they lost by 10-70% at 51k to 1.9M DoF, and the ladder was most of
+  // the tuner's time (11 s at 1.9M DoF).  Nor are they below 2048 rows, where
+  // every layout takes the 3 us of a launch and the ladder took 0.1 s.  Else:
+  // tile capacities on a geometric ladder from the longest row (a tile must hold
+  // one row) up to 64 KB of LDS per workgroup
   int64_t longest = 0;
   for (int64_t r = 0; r < M.nb; ++r) longest = std::max(longest, M.h_browptr[r + 1] - M.h_browptr[r]);
-  const int limit = K <= 16 ? std::min(65535, tile_cap_limit(K)) : 0;  // no LDS tiles beyond K = 16
+  const int limit = K <= 16 && !tiles && blocked && M.nb >= 2048 ? std::min(65535, tile_cap_limit(K)) : 0;  // none beyond K = 16
   std::vector<int> caps;
   for (double f = 1.0; f * (double)longest <= (double)limit * 1.0001; f *= 1.28)
     caps.push_back((int)std::ceil(f * (double)longest));
@@ -3249,20 +3294,21 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
       if (K * R > 64) continue;
       for (int tb : {1024, 256}) {
         build_tiling(M, K, cap, R, tb);
-        consider(time_launches(s, reps, [&] { k_block_spmv(K, M, x.p, y.p, s, fp32); }), 2, 0, R, cap,
+        consider(time_candidate(s, reps, op), 2, 0, R, cap,
                  M.tiling[idx] ? M.tiling[idx]->ntiles : 0, tb);
       }
     }
     if (M.layout == L_MASS3 && K >= 2)
       for (int G : {4, 8, 16}) {
         build_tiling(M, K, cap, 1, 1024, G);
-        consider(time_launches(s, reps, [&] { k_block_spmv(K, M, x.p, y.p, s, fp32); }), 5, 0, G, cap,
+        consider(time_candidate(s, reps, op), 5, 0, G, cap,
                  M.tiling[idx] ? M.tiling[idx]->ntiles : 0, 1024);
       }
   }
   // apply the winner
   build_tiling(M, K, 0, 1);
   M.block_map[idx] = 0;
+  if (K == 1) M.single_blocked = false;
   M.tuned[idx] = true;
   if (best.kind == 7) {
     // no explicit layout: the node tiles

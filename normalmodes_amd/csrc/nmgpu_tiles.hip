@@ -654,6 +654,8 @@ static void launch_tile(const DevMat& M, const TilePlan& P, const VT* v, const X
   NMG_HIP(hipGetLastError());
 }
 
+bool tiles_taken(const DevMat& M, int K) { return tile_set(M, K, 8) != nullptr; }
+
 template <bool BSR, class XT, class Epi>
 static bool tile_product(const DevMat& M, const XT* x, int K, Epi epi, hipStream_t s, bool fp32,
                          std::initializer_list<const void*> others) {
