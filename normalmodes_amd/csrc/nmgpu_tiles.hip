@@ -155,8 +155,10 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
   if (q * 64 > (int64_t)1 << 30) return false;
   H.quads = q;
   // work units: the slices of a tile cut into runs of at most m quads, m the
-  // smallest that needs no more units than a workgroup has wavefronts; the
-  // runs of one slice after its first leave partial sums
+  // smallest that leaves no more partial sums (one for each run of a slice after
+  // its first) than a full tile has wavefronts to spare: short tiles would
+  // otherwise cost every workgroup LDS for up to 15 of them, and with it the
+  // second workgroup of a CU (223k DoF, K = 16, 128 rows: 63 us so, 43 now)
   H.un.assign(nt * waves, TileUnit{0, 1, 0, 0, 0, 0, -1, 0});
   H.max_extra = 0;
   for (int64_t t = 0; t < nt; ++t) {
@@ -169,7 +171,7 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
       return n;
     };
     int m = pack;
-    while (units(m) > waves) m += pack;
+    while (units(m) - ns > waves - spt) m += pack;
     int u = 0, extra = 0;
     for (int w = 0; w < waves; ++w) {
       H.un[t * waves + w].list = (int)first[t];
@@ -276,16 +278,20 @@ void fill_tile_values(DevMat& M, hipStream_t s, bool fp64) {
   }
 }
 
-// Rows of a tile.  Large matrices: as many as two workgroups per CU leave LDS
-// for -- 192 rows of up to 1400 nodes while a node takes at most 48 bytes (K <=
-// 2; FP32 vectors), 128 rows of up to 700 nodes at 96 bytes (K >= 4): at 1.9M
-// DoF K = 1 took 52 us with 192 rows against 65 with 128, K = 4 took 107 us
-// with 128 rows against 129 with 192 (one workgroup per CU); 96 rows for the
-// stiffness (K = 4: 360 us against 369 with 128).  Small ones: one tile per CU
-// (51.5k DoF, K = 4: 5.7 us with 80 rows, 6.3 with 48, 6.6 with 128).
+// Rows of a tile: as few as fill the rounds of 256 tiles, one to a CU, that
+// tiles of `most` rows need -- a round begun for a few tiles costs as much as a
+// full one (223k DoF, K = 1: 6.9 us with 160 rows, 466 tiles; 9.1 with 144 rows,
+// 517 tiles; 56.7k DoF, K = 4: 5.4 us with 80 rows, 237 tiles; 6.1 with 48, 6.5
+// with 128).  `most` is what the LDS of two workgroups per CU leaves room for:
+// at 24 or 48 bytes a node (K <= 2, FP32 vectors) 224 rows of up to 1400 nodes
+// (1.28M DoF, K = 1: 32.4 us, against 34.1 with 192 rows, 42.5 with 128 and 33.0
+// with 256), at 96 bytes (K >= 4) 128 rows of up to 700 nodes (K = 4: 64 us,
+// against 73 with 192 rows and 67 with 96), or 160 where that leaves two rounds
+// (223k DoF, K = 4: 13.5 us against 15.8 with 128); 96 rows for the stiffness
+// (439k DoF, K = 1: 62 us against 66 with 128).
 static int tile_rows(const DevMat& M, int most) {
-  const int64_t r = (M.nb + 256 * kSliceRows - 1) / (256 * kSliceRows) * kSliceRows;
-  return (int)std::min<int64_t>(r, most);
+  const int64_t round = 256 * std::max<int64_t>(1, (M.nb + 256 * most - 1) / (256 * most));
+  return (int)std::min<int64_t>((M.nb + round * kSliceRows - 1) / (round * kSliceRows) * kSliceRows, most);
 }
 
 void build_tiles(DevMat& M, hipStream_t s) {
@@ -294,12 +300,13 @@ void build_tiles(DevMat& M, hipStream_t s) {
   if (M.layout == L_CSR || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return;
   if (M.tset[0].use.load()) return;
   const bool bsr = M.layout == L_BSR3;
-  const int small = tile_rows(M, bsr ? 96 : 128), large = tile_rows(M, bsr ? 96 : 192);
-  for (int i = 0; i < (small == large ? 1 : 2); ++i) {
+  const int small = tile_rows(M, bsr ? 96 : (M.nb <= 512 * 160 ? 160 : 128)), large = bsr ? small : tile_rows(M, 224);
+  const bool two = small != large || small > 128;
+  for (int i = 0; i < (two ? 2 : 1); ++i) {
     TileSet& T = M.tset[i];
     if (!T.plan) {  // else: the pattern of the matrix this one was copied from
       HostTiles H;
-      const bool wide = i == 0 && small != large;
+      const bool wide = i == 0 && two;
       if (!tile_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), wide ? large : small, wide ? 1400 : 700,
                        bsr ? 8 : 16, bsr ? 1 : 2, H))
         break;

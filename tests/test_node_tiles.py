@@ -63,6 +63,7 @@ def _product(M, L, x, pack):
     x through the tile's list; later parts of a slice added to its first."""
     y = np.full((M.shape[0], x.shape[1]), np.nan)
     seen = np.zeros(M.nnz, dtype=int)
+    assert L["max_extra"] <= L["units"].shape[1] - L["spt"]  # short tiles included
     for tile in L["units"]:
         for w, (lst, nodes, row0, own, q0, nq, sl, part) in enumerate(tile):
             if sl < 0:
