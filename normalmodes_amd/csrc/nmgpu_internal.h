@@ -78,13 +78,31 @@ struct TileUnit {
   int slice;        // -1: none
   int part;         // part | parts << 8 | slot of the slice's first partial sum << 16
 };
+// A vector whose elements are left uninitialised by resize(): large tables that
+// the threads filling them should also be the first to touch.
+template <class T>
+struct RawAlloc : std::allocator<T> {
+  template <class U>
+  struct rebind {
+    using other = RawAlloc<U>;
+  };
+  template <class U>
+  void construct(U*) noexcept {}
+  template <class U, class A>
+  void construct(U* p, A&& a) {
+    ::new ((void*)p) U(std::forward<A>(a));
+  }
+};
+template <class T>
+using RawVec = std::vector<T, RawAlloc<T>>;
 struct HostTiles {
   int64_t ntiles = 0, quads = 0;
   int spt = 0, max_nodes = 0, max_extra = 0;
   std::vector<TileUnit> un;          // per tile and wavefront
   std::vector<int32_t> tcols;        // node lists, ascending
-  std::vector<uint16_t> lrow, eidx;  // row of each slice place within its tile (0xffff: none); entries' list places
-  std::vector<int32_t> perm;         // entry of each slot (-1: padding)
+  std::vector<uint16_t> lrow;        // row of each slice place within its tile (0xffff: none)
+  RawVec<uint16_t> eidx;             // entries' list places
+  RawVec<int32_t> perm;              // entry of each slot (-1: padding)
 };
 struct TilePlan {
   int64_t ntiles = 0, quads = 0;

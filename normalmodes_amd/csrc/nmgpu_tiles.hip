@@ -54,8 +54,8 @@ TilePlan::~TilePlan() {
     if (p) (void)hipFree(p);
 }
 
-template <class T>
-static T* to_device(const std::vector<T>& v) {
+template <class T, class A>
+static T* to_device(const std::vector<T, A>& v) {
   T* p = nullptr;
   NMG_HIP(hipMalloc(&p, sizeof(T) * std::max<size_t>(v.size(), 1)));
   const hipError_t e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
@@ -193,8 +193,8 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
     }
     H.max_extra = std::max(H.max_extra, extra);
   }
-  H.eidx.assign(q * 64, 0);
-  H.perm.assign(q * 64, -1);
+  H.eidx.resize(q * 64);
+  H.perm.resize(q * 64);
   // Entries of a row in an order that spreads the simultaneous LDS reads of
   // four neighbouring rows over the banks: row i of a slice takes at place e
   // an entry whose node's place in the list is (e + i) mod 4, while it has one
@@ -206,7 +206,9 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
     for (int64_t t = 0; t < nt; ++t) {
       const Cut& c = *cut[t];
       for (size_t i = 0; i < c.nodes.size(); ++i) local[c.nodes[i]] = (uint16_t)i;
-      for (int64_t s = t * spt; s < (t + 1) * spt; ++s)
+      for (int64_t s = t * spt; s < (t + 1) * spt; ++s) {
+        std::fill_n(H.eidx.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, (uint16_t)0);
+        std::fill_n(H.perm.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, -1);
         for (int j = 0; j < kSliceRows; ++j) {
           if (H.lrow[s * kSliceRows + j] == 0xffff) continue;
           const int64_t r = c.r0 + H.lrow[s * kSliceRows + j];
@@ -219,22 +221,15 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
                 if (by[b].size() > by[cl].size()) cl = b;
             const int64_t k = by[cl].back();
             by[cl].pop_back();
-            const int64_t slot = (sd[s].x + e / 4) * 64 + j * 4 + e % 4;
-            H.eidx[slot] = local[ci[k]];
-            H.perm[slot] = (int32_t)k;
+            const int64_t quad = sd[s].x + e / 4, l = j * 4 + e % 4;
+            // the two indices of a pair of quads side by side
+            H.eidx[pack == 2 ? quad / 2 * 128 + 2 * l + quad % 2 : quad * 64 + l] = local[ci[k]];
+            H.perm[quad * 64 + l] = (int32_t)k;
           }
         }
+      }
     }
   }
-  if (pack == 2)  // the two indices of a pair of quads side by side
-    for (int64_t p = 0; p < q / 2; ++p) {
-      uint16_t t[128];
-      for (int l = 0; l < 64; ++l) {
-        t[2 * l] = H.eidx[p * 128 + l];
-        t[2 * l + 1] = H.eidx[p * 128 + 64 + l];
-      }
-      std::copy(t, t + 128, H.eidx.begin() + p * 128);
-    }
   return true;
 }
 
@@ -294,21 +289,30 @@ static int tile_rows(const DevMat& M, int most) {
   return (int)std::min<int64_t>((M.nb + round * kSliceRows - 1) / (round * kSliceRows) * kSliceRows, most);
 }
 
+// Scalar masses of few rows take a second plan of twice the rows for K >= 16:
+// four workgroups or more share a tile's rows there, one per four columns, and
+// half the tiles, with fewer reads of x per row, fill the CUs as well (K = 16:
+// 10.6k DoF 8.2 us with 16 rows, 6.1 with 32; 20.1k 9.8 : 7.6; 38.8k 12.4 : 10.7;
+// 56.7k 15.2 : 13.5; K = 8 5.1 : 4.6, 5.7 : 5.3, 6.9 : 6.8 and 7.9 : 8.1).
+static int deep_rows(const DevMat& M) { return (int)((M.nb + 128 * kSliceRows - 1) / (128 * kSliceRows) * kSliceRows); }
+static bool deep_tiles(const DevMat& M) { return M.layout == L_MASS3 && M.nb <= 128 * 160; }
+
 void build_tiles(DevMat& M, hipStream_t s) {
   static std::mutex mu;  // two solvers may set up on one matrix at once
   std::lock_guard<std::mutex> lk(mu);
   if (M.layout == L_CSR || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return;
   if (M.tset[0].use.load()) return;
   const bool bsr = M.layout == L_BSR3;
-  const int small = tile_rows(M, bsr ? 96 : (M.nb <= 512 * 160 ? 160 : 128)), large = bsr ? small : tile_rows(M, 224);
-  const bool two = small != large || small > 128;
+  const int rows0 = tile_rows(M, bsr ? 96 : 224);
+  const int rows1 = bsr ? rows0 : (deep_tiles(M) ? deep_rows(M) : tile_rows(M, M.nb <= 512 * 160 ? 160 : 128));
+  const bool two = rows0 != rows1 || (!bsr && rows0 > 128);
   for (int i = 0; i < (two ? 2 : 1); ++i) {
     TileSet& T = M.tset[i];
     if (!T.plan) {  // else: the pattern of the matrix this one was copied from
       HostTiles H;
-      const bool wide = i == 0 && two;
-      if (!tile_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), wide ? large : small, wide ? 1400 : 700,
-                       bsr ? 8 : 16, bsr ? 1 : 2, H))
+      const int cap = i == 0 && two && !deep_tiles(M) ? 1400 : 700;
+      if (!tile_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), i == 0 ? rows0 : rows1, cap, bsr ? 8 : 16,
+                       bsr ? 1 : 2, H))
         break;
       auto P = std::make_shared<TilePlan>();
       P->ntiles = H.ntiles;
@@ -341,7 +345,7 @@ static const TileSet* tile_set(const DevMat& M, int K, int size) {
   if (M.layout == L_CSR || !M.tile_use(K)) return nullptr;
   const int64_t least = M.layout == L_BSR3 ? (K == 1 ? 65536 : 1024) : (K >= 8 ? 1 : 2048);
   if (M.nb < least) return nullptr;
-  const int i = M.tset[1].use.load() && std::min(K, 4) * size > 16 ? 1 : 0;
+  const int i = M.tset[1].use.load() && (deep_tiles(M) ? K >= 16 : std::min(K, 4) * size > 16) ? 1 : 0;
   return M.tset[i].use.load() ? &M.tset[i] : nullptr;
 }
 

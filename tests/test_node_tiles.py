@@ -127,7 +127,7 @@ def _handles(M, kind, seed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,nb,long_row", [
     ("mass", 2048, 0), ("mass", 2049, 0), ("mass", 6000, 300), ("mass", 40000, 0), ("mass", 3000, 1500), ("mass", 40, 0),
-    ("bsr", 1024, 0), ("bsr", 1025, 300), ("bsr", 30000, 0), ("bsr", 66000, 0)])
+    ("mass", 20480, 0), ("mass", 20481, 0), ("bsr", 1024, 0), ("bsr", 1025, 300), ("bsr", 30000, 0), ("bsr", 66000, 0)])
 def test_products(kind, nb, long_row):
     """A x (or B x) on 1 to 64 columns, FP64 and FP32 values; the filter's fused
     step through it on the same matrix as A~ of a diagonal-mass pencil."""
