@@ -342,8 +342,12 @@ int nmg_set_split_filter(nmg_handle h, int on);
  * executable graph per distinct set of buffers, so that a solve costs one
  * host launch instead of one per step (no reference counterpart; on = 0 or
  * 1, default 0).  A change of the B matrix's kernel layout (autotuning,
- * tiling, value order, …) retires the graphs captured before it. */
+ * tiling, value order, …) or of the solve (another handle, refinement)
+ * retires the graphs captured before it. */
 int nmg_set_graphs(nmg_handle h, int on);
+/* distinct sets of buffers seen and solves replayed from a graph so far (no
+ * reference counterpart); null pointers are skipped */
+int nmg_graph_stats(nmg_handle h, int *cached, int64_t *replays);
 /* Progress of long solves (no reference counterpart): a line on stderr
  * every `every` Lanczos steps of nmg_lanbounds, nmg_cheblannr and
  * nmg_solve_slices (0, the default: silent). */

@@ -446,6 +446,10 @@ struct FVec {
 
 struct Cheb {
   DevMat* mat = nullptr;
+  // process-unique, and new with every change of how the solve runs: captured
+  // graphs hold buffers of the solve and are keyed on it, since a solve made
+  // after another was freed can lie at the same address with the same bounds
+  uint64_t gen = next_layout_gen();
   double lmin = 0, lmax = 0;
   int deg = 0;
   int64_t ncalls = 0, nmatvec = 0;
@@ -609,7 +613,8 @@ struct Solver {
   bool graphs = false;
   struct GraphKey {
     const void* p[24];
-    uint64_t gen;  // layout generation of the matrix
+    uint64_t gen;       // layout generation of the matrix
+    uint64_t cheb_gen;  // generation of the solve
     int K, parts, fp32, deg, mode;
     double lmin, lmax;
   };
@@ -619,6 +624,7 @@ struct Solver {
     hipGraphExec_t exec;
   };
   std::vector<GraphEntry> gcache;
+  int64_t graph_replays = 0;
   void drop_graphs() {
     // a launched graph may still run on the stream: let it finish first
     if (s && !gcache.empty()) (void)hipStreamSynchronize(s);
@@ -701,6 +707,7 @@ static void run_graphed(Solver& S, const Solver::GraphKey& key, F&& body) {
     }
   if (hit && hit->exec) {
     NMG_HIP(hipGraphLaunch(hit->exec, S.s));
+    S.graph_replays++;
     return;
   }
   if (!hit) {
@@ -745,6 +752,7 @@ static Solver::GraphKey graph_key(const Solver& S, const Cheb& C, int K, int par
   k.p[3] = &C;
   k.p[4] = C.mat;
   k.gen = C.mat->gen;
+  k.cheb_gen = C.gen;
   k.mode = C.mode;
   for (int i = 0; i < 3 * parts && i < 12; ++i) k.p[5 + i] = S.hb[i].p;
   for (int i = 0; i < 4; ++i) k.p[17 + i] = S.hf[i].p;
@@ -2882,6 +2890,14 @@ int nmg_set_graphs(nmg_handle h, int on) {
   });
 }
 
+int nmg_graph_stats(nmg_handle h, int* cached, int64_t* replays) {
+  return guarded([&] {
+    Solver* S = get<Solver>(h, K_SOLVER);
+    if (cached) *cached = (int)S->gcache.size();
+    if (replays) *replays = S->graph_replays;
+  });
+}
+
 int nmg_set_block_size(nmg_handle h, int block) {
   return guarded([&] {
     Solver* S = get<Solver>(h, K_SOLVER);
@@ -3764,6 +3780,7 @@ int nmg_chebiter_set_refine(nmg_handle cheb, int passes, int inner_deg) {
       make_fp32(*C->mat, default_stream());
       NMG_HIP(hipStreamSynchronize(default_stream()));
     }
+    C->gen = next_layout_gen();
     C->refine = passes;
     C->inner_deg = passes > 0 ? inner_deg : 0;
     // the single-column solve's FP32 work, allocated here so that a solve

@@ -349,6 +349,13 @@ def set_graphs(h: Handle, on: bool = True):
     _check(_lib().nmg_set_graphs(_i64(h), ctypes.c_int(int(bool(on)))))
 
 
+def graph_stats(h: Handle):
+    """(distinct sets of buffers seen, solves replayed from a graph so far)."""
+    n, r = ctypes.c_int(), ctypes.c_int64()
+    _check(_lib().nmg_graph_stats(_i64(h), ctypes.byref(n), ctypes.byref(r)))
+    return n.value, r.value
+
+
 def set_split_streams(h: Handle, parts: int = 2):
     """k-column B-solves in `parts` (2 or 4) concurrent parts on as many streams; 0 turns it off."""
     _check(_lib().nmg_set_split_streams(_i64(h), ctypes.c_int(int(parts))))

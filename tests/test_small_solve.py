@@ -81,3 +81,51 @@ def test_small_solve(nb, per_row, long_row):
         for f, v in handles:
             f(v)
         pv.csr_free(m)
+
+
+def _open(n, m, ch, graphs=False):
+    h = pv.pevsl_start(0)
+    pv.pevsl_setprobsizes(h, n, n, -1)
+    pv.pevsl_setbmv(h, m)
+    pv.pevsl_setbsol_chebiter(h, 2, ch)
+    pv.pevsl_setamv(h, m)
+    pv.pevsl_set_geneig(h)
+    pv.set_graphs(h, graphs)
+    return h
+
+
+@pytest.mark.parametrize("nb", [300, 2300])
+def test_graphs_belong_to_one_solve(nb):
+    """A graph captured from one Chebyshev solve is not replayed for another
+    with the same bounds and degree (which may lie where the freed one lay),
+    nor after the solve's refinement changed."""
+    D = sp.kron(_mass(nb, 12, nb), sp.identity(3), format="csr")
+    D.sort_indices()
+    n, lo, hi, deg = D.shape[0], 1.0, 3.0, 12
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    rng = np.random.default_rng(3)
+    ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+    eager, graph = _open(n, m, ch), _open(n, m, ch, graphs=True)
+    try:
+        for K in (1, 2):
+            for new in ("first", "another solve", "one coarse pass", "no passes"):
+                if new == "another solve":
+                    pv.pevsl_chebiter_free(ch)
+                    ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+                    for h in (eager, graph):
+                        pv.pevsl_setbsol_chebiter(h, 2, ch)
+                elif new == "one coarse pass":
+                    pv.chebiter_set_refine(ch, 1, 1)
+                elif new == "no passes":
+                    pv.chebiter_set_refine(ch, 0)
+                before = pv.graph_stats(graph)[1]
+                for i in range(4):  # eager first use, capture, replays
+                    X = rng.standard_normal((K, n))
+                    want, got = pv.apply_block(eager, 2, X), pv.apply_block(graph, 2, X)
+                    assert np.linalg.norm(got - want) <= 1e-15 * np.linalg.norm(want), (K, new, i)
+                    assert pv.graph_stats(graph)[1] - before == max(0, i - 1), (K, new, i)
+    finally:
+        pv.pevsl_finish(eager)
+        pv.pevsl_finish(graph)
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
