@@ -464,10 +464,6 @@ struct Cheb {
   // Chebyshev solve of degree inner_deg with FP32 values and FP32 iterates
   // on the FP64 residual b - B~x of the sum so far, added in FP64
   int refine = 0, inner_deg = 0;
-  // one-launch solve of a small system (null: the matrix does not fit), with
-  // the step weights w_1 .. w_deg on the device
-  std::shared_ptr<const SmallPlan> small;
-  DVec wts;
   FVec own32;           // inner work (3 n K floats) when the caller brings none
   PersistPlan plan[2];  // FP64 / FP32 values
   bool planned[2] = {false, false};
@@ -765,18 +761,21 @@ static Solver::GraphKey graph_key(const Solver& S, const Cheb& C, int K, int par
   return k;
 }
 
+// The whole solve of K columns in one launch where the matrix is small enough
+// (nmgpu_small.hip) and no layout was set explicitly for that width.  It reads
+// buffers of the matrix only, as the step launches do: a graph that captured it
+// stays valid while the matrix lives.
+static bool small_solve(const Cheb& C, int K, const double* b, double* out, hipStream_t s, bool fp32) {
+  if (!C.mat->small_use(K)) return false;
+  k_cheb_small(*C.mat, K, C.deg, C.lmin, C.lmax, b, out, s, fp32);
+  return true;
+}
+
 // x ~ B~^{-1} b by the Chebyshev semi-iteration (x_0 = 0, deg products):
 //   x_1 = b/th,  x_{k+1} = x_{k-1} + w_{k+1}(x_k - x_{k-1} + (b - B x_k)/th),
 //   w_1 = 2, w_{k+1} = 1/(1 - w_k/(4 s^2)), th = (lmax+lmin)/2, s = th/de.
 // The result lands in `out`; `tmp` is a second buffer.
-// The whole solve of K columns in one launch where the matrix is small enough
-// (nmgpu_small.hip) and no layout was set explicitly for that width.
-static bool small_solve(const Cheb& C, int K, const double* b, double* out, hipStream_t s, bool fp32) {
-  if (!C.small || !C.mat->small_use(K)) return false;
-  k_cheb_small(*C.small, *C.mat, K, C.deg, 2.0 / (C.lmax + C.lmin), C.wts.p, b, out, s, fp32);
-  return true;
-}
-
+//
 // The Chebyshev semi-iteration as one fused launch per step: x_1 = b/th,
 // x_0 = 0 (cleared here), x_{k+1} from the fused product + update; the
 // iterates alternate between out and tmp so that the last lands in out.
@@ -862,7 +861,7 @@ static void cheb_solve(Cheb& C, const double* b, double* out, double* tmp, hipSt
     return;
   }
   const bool pr = probe && probe->armed();
-  if (C.small && C.mat->small_use(1)) {  // a sampled solve is bracketed whole
+  if (C.mat->small_use(1)) {  // a sampled solve is bracketed whole
     if (pr) probe->before(s);
     small_solve(C, 1, b, out, s, fp32);
     if (pr) probe->after(s);
@@ -1425,7 +1424,7 @@ static void block_cheb(Cheb& C, int K, const double* b, double* out, double* tmp
     return;
   }
   const bool pr = probe && probe->armed();
-  if (C.small && C.mat->small_use(K)) {  // a sampled solve is bracketed whole
+  if (C.mat->small_use(K)) {  // a sampled solve is bracketed whole
     if (pr) probe->before(s);
     small_solve(C, K, b, out, s, fp32);
     if (pr) probe->after(s);
@@ -2531,20 +2530,12 @@ int nmg_setup_chebiter(double lmin, double lmax, int deg, nmg_handle mat, nmg_ha
     NMG_CHECK(deg >= 1 && deg <= 100000, NMG_EINVAL, "chebiter degree must be >= 1");
     NMG_CHECK(M->nrow == M->ncol, NMG_EINVAL, "chebiter needs a square matrix");
     build_tiles(*M, default_stream());
+    build_small(*M);
     std::unique_ptr<Cheb> C(new Cheb());
     C->mat = M;
     C->lmin = lmin;
     C->lmax = lmax;
     C->deg = deg;
-    C->small = plan_small(*M);
-    if (C->small) {
-      std::vector<double> w(deg);
-      const double sg = (lmax + lmin) / (lmax - lmin);
-      double wk = 2.0;
-      for (int k = 0; k < deg; ++k) w[k] = wk = 1.0 / (1.0 - wk / (4.0 * sg * sg));
-      C->wts.ensure(deg);
-      NMG_HIP(hipMemcpy(C->wts.p, w.data(), sizeof(double) * deg, hipMemcpyHostToDevice));
-    }
     *cheb = reg(C.release(), K_CHEB);
   });
 }

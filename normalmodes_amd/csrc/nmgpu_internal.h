@@ -133,7 +133,7 @@ struct HostSmall {
 };
 struct SmallPlan {
   int quads = 0, slices = 0;
-  uint32_t* head = nullptr;
+  uint32_t* ends = nullptr;
   uint16_t* rows = nullptr;
   uint16_t* eidx = nullptr;
   int32_t* perm = nullptr;
@@ -209,7 +209,9 @@ struct DevMat {
     for (int i = 0; i < 7; ++i)
       if ((1 << i) == K) tuned[i] = false;
   }
+  std::shared_ptr<const SmallPlan> small;  // one-launch solves (null: the matrix does not fit, or no solve was set up)
   bool small_use(int K) const {
+    if (!small) return false;
     for (int i = 0; i < 7; ++i)
       if ((1 << i) == K) return tuned[i] || tile_use(K);
     return false;
@@ -291,12 +293,12 @@ bool k_tile_cheb_step32(int K, const DevMat& M, const float* b, const float* xk,
 bool k_tile_filter_step(int K, const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
                         const double* mu, double mu0, double t, double cc, bool first, hipStream_t s, bool fp32);
 
-// one-launch solves of small systems: null when M does not fit; x ~ M^-1 b on K
-// interleaved columns by deg steps with the weights wts[deg] (device)
+// one-launch solves of small systems: M.small is set when M fits; x ~ M^-1 b on
+// K interleaved columns by deg steps for the bounds lmin, lmax
 bool small_layout(int64_t nb, const int64_t* rp, const int32_t* ci, HostSmall& H);
-std::shared_ptr<const SmallPlan> plan_small(const DevMat& M);
-void k_cheb_small(const SmallPlan& P, const DevMat& M, int K, int deg, double ith, const double* wts, const double* b,
-                  double* out, hipStream_t s, bool fp32);
+void build_small(DevMat& M);
+void k_cheb_small(const DevMat& M, int K, int deg, double lmin, double lmax, const double* b, double* out,
+                  hipStream_t s, bool fp32);
 
 // ---------------------------------------------------------------------------
 // kernel launchers (nmgpu_kernels.hip); all asynchronous on stream s

@@ -21,7 +21,9 @@
 // and step at 614 nodes).  Reading each slice's rows and iterates from LDS at
 // its end took 1.06 us at 614 nodes; 32 quads per wavefront spill (2.7 us).
 #include <algorithm>
+#include <cmath>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <vector>
 
@@ -35,7 +37,7 @@ constexpr int kSmallQuads = 24;  // quads per wavefront that the registers hold
 constexpr int kSmallWeights = 1024;
 
 SmallPlan::~SmallPlan() {
-  for (void* p : {(void*)head, (void*)rows, (void*)eidx, (void*)perm})
+  for (void* p : {(void*)ends, (void*)rows, (void*)eidx, (void*)perm})
     if (p) (void)hipFree(p);
 }
 
@@ -128,18 +130,20 @@ static T* upload(const std::vector<T>& v) {
   return p;
 }
 
-std::shared_ptr<const SmallPlan> plan_small(const DevMat& M) {
-  if (M.layout != L_MASS3 || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return nullptr;
+void build_small(DevMat& M) {
+  static std::mutex mu;  // two solves may be set up on one matrix at once
+  std::lock_guard<std::mutex> lk(mu);
+  if (M.small || M.layout != L_MASS3 || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return;
   HostSmall H;
-  if (!small_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), H)) return nullptr;
+  if (!small_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), H)) return;
   auto P = std::make_shared<SmallPlan>();
   P->quads = H.quads;
   P->slices = H.slices;
-  P->head = upload(H.ends);
+  P->ends = upload(H.ends);
   P->rows = upload(H.rows);
   P->eidx = upload(H.eidx);
   P->perm = upload(H.perm);
-  return P;
+  M.small = P;
 }
 
 struct SmallView {
@@ -150,13 +154,24 @@ struct SmallView {
   int slices;
 };
 
+// Step weights of the semi-iteration: the recurrence w_0 = 2, w_k = 1/(1 -
+// w_{k-1}/(4 s^2)), s = (lmax + lmin)/(lmax - lmin), is w_k = 2 s T_k(s)/T_{k+1}(s)
+// (T_k the Chebyshev polynomials), so with s = cosh a each weight stands by
+// itself: w_k = 2 s e^-a (1 + e^{-2ka})/(1 + e^{-2(k+1)a}).
+struct SmallWeights {
+  double a, first;  // a, 2 s e^-a
+  __device__ __forceinline__ double operator()(int k) const {
+    return first * (1.0 + exp(-2.0 * k * a)) / (1.0 + exp(-2.0 * (k + 1) * a));
+  }
+};
+
 // Slice sl of a wavefront belongs to the lanes with (lane & 3) == sl & 3: after
 // a row's four lanes have its sum, that one keeps it, so the update of up to
 // four slices runs once, on all 64 lanes, with b and both iterates of a lane's
 // own rows in registers (NS rows for up to 4 NS slices).
 template <int QW, int NS, class VT>
 __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, const VT* __restrict__ val, int nb, int K,
-                                                                 int deg, double ith, const double* __restrict__ wts,
+                                                                 int deg, double ith, SmallWeights wts,
                                                                  const double* __restrict__ b,
                                                                  double* __restrict__ out) {
   extern __shared__ double small_lds[];  // two iterates of nb values, then the step weights
@@ -187,12 +202,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
     xo[j] = bo[j] * ith;
     mo[j] = 0.0;
   }
-  // step weights in LDS, kSmallWeights at a time: a global load per step costs
-  // more than the step
+  // step weights in LDS, kSmallWeights at a time, one per thread
   double* const ws = small_lds + 2 * nb;
   for (int k = 0; k < deg; ++k) {
     if (k % kSmallWeights == 0)
-      for (int i = tid; i < kSmallWeights && k + i < deg; i += 64 * kSmallWaves) ws[i] = wts[k + i];
+      for (int i = tid; i < kSmallWeights && k + i < deg; i += 64 * kSmallWaves) ws[i] = wts(k + i + 1);
     if (k % kSmallWeights == 0) __syncthreads();
     const double w = ws[k % kSmallWeights];
     const uint32_t from = k & 1 ? (uint32_t)nb * 8 : 0;
@@ -241,9 +255,9 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
 }
 
 template <int QW, class VT>
-static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const double* wts,
+static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, SmallWeights wts,
                            const double* b, double* out, hipStream_t s) {
-  const SmallView V{P.head, P.rows, P.eidx, P.perm, P.slices};
+  const SmallView V{P.ends, P.rows, P.eidx, P.perm, P.slices};
   const size_t lds = (size_t)nb * 16 + (size_t)std::min(deg, kSmallWeights) * 8;
   const dim3 grid(3 * (unsigned)K), tb(64 * kSmallWaves);
   if (P.slices <= 4)
@@ -256,7 +270,7 @@ static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int
 }
 
 template <class VT>
-static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const double* wts,
+static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, SmallWeights wts,
                          const double* b, double* out, hipStream_t s) {
   switch (P.quads) {
     case 8: launch_small_q<8>(P, val, nb, K, deg, ith, wts, b, out, s); break;
@@ -265,10 +279,14 @@ static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int d
   }
 }
 
-void k_cheb_small(const SmallPlan& P, const DevMat& M, int K, int deg, double ith, const double* wts, const double* b,
-                  double* out, hipStream_t s, bool fp32) {
-  if (fp32 && M.bval32) launch_small(P, (const float*)M.bval32, (int)M.nb, K, deg, ith, wts, b, out, s);
-  else launch_small(P, (const double*)M.bval, (int)M.nb, K, deg, ith, wts, b, out, s);
+void k_cheb_small(const DevMat& M, int K, int deg, double lmin, double lmax, const double* b, double* out,
+                  hipStream_t s, bool fp32) {
+  const SmallPlan& P = *M.small;
+  // cosh a = 1 + e with e = 2 lmin/(lmax - lmin), small for ill-conditioned matrices
+  const double e = 2.0 * lmin / (lmax - lmin), a = std::log1p(e + std::sqrt(e * (2.0 + e))), ith = 2.0 / (lmax + lmin);
+  const SmallWeights w{a, 2.0 * (1.0 + e) * std::exp(-a)};
+  if (fp32 && M.bval32) launch_small(P, (const float*)M.bval32, (int)M.nb, K, deg, ith, w, b, out, s);
+  else launch_small(P, (const double*)M.bval, (int)M.nb, K, deg, ith, w, b, out, s);
 }
 
 }  // namespace nmg

@@ -2,6 +2,8 @@
 recurrence in numpy and against the step-by-step kernels (a layout set by hand
 turns the one-launch form off), at one node, empty and long rows, the sizes
 around its limits, 1 to 64 columns, FP64 and FP32 values."""
+import ctypes
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -127,5 +129,104 @@ def test_graphs_belong_to_one_solve(nb):
     finally:
         pv.pevsl_finish(eager)
         pv.pevsl_finish(graph)
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+class _Hip:
+    """The HIP runtime that the library is linked to."""
+
+    def __init__(self):
+        pv._lib()
+        self.h = ctypes.CDLL("libamdhip64.so")
+
+    def __getattr__(self, name):
+        def call(*args):
+            assert getattr(self.h, name)(*args) == 0, name
+        return call
+
+
+@pytest.mark.parametrize("nb", [300, 2300])
+def test_captured_solve_outlives_its_handle(nb):
+    """A caller's own graph of nmg_chebiter_noalloc holds the matrix and the
+    caller's vectors only: replayed on new inputs after the solve's handle was
+    freed and another solve was set up, with eager solves in between."""
+    D = sp.kron(_mass(nb, 12, nb), sp.identity(3), format="csr")
+    D.sort_indices()
+    n, vp = D.shape[0], ctypes.c_void_p
+    lib, hip, rng = pv._lib(), _Hip(), np.random.default_rng(6)
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    ch = pv.pevsl_setup_chebiter(1.0, 3.0, 20, m)
+    b, x, s, g, ex = vp(), vp(), vp(), vp(), vp()
+    for p in (b, x):
+        hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(8 * n))
+    hip.hipStreamCreate(ctypes.byref(s))
+
+    def replay(want_of):
+        v, out = rng.standard_normal(n), np.empty(n)
+        hip.hipMemcpy(b, v.ctypes.data_as(vp), ctypes.c_size_t(8 * n), 1)
+        hip.hipGraphLaunch(ex, s)
+        hip.hipStreamSynchronize(s)
+        hip.hipMemcpy(out.ctypes.data_as(vp), x, ctypes.c_size_t(8 * n), 2)
+        want = pv.pevsl_chebiter(2, v, want_of)
+        assert np.linalg.norm(out - want) <= 1e-15 * np.linalg.norm(want)
+
+    def noalloc():
+        pv._check(lib.nmg_chebiter_noalloc(ctypes.c_int(2), b, x, ctypes.c_int64(ch), s))
+
+    try:
+        noalloc()
+        hip.hipStreamSynchronize(s)
+        hip.hipStreamBeginCapture(s, 1)                    # thread local
+        noalloc()
+        hip.hipStreamEndCapture(s, ctypes.byref(g))
+        hip.hipGraphInstantiate(ctypes.byref(ex), g, None, None, ctypes.c_size_t(0))
+        for _ in range(3):
+            replay(ch)
+        pv.pevsl_chebiter_free(ch)
+        others = [pv.pevsl_setup_chebiter(0.5, 7.0, 20, m) for _ in range(3)]
+        ch = pv.pevsl_setup_chebiter(1.0, 3.0, 20, m)
+        for _ in range(3):
+            replay(ch)
+        for o in others:
+            pv.pevsl_chebiter_free(o)
+        hip.hipGraphExecDestroy(ex)
+        hip.hipGraphDestroy(g)
+    finally:
+        hip.hipFree(b)
+        hip.hipFree(x)
+        hip.hipStreamDestroy(s)
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@pytest.mark.parametrize("lo,hi,deg", [(1.0, 3.0, 1500), (1e-3, 1.0, 400), (1e-6, 1.0, 2500), (0.999, 1.0, 3)])
+def test_small_solve_weights(lo, hi, deg):
+    """The one-launch solve's step weights from their closed form, over the
+    chunks of a long solve and from ill- to well-conditioned bounds, against
+    the recurrence: diagonal systems, whose every entry is one polynomial of
+    its eigenvalue."""
+    nb = 48
+    lam = np.linspace(lo, hi, nb)
+    D = sp.kron(sp.diags(lam), sp.identity(3), format="csr")
+    th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
+    rng = np.random.default_rng(8)
+    b = rng.standard_normal(3 * nb)
+    xm, xk, w = np.zeros(3 * nb, np.longdouble), b / np.longdouble(th), np.longdouble(2.0)
+    d = np.repeat(lam, 3).astype(np.longdouble)
+    for _ in range(deg):
+        w = 1 / (1 - w / (4 * np.longdouble(sg) ** 2))
+        xm, xk = xk, xm + w * (xk - xm + (b - d * xk) / np.longdouble(th))
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+    try:
+        assert pv.csr_info(m)["layout"] == "mass3"
+        got = pv.pevsl_chebiter(2, b, ch)
+        pv.set_kernel_map(m, 32)                           # by hand: step by step
+        step = pv.pevsl_chebiter(2, b, ch)
+        err = [float(np.linalg.norm(v - xk) / np.linalg.norm(xk)) for v in (got, step)]
+        # rounding of the iteration itself grows with deg and the condition
+        assert err[0] <= 2.0 * err[1] + 1e-15 * min(deg, hi / lo), err
+    finally:
         pv.pevsl_chebiter_free(ch)
         pv.csr_free(m)
