@@ -765,10 +765,11 @@ static Solver::GraphKey graph_key(const Solver& S, const Cheb& C, int K, int par
 // (nmgpu_small.hip) and no layout was set explicitly for that width.  It reads
 // buffers of the matrix only, as the step launches do: a graph that captured it
 // stays valid while the matrix lives.
-static bool small_solve(const Cheb& C, int K, const double* b, double* out, hipStream_t s, bool fp32) {
-  if (!C.mat->small_use(K)) return false;
+static bool small_taken(const Cheb& C, int K) {
+  return C.mat->small_use(K) && small_steps(C.deg, C.lmin, C.lmax);
+}
+static void small_solve(const Cheb& C, int K, const double* b, double* out, hipStream_t s, bool fp32) {
   k_cheb_small(*C.mat, K, C.deg, C.lmin, C.lmax, b, out, s, fp32);
-  return true;
 }
 
 // x ~ B~^{-1} b by the Chebyshev semi-iteration (x_0 = 0, deg products):
@@ -861,7 +862,7 @@ static void cheb_solve(Cheb& C, const double* b, double* out, double* tmp, hipSt
     return;
   }
   const bool pr = probe && probe->armed();
-  if (C.mat->small_use(1)) {  // a sampled solve is bracketed whole
+  if (small_taken(C, 1)) {  // a sampled solve is bracketed whole
     if (pr) probe->before(s);
     small_solve(C, 1, b, out, s, fp32);
     if (pr) probe->after(s);
@@ -1424,7 +1425,7 @@ static void block_cheb(Cheb& C, int K, const double* b, double* out, double* tmp
     return;
   }
   const bool pr = probe && probe->armed();
-  if (C.mat->small_use(K)) {  // a sampled solve is bracketed whole
+  if (small_taken(C, K)) {  // a sampled solve is bracketed whole
     if (pr) probe->before(s);
     small_solve(C, K, b, out, s, fp32);
     if (pr) probe->after(s);
@@ -2599,7 +2600,9 @@ int nmg_chebiter_noalloc(int type, const double* b, double* x, nmg_handle cheb, 
     NMG_CHECK(n <= kScratchDoubles, NMG_EINVAL,
               "nmg_chebiter_noalloc: the matrix has more rows than the scratch array holds (4194304)");
     double* tmp = scratch_on_current_device();
-    if (!small_solve(*C, 1, b, x, static_cast<hipStream_t>(stream), false))
+    if (small_taken(*C, 1))
+      small_solve(*C, 1, b, x, static_cast<hipStream_t>(stream), false);
+    else
       cheb_steps(*C, b, x, tmp, static_cast<hipStream_t>(stream), false, nullptr);
     NMG_HIP(hipGetLastError());
     C->ncalls++;

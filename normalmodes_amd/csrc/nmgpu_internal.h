@@ -297,6 +297,9 @@ bool k_tile_filter_step(int K, const DevMat& A, const double* x, const double* v
 // K interleaved columns by deg steps for the bounds lmin, lmax
 bool small_layout(int64_t nb, const int64_t* rp, const int32_t* ci, HostSmall& H);
 void build_small(DevMat& M);
+// whether the weights of a solve of that many steps are held or have settled (to
+// rounding) before the last one held: deg <= 8192, or lmax/lmin below 8e5
+bool small_steps(int deg, double lmin, double lmax);
 void k_cheb_small(const DevMat& M, int K, int deg, double lmin, double lmax, const double* b, double* out,
                   hipStream_t s, bool fp32);
 

@@ -34,7 +34,7 @@ namespace nmg {
 
 constexpr int kSmallWaves = 16;
 constexpr int kSmallQuads = 24;  // quads per wavefront that the registers hold
-constexpr int kSmallWeights = 1024;
+constexpr int kSmallWeights = 8192;  // step weights held in LDS; longer solves repeat the last
 
 SmallPlan::~SmallPlan() {
   for (void* p : {(void*)ends, (void*)rows, (void*)eidx, (void*)perm})
@@ -156,14 +156,31 @@ struct SmallView {
 
 // Step weights of the semi-iteration: the recurrence w_0 = 2, w_k = 1/(1 -
 // w_{k-1}/(4 s^2)), s = (lmax + lmin)/(lmax - lmin), is w_k = 2 s T_k(s)/T_{k+1}(s)
-// (T_k the Chebyshev polynomials), so with s = cosh a each weight stands by
-// itself: w_k = 2 s e^-a (1 + e^{-2ka})/(1 + e^{-2(k+1)a}).
+// (T_k the Chebyshev polynomials), so with s = cosh a and r = e^-2a each weight
+// stands by itself: w_k = 2 s e^-a (1 + r^k)/(1 + r^{k+1}), and a launch needs no
+// buffer of them that would have to outlive it.
 struct SmallWeights {
-  double a, first;  // a, 2 s e^-a
+  static constexpr int kBits = 14;  // k <= kSmallWeights
+  double first;                     // 2 s e^-a
+  double power[kBits];              // r^(2^i)
   __device__ __forceinline__ double operator()(int k) const {
-    return first * (1.0 + exp(-2.0 * k * a)) / (1.0 + exp(-2.0 * (k + 1) * a));
+    double p = 1.0;
+#pragma unroll
+    for (int i = 0; i < kBits; ++i) p *= k >> i & 1 ? power[i] : 1.0;
+    return first * (1.0 + p) / (1.0 + p * power[0]);
   }
 };
+static_assert(kSmallWeights < 1 << SmallWeights::kBits, "powers for every weight");
+
+// a above; cosh a = 1 + e, e small for ill-conditioned matrices
+static double small_arg(double lmin, double lmax) {
+  const double e = 2.0 * lmin / (lmax - lmin);
+  return std::log1p(e + std::sqrt(e * (2.0 + e)));
+}
+
+bool small_steps(int deg, double lmin, double lmax) {
+  return deg <= kSmallWeights || 2.0 * kSmallWeights * small_arg(lmin, lmax) > 37.5;
+}
 
 // Slice sl of a wavefront belongs to the lanes with (lane & 3) == sl & 3: after
 // a row's four lanes have its sum, that one keeps it, so the update of up to
@@ -179,6 +196,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t o = (int64_t)(blockIdx.x % 3) * K + blockIdx.x / 3;  // component, column
+  // the step weights, all before the loop: a global load per step costs more
+  // than the step, and code in the loop that refills them 0.04 us of each
+  double* const ws = small_lds + 2 * nb;
+  for (int i = tid; i < min(deg, kSmallWeights); i += 64 * kSmallWaves) ws[i] = wts(i + 1);
   for (int i = tid; i < nb; i += 64 * kSmallWaves) small_lds[i] = b[3 * (int64_t)i * K + o] * ith;
   const uint32_t ends = P.ends[wave], wide = P.ends[kSmallWaves + wave];
   VT v[QW];
@@ -202,13 +223,9 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
     xo[j] = bo[j] * ith;
     mo[j] = 0.0;
   }
-  // step weights in LDS, kSmallWeights at a time, one per thread
-  double* const ws = small_lds + 2 * nb;
+  __syncthreads();
   for (int k = 0; k < deg; ++k) {
-    if (k % kSmallWeights == 0)
-      for (int i = tid; i < kSmallWeights && k + i < deg; i += 64 * kSmallWaves) ws[i] = wts(k + i + 1);
-    if (k % kSmallWeights == 0) __syncthreads();
-    const double w = ws[k % kSmallWeights];
+    const double w = ws[min(k, kSmallWeights - 1)];
     const uint32_t from = k & 1 ? (uint32_t)nb * 8 : 0;
     double s = 0.0, kept[NS];
     int sl = 0;
@@ -255,7 +272,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
 }
 
 template <int QW, class VT>
-static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, SmallWeights wts,
+static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const SmallWeights& wts,
                            const double* b, double* out, hipStream_t s) {
   const SmallView V{P.ends, P.rows, P.eidx, P.perm, P.slices};
   const size_t lds = (size_t)nb * 16 + (size_t)std::min(deg, kSmallWeights) * 8;
@@ -270,7 +287,7 @@ static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int
 }
 
 template <class VT>
-static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, SmallWeights wts,
+static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const SmallWeights& wts,
                          const double* b, double* out, hipStream_t s) {
   switch (P.quads) {
     case 8: launch_small_q<8>(P, val, nb, K, deg, ith, wts, b, out, s); break;
@@ -282,9 +299,10 @@ static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int d
 void k_cheb_small(const DevMat& M, int K, int deg, double lmin, double lmax, const double* b, double* out,
                   hipStream_t s, bool fp32) {
   const SmallPlan& P = *M.small;
-  // cosh a = 1 + e with e = 2 lmin/(lmax - lmin), small for ill-conditioned matrices
-  const double e = 2.0 * lmin / (lmax - lmin), a = std::log1p(e + std::sqrt(e * (2.0 + e))), ith = 2.0 / (lmax + lmin);
-  const SmallWeights w{a, 2.0 * (1.0 + e) * std::exp(-a)};
+  const double a = small_arg(lmin, lmax), ith = 2.0 / (lmax + lmin);
+  SmallWeights w;
+  w.first = 2.0 * std::cosh(a) * std::exp(-a);
+  for (int i = 0; i < SmallWeights::kBits; ++i) w.power[i] = std::exp(-2.0 * a * (double)(1 << i));
   if (fp32 && M.bval32) launch_small(P, (const float*)M.bval32, (int)M.nb, K, deg, ith, w, b, out, s);
   else launch_small(P, (const double*)M.bval, (int)M.nb, K, deg, ith, w, b, out, s);
 }

@@ -200,13 +200,15 @@ def test_captured_solve_outlives_its_handle(nb):
         pv.csr_free(m)
 
 
-@pytest.mark.parametrize("lo,hi,deg", [(1.0, 3.0, 1500), (1e-3, 1.0, 400), (1e-6, 1.0, 2500), (0.999, 1.0, 3)])
+@pytest.mark.parametrize("lo,hi,deg", [
+    (1.0, 3.0, 1500), (1e-3, 1.0, 400), (1e-6, 1.0, 2500), (0.999, 1.0, 3), (1e-4, 1.0, 8192), (1e-4, 1.0, 8500),
+    (1e-8, 1.0, 8500)])
 def test_small_solve_weights(lo, hi, deg):
-    """The one-launch solve's step weights from their closed form, over the
-    chunks of a long solve and from ill- to well-conditioned bounds, against
-    the recurrence: diagonal systems, whose every entry is one polynomial of
+    """The one-launch solve's step weights from their closed form, up to and
+    beyond the 8192 held, from ill- to well-conditioned bounds (1e-8 with 8500
+    steps: not settled by then, so step by step), against the recurrence: diagonal systems, whose every entry is one polynomial of
     its eigenvalue."""
-    nb = 48
+    nb = 4096 if deg == 8500 else 48                       # 128 KB of LDS, and little
     lam = np.linspace(lo, hi, nb)
     D = sp.kron(sp.diags(lam), sp.identity(3), format="csr")
     th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
