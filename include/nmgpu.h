@@ -518,6 +518,14 @@ int nmg_tiling_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int m
  * eidx[64*quads] and perm[64*quads]; null pointers are skipped. */
 int nmg_node_tiles_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int rows, int cap, int waves, int pack,
                         int64_t *sizes, int32_t *units, int32_t *lists, uint16_t *lrow, uint16_t *eidx, int32_t *perm);
+/* The layout of the one-launch Chebyshev solves (nmgpu_small.hip) of a node
+ * pattern, computed on the host only (no reference counterpart; no device use).
+ * sizes[2]: quads and slices per wavefront of 16 (0: the pattern does not fit).
+ * Then with ends[32] (per wavefront the bits of the quads that end a slice; then
+ * those that end one of 16 lanes per row), rows[16*16*slices] (0xffff: none),
+ * eidx[16*64*quads] (nodes; nb: padding) and perm[16*64*quads] (entries; -1). */
+int nmg_small_layout_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int64_t *sizes, uint32_t *ends,
+                          uint16_t *rows, uint16_t *eidx, int32_t *perm);
 /* Autotuner (no reference counterpart): times the layouts of mat for K columns
  * on the device, as the fused Chebyshev step of a scalar mass, the fused filter
  * step of 3x3 blocks or the product of a rectangular matrix, and keeps the

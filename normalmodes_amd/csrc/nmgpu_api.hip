@@ -3345,6 +3345,14 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
 }
 }  // namespace nmg
 
+// node patterns of the host-only layout entries, as nmg_csr_create checks them
+static void check_pattern(int64_t nb, const int64_t* rp, const int32_t* ci) {
+  NMG_CHECK(nb > 0 && rp && ci && rp[0] == 0, NMG_EINVAL, "null pattern");
+  for (int64_t r = 0; r < nb; ++r) NMG_CHECK(rp[r + 1] >= rp[r], NMG_EINVAL, "row offsets must be non-decreasing");
+  for (int64_t k = 0; k < rp[nb]; ++k)
+    NMG_CHECK(ci[k] >= 0 && ci[k] < nb, NMG_EINVAL, "column index out of range");
+}
+
 extern "C" {
 
 int nmg_csr_autotune(nmg_handle mat, int K, int reps, int fp32, double* seconds, int* kind, int* rows,
@@ -3443,9 +3451,10 @@ int nmg_tiling_host(int64_t nb, const int64_t* rowptr, const int32_t* col, int m
 int nmg_node_tiles_host(int64_t nb, const int64_t* rowptr, const int32_t* col, int rows, int cap, int waves, int pack,
                         int64_t* sizes, int32_t* units, int32_t* lists, uint16_t* lrow, uint16_t* eidx, int32_t* perm) {
   return guarded([&] {
-    NMG_CHECK(nb > 0 && rowptr && col && sizes, NMG_EINVAL, "null pattern");
-    NMG_CHECK(rows > 0 && rows % kSliceRows == 0 && cap > 0 && waves > 0 && (pack == 1 || pack == 2), NMG_EINVAL,
-              "rows must be a multiple of 16, cap and waves positive, pack 1 or 2");
+    check_pattern(nb, rowptr, col);
+    NMG_CHECK(sizes, NMG_EINVAL, "null sizes");
+    NMG_CHECK(rows > 0 && rows % kSliceRows == 0 && cap > 0 && waves > 0 && waves <= 64 && (pack == 1 || pack == 2),
+              NMG_EINVAL, "rows must be a multiple of 16, cap positive, waves 1 to 64, pack 1 or 2");
     HostTiles H;
     const bool ok = tile_layout(nb, rowptr, col, rows, cap, waves, pack, H);
     sizes[0] = ok ? H.ntiles : 0;
@@ -3461,6 +3470,26 @@ int nmg_node_tiles_host(int64_t nb, const int64_t* rowptr, const int32_t* col, i
     if (units) std::memcpy(units, H.un.data(), sizeof(TileUnit) * H.un.size());
     out(lists, H.tcols);
     out(lrow, H.lrow);
+    out(eidx, H.eidx);
+    out(perm, H.perm);
+  });
+}
+
+int nmg_small_layout_host(int64_t nb, const int64_t* rowptr, const int32_t* col, int64_t* sizes, uint32_t* ends,
+                          uint16_t* rows, uint16_t* eidx, int32_t* perm) {
+  return guarded([&] {
+    check_pattern(nb, rowptr, col);
+    NMG_CHECK(sizes, NMG_EINVAL, "null sizes");
+    HostSmall H;
+    const bool ok = small_layout(nb, rowptr, col, H);
+    sizes[0] = ok ? H.quads : 0;
+    sizes[1] = ok ? H.slices : 0;
+    if (!ok) return;
+    auto out = [](auto* to, const auto& v) {
+      if (to) std::memcpy(to, v.data(), sizeof(v[0]) * v.size());
+    };
+    out(ends, H.ends);
+    out(rows, H.rows);
     out(eidx, H.eidx);
     out(perm, H.perm);
   });

@@ -124,7 +124,8 @@ struct TileSet {
 
 // One-launch Chebyshev solves of small scalar-mass systems (nmgpu_small.hip):
 // per wavefront the bits of the quads that end a slice (then those that end one
-// of 16 lanes per row), the rows of its slices (0xffff: none), and each slot's node and matrix entry (-1: padding).
+// of 16 lanes per row), the rows of its slices (0xffff: none), and each slot's
+// node and matrix entry (padding: nb and -1).
 struct HostSmall {
   int quads = 0, slices = 0;  // per wavefront
   std::vector<uint32_t> ends;

@@ -3,7 +3,7 @@
 // Below some 800 (P2) to 1400 (P1) nodes a fused step is nothing but its
 // launch: 2.9-3.9 us for 0.1-0.2 us of work.  M (x) I3 does not couple the
 // three components, so one workgroup takes one component of one column through
-// all steps by itself: b and two iterates in LDS (24 bytes per node), the
+// all steps by itself: two iterates in LDS (16 bytes per node), the
 // matrix in registers (2.5 per slot), one workgroup barrier per step and no
 // communication between workgroups.
 //
@@ -76,7 +76,9 @@ bool small_layout(int64_t nb, const int64_t* rp, const int32_t* ci, HostSmall& H
   H.quads = (most + 7) / 8 * 8;
   H.ends.assign(2 * kSmallWaves, 0);
   H.rows.assign((size_t)kSmallWaves * H.slices * kSliceRows, 0xffff);
-  H.eidx.assign((size_t)kSmallWaves * H.quads * 64, 0);
+  // padding points at the zero behind each iterate: 0 * x of any node would carry
+  // an infinity or NaN into rows that do not touch it
+  H.eidx.assign((size_t)kSmallWaves * H.quads * 64, (uint16_t)nb);
   H.perm.assign((size_t)kSmallWaves * H.quads * 64, -1);
   for (int w = 0; w < kSmallWaves; ++w) {
     int q0 = 0;
@@ -191,16 +193,19 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
                                                                  int deg, double ith, SmallWeights wts,
                                                                  const double* __restrict__ b,
                                                                  double* __restrict__ out) {
-  extern __shared__ double small_lds[];  // two iterates of nb values, then the step weights
+  // two iterates of nb values and a zero each, then the step weights
+  extern __shared__ double small_lds[];
+  const int ld = nb + 1;
   char* const xs = reinterpret_cast<char*>(small_lds);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t o = (int64_t)(blockIdx.x % 3) * K + blockIdx.x / 3;  // component, column
   // the step weights, all before the loop: a global load per step costs more
   // than the step, and code in the loop that refills them 0.04 us of each
-  double* const ws = small_lds + 2 * nb;
+  double* const ws = small_lds + 2 * ld;
   for (int i = tid; i < min(deg, kSmallWeights); i += 64 * kSmallWaves) ws[i] = wts(i + 1);
   for (int i = tid; i < nb; i += 64 * kSmallWaves) small_lds[i] = b[3 * (int64_t)i * K + o] * ith;
+  if (tid < 2) small_lds[tid * ld + nb] = 0.0;
   const uint32_t ends = P.ends[wave], wide = P.ends[kSmallWaves + wave];
   VT v[QW];
   uint32_t id[QW / 2];  // two byte offsets of x
@@ -226,7 +231,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
   __syncthreads();
   for (int k = 0; k < deg; ++k) {
     const double w = ws[min(k, kSmallWeights - 1)];
-    const uint32_t from = k & 1 ? (uint32_t)nb * 8 : 0;
+    const uint32_t from = k & 1 ? (uint32_t)ld * 8 : 0;
     double s = 0.0, kept[NS];
     int sl = 0;
 #pragma unroll
@@ -257,7 +262,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
         }
       }
     }
-    char* const to = xs + ((uint32_t)nb * 8 - from);
+    char* const to = xs + ((uint32_t)ld * 8 - from);
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       const double x = mo[j] + w * (xo[j] - mo[j] + (bo[j] - kept[j]) * ith);
@@ -267,7 +272,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
     }
     __syncthreads();
   }
-  const double* const x = small_lds + (deg & 1 ? nb : 0);
+  const double* const x = small_lds + (deg & 1 ? ld : 0);
   for (int i = tid; i < nb; i += 64 * kSmallWaves) out[3 * (int64_t)i * K + o] = x[i];
 }
 
@@ -275,7 +280,7 @@ template <int QW, class VT>
 static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const SmallWeights& wts,
                            const double* b, double* out, hipStream_t s) {
   const SmallView V{P.ends, P.rows, P.eidx, P.perm, P.slices};
-  const size_t lds = (size_t)nb * 16 + (size_t)std::min(deg, kSmallWeights) * 8;
+  const size_t lds = (size_t)(nb + 1) * 16 + (size_t)std::min(deg, kSmallWeights) * 8;
   const dim3 grid(3 * (unsigned)K), tb(64 * kSmallWaves);
   if (P.slices <= 4)
     hipLaunchKernelGGL((cheb_small_k<QW, 1, VT>), grid, tb, lds, s, V, val, nb, K, deg, ith, wts, b, out);

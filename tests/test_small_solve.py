@@ -10,7 +10,7 @@ import scipy.sparse as sp
 
 from normalmodes_amd import pevsl as pv
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 
 
 def _mass(nb, per_row, seed, long_row=0):
@@ -29,8 +29,62 @@ def _mass(nb, per_row, seed, long_row=0):
     return M
 
 
+def _layout(M):
+    rp, ci = M.indptr.astype(np.int64), M.indices.astype(np.int32)
+    sz, c = np.zeros(2, dtype=np.int64), ctypes
+
+    def call(*out):
+        pv._check(pv._lib().nmg_small_layout_host(
+            c.c_int64(M.shape[0]), *(a.ctypes.data_as(c.c_void_p) for a in (rp, ci, sz)),
+            *(None if o is None else o.ctypes.data_as(c.c_void_p) for o in out)))
+
+    call(None, None, None, None)
+    quads, slices = (int(v) for v in sz)
+    if quads == 0:
+        return None
+    out = (np.zeros(32, np.uint32), np.zeros((16, slices, 16), np.uint16), np.zeros((16, quads, 64), np.uint16),
+           np.zeros((16, quads, 64), np.int32))
+    call(*out)
+    return out
+
+
+@pytest.mark.parametrize("nb,per_row,long_row,fits", [
+    (1, 1, 0, True), (16, 6, 0, True), (17, 6, 0, True), (555, 28, 0, True), (300, 60, 0, True), (700, 40, 400, None),
+    (4096, 3, 0, True), (4097, 3, 0, False), (3000, 40, 0, False)])
+def test_small_layout(nb, per_row, long_row, fits):
+    """The host layout: every row in one place, its entries once each in the
+    slots of its lanes and slice, everything else padding at the zero."""
+    M = _mass(nb, per_row, nb, long_row)
+    L = _layout(M)
+    if fits is not None:
+        assert (L is not None) == fits
+    if L is None:
+        return
+    ends, rows, eidx, perm = L
+    quads = perm.shape[1]
+    assert quads in (8, 16, 24) and rows.shape[1] <= 16
+    pad = perm < 0
+    assert (eidx[pad] == nb).all() and (eidx[~pad] == M.indices[perm[~pad]]).all()
+    assert (np.bincount(perm[~pad], minlength=M.nnz) == 1).all()
+    assert (np.sort(rows[rows != 0xffff]) == np.arange(nb)).all()
+    for w in range(16):
+        last = [q for q in range(32) if ends[w] >> q & 1]
+        assert not ends[16 + w] & ~ends[w] and all(q < quads for q in last)
+        q0 = 0
+        for i, q in enumerate(last):
+            lanes = 16 if ends[16 + w] >> q & 1 else 4
+            for lane in range(64):
+                ks = perm[w, q0:q + 1, lane]
+                r = rows[w, i, lane // lanes * lanes // 4]
+                assert (M.indptr[r] <= ks[ks >= 0]).all() and (ks[ks >= 0] < M.indptr[r + 1]).all() if r != 0xffff \
+                    else (ks < 0).all()
+            q0 = q + 1
+        assert (perm[w, q0:] < 0).all() and (rows[w, len(last):] == 0xffff).all()
+
+
 # (nodes, entries per row): one slot per wavefront, a whole and a broken slice,
 # both sides of each register size (8, 16, 24, 32 quads) and sizes too large
+@gpu
 @pytest.mark.parametrize("nb,per_row,long_row", [
     (1, 1, 0), (15, 6, 0), (16, 6, 0), (17, 6, 0), (555, 28, 0), (614, 15, 0), (700, 40, 400), (1100, 28, 0),
     (2300, 12, 0), (4096, 3, 0), (4097, 3, 0), (3000, 40, 0)])
@@ -96,6 +150,7 @@ def _open(n, m, ch, graphs=False):
     return h
 
 
+@gpu
 @pytest.mark.parametrize("nb", [300, 2300])
 def test_graphs_belong_to_one_solve(nb):
     """A graph captured from one Chebyshev solve is not replayed for another
@@ -146,6 +201,7 @@ class _Hip:
         return call
 
 
+@gpu
 @pytest.mark.parametrize("nb", [300, 2300])
 def test_captured_solve_outlives_its_handle(nb):
     """A caller's own graph of nmg_chebiter_noalloc holds the matrix and the
@@ -200,6 +256,7 @@ def test_captured_solve_outlives_its_handle(nb):
         pv.csr_free(m)
 
 
+@gpu
 @pytest.mark.parametrize("lo,hi,deg", [
     (1.0, 3.0, 1500), (1e-3, 1.0, 400), (1e-6, 1.0, 2500), (0.999, 1.0, 3), (1e-4, 1.0, 8192), (1e-4, 1.0, 8500),
     (1e-8, 1.0, 8500)])
@@ -230,5 +287,36 @@ def test_small_solve_weights(lo, hi, deg):
         # rounding of the iteration itself grows with deg and the condition
         assert err[0] <= 2.0 * err[1] + 1e-15 * min(deg, hi / lo), err
     finally:
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@gpu
+@pytest.mark.parametrize("nb", [200, 900])
+def test_non_finite_stays_in_its_component(nb):
+    """Two systems that do not touch, numbered alternately: an infinity or NaN
+    in the right-hand side of one leaves the other's solution as it is."""
+    M = _mass(nb, 12, nb)
+    two = sp.kron(M, sp.identity(2), format="csr")           # node 2r and 2r + 1: M twice
+    assert _layout(two) is not None
+    D = sp.kron(two, sp.identity(3), format="csr")
+    D.sort_indices()
+    n = D.shape[0]
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    ch = pv.pevsl_setup_chebiter(1.0, 3.0, 9, m)
+    h = _open(n, m, ch)
+    rng = np.random.default_rng(9)
+    even = np.repeat(np.arange(2 * nb) % 2 == 0, 3)
+    try:
+        for K in (1, 2, 4):
+            X = rng.standard_normal((K, n))
+            want = pv.apply_block(h, 2, X)
+            for side, bad in ((even, np.inf), (~even, np.nan)):
+                Y = X.copy()
+                Y[:, side] = bad                             # node 0 (and the last) among them
+                got = pv.apply_block(h, 2, Y)
+                assert (got[:, ~side] == want[:, ~side]).all() and not np.isfinite(got[:, side]).all()
+    finally:
+        pv.pevsl_finish(h)
         pv.pevsl_chebiter_free(ch)
         pv.csr_free(m)
