@@ -515,7 +515,8 @@ int nmg_tiling_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int m
  * fit), quads, list entries, slices per tile, longest list, partial sums of a
  * tile.  Then with units[8*waves*tiles] (list, nodes, row0, own, q0, nq,
  * slice, part | parts << 8 | slot << 16), lists, lrow[16*slices],
- * eidx[64*quads] and perm[64*quads]; null pointers are skipped. */
+ * eidx[64*quads] (list places; 65535: padding, which reads a zero) and
+ * perm[64*quads] (entries; -1: padding); null pointers are skipped. */
 int nmg_node_tiles_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int rows, int cap, int waves, int pack,
                         int64_t *sizes, int32_t *units, int32_t *lists, uint16_t *lrow, uint16_t *eidx, int32_t *perm);
 /* The layout of the one-launch Chebyshev solves (nmgpu_small.hip) of a node

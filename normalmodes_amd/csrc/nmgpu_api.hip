@@ -3470,7 +3470,8 @@ int nmg_node_tiles_host(int64_t nb, const int64_t* rowptr, const int32_t* col, i
     if (units) std::memcpy(units, H.un.data(), sizeof(TileUnit) * H.un.size());
     out(lists, H.tcols);
     out(lrow, H.lrow);
-    out(eidx, H.eidx);
+    if (eidx)
+      for (size_t i = 0; i < H.eidx.size(); ++i) eidx[i] = (uint16_t)(H.eidx[i] - 1);
     out(perm, H.perm);
   });
 }

@@ -101,7 +101,7 @@ struct HostTiles {
   std::vector<TileUnit> un;          // per tile and wavefront
   std::vector<int32_t> tcols;        // node lists, ascending
   std::vector<uint16_t> lrow;        // row of each slice place within its tile (0xffff: none)
-  RawVec<uint16_t> eidx;             // entries' list places
+  RawVec<uint16_t> eidx;             // entries' list places + 1 (padding: 0)
   RawVec<int32_t> perm;              // entry of each slot (-1: padding)
 };
 struct TilePlan {

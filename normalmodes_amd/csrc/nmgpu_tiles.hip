@@ -49,6 +49,11 @@
 
 namespace nmg {
 
+// Place 0 of a tile's nodes in LDS is a node of zeros, which the slots that pad
+// a row's quads point at: 0 * x of some node would carry an infinity or NaN
+// into rows that do not touch it.
+constexpr uint16_t kTileZero = 0;
+
 TilePlan::~TilePlan() {
   for (void* p : {(void*)un, (void*)tcols, (void*)lrow, (void*)eidx, (void*)perm})
     if (p) (void)hipFree(p);
@@ -73,7 +78,7 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
   const int64_t nblk = (nb + rows - 1) / rows;
   int64_t longest = 0;
   for (int64_t r = 0; r < nb; ++r) longest = std::max(longest, rp[r + 1] - rp[r]);
-  if (longest + 1 > cap || cap > 65535 || rp[nb] > (int64_t)1 << 28 || nb > (int64_t)1 << 28) return false;
+  if (longest + 1 > cap || cap > 65534 || rp[nb] > (int64_t)1 << 28 || nb > (int64_t)1 << 28) return false;
   // cut every aligned run of `rows` rows where its node list would pass cap
   struct Cut {
     int64_t r0, r1;
@@ -207,7 +212,7 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
       const Cut& c = *cut[t];
       for (size_t i = 0; i < c.nodes.size(); ++i) local[c.nodes[i]] = (uint16_t)i;
       for (int64_t s = t * spt; s < (t + 1) * spt; ++s) {
-        std::fill_n(H.eidx.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, (uint16_t)0);
+        std::fill_n(H.eidx.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, kTileZero);
         std::fill_n(H.perm.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, -1);
         for (int j = 0; j < kSliceRows; ++j) {
           if (H.lrow[s * kSliceRows + j] == 0xffff) continue;
@@ -223,7 +228,7 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
             by[cl].pop_back();
             const int64_t quad = sd[s].x + e / 4, l = j * 4 + e % 4;
             // the two indices of a pair of quads side by side
-            H.eidx[pack == 2 ? quad / 2 * 128 + 2 * l + quad % 2 : quad * 64 + l] = local[ci[k]];
+            H.eidx[pack == 2 ? quad / 2 * 128 + 2 * l + quad % 2 : quad * 64 + l] = (uint16_t)(local[ci[k]] + 1);
             H.perm[quad * 64 + l] = (int32_t)k;
           }
         }
@@ -412,7 +417,6 @@ struct TEpiFilter {
 };
 
 typedef double d2 __attribute__((ext_vector_type(2)));
-typedef double d2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -481,7 +485,7 @@ template <int KG, bool BSR, class VT, class XT, class Epi>
 __global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
     TileView T, const VT* __restrict__ val, const XT* __restrict__ x, int K, int lgroups, int part_off, Epi epi,
     int flags) {
-  extern __shared__ double2 tile_lds[];
+  extern __shared__ double2 tile_lds[];  // a node of zeros (kTileZero), the tile's nodes, partial sums
   char* const xs = reinterpret_cast<char*>(tile_lds);
   double* const partial = reinterpret_cast<double*>(xs + part_off);
   constexpr int NW = BSR ? 8 : 16, TB = 64 * NW;
@@ -511,6 +515,8 @@ __global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
 #pragma unroll
   for (int u = 0; u < QD; ++u)
     if (u < ne) en[u].load(val, T.eidx, e0 + u, lane);
+  char* const xn = xs + NB;
+  if (tid < NB / 4) reinterpret_cast<int*>(xs)[tid] = 0;
   // stage x: each wavefront a run of the tile's units, the list read once per
   // SB units and handed to the lanes across the wavefront
   {
@@ -530,7 +536,7 @@ __global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
       if constexpr (UB == 16) {
 #pragma unroll
         for (int u = 0; u < SB; ++u)
-          if (b0 + u * 64 < total) lds_load16(at(x + c0, src[u]), xs + (size_t)(b0 + u * 64) * 16);
+          if (b0 + u * 64 < total) lds_load16(at(x + c0, src[u]), xn + (size_t)(b0 + u * 64) * 16);
       } else {
         using U = std::conditional_t<UB == 8, double, float>;
         U v[SB];
@@ -538,7 +544,7 @@ __global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
         for (int u = 0; u < SB; ++u) v[u] = *reinterpret_cast<const U*>(at(x + c0, src[u]));
 #pragma unroll
         for (int u = 0; u < SB; ++u)
-          if (b0 + u * 64 + lane < total) reinterpret_cast<U*>(xs)[b0 + u * 64 + lane] = v[u];
+          if (b0 + u * 64 + lane < total) reinterpret_cast<U*>(xn)[b0 + u * 64 + lane] = v[u];
       }
     }
   }
@@ -556,10 +562,10 @@ __global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
   __syncthreads();
 
   double y[3] = {0.0, 0.0, 0.0};
-  auto madd = [&](const VT* m, const char* xn) {
+  auto madd = [&](const VT* m, const char* xe) {
     double xv[3];
 #pragma unroll
-    for (int p = 0; p < 3; ++p) xv[p] = (double)*reinterpret_cast<const XT*>(xn + p * SEG);
+    for (int p = 0; p < 3; ++p) xv[p] = (double)*reinterpret_cast<const XT*>(xe + p * SEG);
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       if constexpr (BSR) {
@@ -642,7 +648,7 @@ __global__ __launch_bounds__(BSR ? 512 : 1024, BSR ? 4 : 8) void node_tile_k(
 #pragma unroll
     for (int p = 0; p < NP; ++p)
       if (comp(p) < 3) {
-        const double own = (double)*reinterpret_cast<const XT*>(xc + (un.own + lr) * NB + comp(p) * SEG);
+        const double own = (double)*reinterpret_cast<const XT*>(xc + (un.own + lr + 1) * NB + comp(p) * SEG);
         epi.store(o, l0 + comp(p) * K, c0 + col, sum[p], own, pre[p]);
       }
   }
@@ -654,7 +660,9 @@ static void launch_tile(const DevMat& M, const TilePlan& P, const VT* v, const X
   while ((KG << lg) < K) ++lg;
   const TileView T{P.un, P.tcols, P.lrow, P.eidx};
   constexpr int NP = KG == 4 ? 3 : (KG == 2 ? 2 : 1);
-  size_t lds = ((size_t)P.max_nodes * 3 * KG * sizeof(XT) + 1023) / 1024 * 1024;
+  // the node of zeros, then the nodes, staged in whole wavefronts of 16 bytes a lane
+  size_t lds = 3 * KG * sizeof(XT) + ((size_t)P.max_nodes * 3 * KG * sizeof(XT) + 1023) / 1024 * 1024;
+  lds = (lds + 15) / 16 * 16;
   int part_off = 0;  // no slice is split
   if (P.max_extra > 0) {
     part_off = (int)lds;

@@ -103,6 +103,15 @@ def test_layout_forms_the_product(nb, rows, cap, waves, pack, long_row):
     assert (abs(_product(M, L, x, pack) - M @ x) <= bound).all()
 
 
+@pytest.mark.parametrize("pack", [1, 2])
+def test_padding_reads_no_node(pack):
+    """Slots that pad a row point at the zero, not at a node of the list."""
+    L = _layout(_pattern(300, 7), 96, 700, 16, pack)
+    pad = L["perm"].reshape(-1, 64) < 0
+    idx = L["eidx"].reshape(-1, 64) if pack == 1 else L["eidx"].reshape(-1, 64, 2).transpose(0, 2, 1).reshape(-1, 64)
+    assert pad.any() and (idx[pad] == 0xffff).all() and (idx[~pad] < L["max_nodes"]).all()
+
+
 def test_layout_refuses_what_a_tile_cannot_hold():
     M = _pattern(200, 3, long_row=150)
     assert _layout(M, 64, 100, 16, 2) is None          # one row references more than 100 nodes
@@ -155,6 +164,44 @@ def test_products(kind, nb, long_row):
             X = rng.standard_normal((K, n))
             tol = (2 * (most + 3) * eps + 2.0 ** -24) * (aD @ abs(X).T).T + 1e-300
             assert (abs(pv.apply_block(h, 0, X) - (D @ X.T).T) <= tol).all(), K
+    finally:
+        if h:
+            pv.pevsl_finish(h)
+        if ch:
+            pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,nb", [("mass", 2100), ("mass", 21000), ("bsr", 1100), ("bsr", 66000)])
+def test_non_finite_x(kind, nb):
+    """Infinities and NaN in x reach the rows that reference them and no others:
+    finite results to the bound, the others of the same kind as scipy's."""
+    M = _pattern(nb, nb)
+    D, m = _handles(M, kind, 5)
+    n = D.shape[0]
+    h = ch = None
+    try:
+        ch = pv.pevsl_setup_chebiter(0.5, 1.5, 1, m)
+        h = pv.pevsl_start(0)
+        pv.pevsl_setprobsizes(h, n, n, -1)
+        pv.pevsl_setbmv(h, m)
+        pv.pevsl_setbsol_chebiter(h, 2, ch)
+        pv.pevsl_setamv(h, m)
+        rng = np.random.default_rng(12)
+        most, eps = int(np.diff(D.indptr).max()), np.finfo(float).eps
+        for K in (1, 2, 4, 16):
+            X = rng.standard_normal((K, n))
+            for c in range(K):
+                X[c, rng.integers(0, n, 40)] = rng.choice([np.inf, -np.inf, np.nan], 40)
+            X[:, 0] = np.nan
+            with np.errstate(invalid="ignore"):
+                want, scale = (D @ X.T).T, (abs(D) @ np.where(np.isfinite(X), abs(X), 0.0).T).T
+            got = pv.apply_block(h, 1, X)
+            ok = np.isfinite(want)
+            assert not ok.all() and (np.isfinite(got) == ok).all()
+            assert (abs(got[ok] - want[ok]) <= 2 * (most + 3) * eps * scale[ok] + 1e-300).all()
+            assert np.array_equal(got[~ok], want[~ok], equal_nan=True)
     finally:
         if h:
             pv.pevsl_finish(h)
