@@ -507,6 +507,11 @@ int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int 
  * then with trp[ntiles+1], tcp[ntiles+1], tcols[tcp[ntiles]], lcol[nnz]. */
 int nmg_tiling_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int max_nodes, int64_t *ntiles,
                     int *max_used, int64_t *trp, int64_t *tcp, int32_t *tcols, uint16_t *lcol);
+/* What K-column products and Chebyshev solves with mat run on now (no reference
+ * counterpart).  tiles: 0 row kernels or a layout set for K, 1 or 2 the node tiles
+ * (which of their two cuts), on 16-byte aligned vectors; one_launch: 1 if solves
+ * run in one launch (in the default mode, unrefined). */
+int nmg_product_route(nmg_handle mat, int K, int fp32_vectors, int *tiles, int *one_launch);
 /* The node tiles of a node pattern (nb rows, columns < nb) as the LDS-staged
  * products of nmgpu_tiles.hip use them, computed on the host only (no
  * reference counterpart; no device use): tiles of at most `rows` rows (a

@@ -343,16 +343,18 @@ void build_row_groups(DevMat& M, int per_wave) {
 }
 
 void build_tiling(DevMat& M, int K, int max_nodes, int rows_per_wave, int block, int wide) {
-  M.touch();
   int idx = -1;
   for (int i = 0; i < 7; ++i)
     if ((1 << i) == K) idx = i;
   NMG_CHECK(idx >= 0, NMG_EINVAL, "K must be 1, 2, 4, 8, 16, 32 or 64");
-  delete M.tiling[idx];
-  M.tiling[idx] = nullptr;
   NMG_CHECK(max_nodes <= 0 || K <= 16, NMG_EINVAL, "LDS tiles are built for K <= 16");
-  M.tiling[idx] = nullptr;
-  if (max_nodes <= 0 || M.layout == L_CSR) return;
+  // a refused tiling leaves the one in use as it is
+  auto use = [&](Tiling* T) {
+    M.touch();
+    delete M.tiling[idx];
+    M.tiling[idx] = T;
+  };
+  if (max_nodes <= 0 || M.layout == L_CSR) return use(nullptr);
   NMG_CHECK((int64_t)M.h_browptr.size() == M.nb + 1, NMG_ESTATE, "no host pattern for tiling");
   HostTiling H;
   compute_tiling(M.nb, M.h_browptr.data(), M.h_bcol.data(), max_nodes, H);
@@ -375,7 +377,7 @@ void build_tiling(DevMat& M, int K, int max_nodes, int rows_per_wave, int block,
   NMG_HIP(hipMemcpy(T->tcp, H.tcp.data(), sizeof(int64_t) * H.tcp.size(), hipMemcpyHostToDevice));
   NMG_HIP(hipMemcpy(T->tcols, H.tcols.data(), sizeof(int32_t) * H.tcols.size(), hipMemcpyHostToDevice));
   NMG_HIP(hipMemcpy(T->lcol, H.lcol.data(), sizeof(uint16_t) * H.lcol.size(), hipMemcpyHostToDevice));
-  M.tiling[idx] = T.release();
+  use(T.release());
 }
 
 DevMat* clone_devmat(const DevMat& S, hipStream_t s) {
@@ -3114,15 +3116,10 @@ int nmg_set_stream_loads(nmg_handle mat, int on) {
 int nmg_set_kernel_map(nmg_handle mat, int group, int K, int rows_per_wave) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
-    M->set_by_hand(K > 0 ? K : 1);
     NMG_CHECK(group == 0 || group == 8 || group == 16 || group == 32 || group == 64, NMG_EINVAL,
               "group must be 0, 8, 16, 32 or 64");
-    M->group = group;
-    M->pipe = 0;
-    M->touch();
-    if (group > 0 || K == 1) build_row_groups(*M, 0);  // the single-column route is set explicitly
+    int idx = -1;
     if (K > 0) {
-      int idx = -1;
       for (int i = 0; i < 7; ++i)
         if ((1 << i) == K) idx = i;
       NMG_CHECK(idx >= 0, NMG_EINVAL, "K must be 1, 2, 4, 8, 16, 32 or 64");
@@ -3130,6 +3127,15 @@ int nmg_set_kernel_map(nmg_handle mat, int group, int K, int rows_per_wave) {
                     rows_per_wave == 8,
                 NMG_EINVAL, "rows per wavefront must be 0, 1, 2, 4 or 8");
       NMG_CHECK(K * std::max(rows_per_wave, 1) <= 64, NMG_EINVAL, "K x rows per wavefront must be <= 64");
+    }
+    // the group and the pipeline are the single column's, whatever K
+    if (group > 0 || K <= 1 || group != M->group || M->pipe > 0) M->set_by_hand(1);
+    if (K > 1) M->set_by_hand(K);
+    M->group = group;
+    M->pipe = 0;
+    M->touch();
+    if (group > 0 || K == 1) build_row_groups(*M, 0);  // the single-column route is set explicitly
+    if (idx >= 0) {
       M->block_map[idx] = rows_per_wave;
       M->wide[idx] = 0;
     }
@@ -3496,14 +3502,24 @@ int nmg_small_layout_host(int64_t nb, const int64_t* rowptr, const int32_t* col,
   });
 }
 
+int nmg_product_route(nmg_handle mat, int K, int fp32_vectors, int* tiles, int* one_launch) {
+  return guarded([&] {
+    DevMat* M = get<DevMat>(mat, K_MAT);
+    NMG_CHECK(K == 1 || K == 2 || K == 4 || K == 8 || K == 16 || K == 32 || K == 64, NMG_EINVAL,
+              "K must be 1, 2, 4, 8, 16, 32 or 64");
+    if (tiles) *tiles = tile_route(*M, K, fp32_vectors ? 4 : 8);
+    if (one_launch) *one_launch = M->small_use(K) && !fp32_vectors ? 1 : 0;
+  });
+}
+
 int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int threads) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
-    M->set_by_hand(K);
     NMG_CHECK(rows_per_wave >= 1 && rows_per_wave <= 8 && K * rows_per_wave <= 64, NMG_EINVAL,
               "bad rows per wavefront");
     NMG_CHECK(max_nodes <= tile_cap_limit(K), NMG_EINVAL, "tile exceeds 64 KB of LDS");
     build_tiling(*M, K, max_nodes, rows_per_wave, threads > 0 ? threads : 1024);
+    M->set_by_hand(K);
     for (int i = 0; i < 5; ++i)
       if ((1 << i) == K) M->wide[i] = 0;
     if (K == 1) {
@@ -3516,10 +3532,10 @@ int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int 
 int nmg_set_tiled_wide(nmg_handle mat, int K, int max_nodes, int lanes) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
-    M->set_by_hand(K);
     NMG_CHECK(K == 2 || K == 4 || K == 8 || K == 16, NMG_EINVAL, "K must be 2, 4, 8 or 16");
     NMG_CHECK(max_nodes * 24 * K <= 64 * 1024, NMG_EINVAL, "tile exceeds 64 KB of LDS");
     build_tiling(*M, K, max_nodes, 1, 1024, max_nodes > 0 ? lanes : 0);
+    M->set_by_hand(K);
     for (int i = 0; i < 5; ++i)
       if ((1 << i) == K) M->wide[i] = 0;
   });
@@ -3528,7 +3544,6 @@ int nmg_set_tiled_wide(nmg_handle mat, int K, int max_nodes, int lanes) {
 int nmg_set_wide(nmg_handle mat, int K, int lanes) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
-    M->set_by_hand(K);
     int idx = -1;
     for (int i = 1; i < 5; ++i)
       if ((1 << i) == K) idx = i;
@@ -3536,6 +3551,7 @@ int nmg_set_wide(nmg_handle mat, int K, int lanes) {
     NMG_CHECK(lanes == 0 || lanes == 4 || lanes == 8 || lanes == 16 || lanes == 32, NMG_EINVAL,
               "lanes per row must be 0, 4, 8, 16 or 32");
     NMG_CHECK(lanes == 0 || M->layout == L_MASS3, NMG_EINVAL, "the wide layout applies to scalar-mass matrices");
+    M->set_by_hand(K);
     M->wide[idx] = lanes;
     M->touch();
   });
@@ -3544,10 +3560,10 @@ int nmg_set_wide(nmg_handle mat, int K, int lanes) {
 int nmg_set_row_pipeline(nmg_handle mat, int lanes, int rows) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
-    M->set_by_hand(1);
     NMG_CHECK(rows == 0 || rows == 2 || rows == 4 || rows == 8, NMG_EINVAL, "rows per lane group must be 0, 2, 4 or 8");
     NMG_CHECK(rows == 0 || lanes == 16 || lanes == 32 || lanes == 64, NMG_EINVAL, "lanes per group must be 16, 32 or 64");
     NMG_CHECK(rows == 0 || M->layout == L_BSR3, NMG_EINVAL, "pipelined rows apply to 3x3-block matrices");
+    M->set_by_hand(1);
     M->pipe = rows;
     if (rows > 0) {  // the single-column products take the lanes-per-row route
       M->group = lanes;
@@ -3561,11 +3577,11 @@ int nmg_set_row_pipeline(nmg_handle mat, int lanes, int rows) {
 int nmg_set_row_groups(nmg_handle mat, int per_wave) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
-    M->set_by_hand(1);
     NMG_CHECK(per_wave == 0 || per_wave == 1 || per_wave == 2 || per_wave == 4 || per_wave == 8, NMG_EINVAL,
               "groups per wavefront must be 0, 1, 2, 4 or 8");
     NMG_CHECK(per_wave == 0 || M->layout != L_CSR, NMG_EINVAL, "row groups apply to the blocked layouts");
     build_row_groups(*M, per_wave);
+    M->set_by_hand(1);
   });
 }
 

@@ -284,6 +284,8 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
 void build_tiles(DevMat& M, hipStream_t s);
 // whether K-column FP64 products take them (no layout set for that width)
 bool tiles_taken(const DevMat& M, int K);
+// 0 none, else 1 + the tile set, for vectors of `size`-byte values
+int tile_route(const DevMat& M, int K, int size);
 // (re)writes the FP32 tile values, and with fp64 (or when new) the FP64 ones
 void fill_tile_values(DevMat& M, hipStream_t s, bool fp64);
 bool k_tile_spmv(int K, const DevMat& M, const double* x, double* y, hipStream_t s, bool fp32);

@@ -673,7 +673,11 @@ static void launch_tile(const DevMat& M, const TilePlan& P, const VT* v, const X
   NMG_HIP(hipGetLastError());
 }
 
-bool tiles_taken(const DevMat& M, int K) { return tile_set(M, K, 8) != nullptr; }
+int tile_route(const DevMat& M, int K, int size) {
+  const TileSet* T = tile_set(M, K, size);
+  return T ? 1 + (int)(T - M.tset) : 0;
+}
+bool tiles_taken(const DevMat& M, int K) { return tile_route(M, K, 8) > 0; }
 
 template <bool BSR, class XT, class Epi>
 static bool tile_product(const DevMat& M, const XT* x, int K, Epi epi, hipStream_t s, bool fp32,

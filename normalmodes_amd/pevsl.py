@@ -582,6 +582,15 @@ def set_row_groups(mat: Handle, per_wave: int):
     _check(_lib().nmg_set_row_groups(_i64(mat), ctypes.c_int(per_wave)))
 
 
+def product_route(mat: Handle, K: int, fp32_vectors: bool = False):
+    """(tiles, one_launch): the node tiles that K-column products take (0: row
+    kernels or a layout set for K), and whether solves run in one launch."""
+    t, o = ctypes.c_int(), ctypes.c_int()
+    _check(_lib().nmg_product_route(_i64(mat), ctypes.c_int(K), ctypes.c_int(int(fp32_vectors)), ctypes.byref(t),
+                                    ctypes.byref(o)))
+    return t.value, bool(o.value)
+
+
 def csr_autotune(mat: Handle, K: int, reps: int = 10, fp32: bool = False):
     s = _d()
     kind, rows, cap, thr = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int()

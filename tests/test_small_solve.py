@@ -320,3 +320,50 @@ def test_non_finite_stays_in_its_component(nb):
         pv.pevsl_finish(h)
         pv.pevsl_chebiter_free(ch)
         pv.csr_free(m)
+
+
+@gpu
+def test_layouts_set_by_hand_come_first():
+    """On a tuned small matrix: a refused layout call changes no route, and a
+    layout set by hand for a width (the single-column map among them, whatever
+    width the call names) turns the one-launch solve of that width off."""
+    D = sp.kron(_mass(600, 14, 600), sp.identity(3), format="csr")
+    D.sort_indices()
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    ch = pv.pevsl_setup_chebiter(1.0, 3.0, 9, m)
+    widths = (1, 2, 4)
+
+    def routes():
+        return [pv.product_route(m, K)[1] for K in widths]
+
+    try:
+        for K in widths:
+            pv.csr_autotune(m, K, 2)
+        assert routes() == [True] * 3
+        for refused in (lambda: pv.set_kernel_map(m, 32, 3, 1), lambda: pv.set_kernel_map(m, 32, 4, 5),
+                        lambda: pv.set_kernel_map(m, 7, 1, 1), lambda: pv.set_kernel_map(m, 0, 2, 64),
+                        lambda: pv.set_tiling(m, 2, 1, 1), lambda: pv.set_tiling(m, 4, 10 ** 6, 1),
+                        lambda: pv.set_tiling(m, 1, 500, 9), lambda: pv.set_tiled_wide(m, 4, 10 ** 6, 4),
+                        lambda: pv.set_tiled_wide(m, 2, 1, 4), lambda: pv.set_wide(m, 2, 5),
+                        lambda: pv.set_row_pipeline(m, 16, 2), lambda: pv.set_row_groups(m, 3)):
+            with pytest.raises(pv.PevslError):
+                refused()
+            assert routes() == [True] * 3
+        x = np.random.default_rng(1).standard_normal(D.shape[0])
+        tuned = pv.pevsl_chebiter(2, x, ch)
+        pv.set_kernel_map(m, 32, 4, 2)
+        assert routes() == [False, True, False]
+        hand = pv.pevsl_chebiter(2, x, ch)
+        assert np.linalg.norm(hand - tuned) <= 1e-13 * np.linalg.norm(tuned)
+        pv.set_kernel_map(m, 0, 4, 0)
+        pv.set_row_groups(m, 0)
+        pv.set_tiling(m, 1, 0)
+        assert routes() == [True] * 3
+        pv.set_wide(m, 2, 8)
+        assert routes() == [True, False, True]
+        pv.set_wide(m, 2, 0)
+        pv.set_row_groups(m, 2)
+        assert routes() == [False, True, True]
+    finally:
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
