@@ -362,6 +362,7 @@ def test_layouts_set_by_hand_come_first():
         pv.set_wide(m, 2, 8)
         assert routes() == [True, False, True]
         pv.set_wide(m, 2, 0)
+        pv.set_kernel_map(m, 0, 2, 0)                      # the tuner's rows per wavefront go too
         pv.set_row_groups(m, 2)
         assert routes() == [False, True, True]
     finally:
