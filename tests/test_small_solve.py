@@ -356,6 +356,7 @@ def test_layouts_set_by_hand_come_first():
         hand = pv.pevsl_chebiter(2, x, ch)
         assert np.linalg.norm(hand - tuned) <= 1e-13 * np.linalg.norm(tuned)
         pv.set_kernel_map(m, 0, 4, 0)
+        pv.set_kernel_map(m, 0, 1, 0)                      # what the tuner chose for one column, too
         pv.set_row_groups(m, 0)
         pv.set_tiling(m, 1, 0)
         assert routes() == [True] * 3
