@@ -507,6 +507,13 @@ int nmg_set_tiling(nmg_handle mat, int K, int max_nodes, int rows_per_wave, int 
  * then with trp[ntiles+1], tcp[ntiles+1], tcols[tcp[ntiles]], lcol[nnz]. */
 int nmg_tiling_host(int64_t nb, const int64_t *rowptr, const int32_t *col, int max_nodes, int64_t *ntiles,
                     int *max_used, int64_t *trp, int64_t *tcp, int32_t *tcols, uint16_t *lcol);
+/* The device memory that the node tiles of mat may take, beside the matrix (no
+ * reference counterpart): -1 (default) no limit, 0 no tiles.  Tiles are a second
+ * copy of the values in their own order, scalar masses mostly two; where they do
+ * not fit the limit or the device, products run on the row kernels.  Tiles in
+ * place, or refused before, are built again within the limit; copies
+ * (nmg_set_amv_dad) take it over. */
+int nmg_set_tile_memory(nmg_handle mat, int64_t bytes);
 /* What K-column products and Chebyshev solves with mat run on now (no reference
  * counterpart).  tiles: 0 row kernels or a layout set for K, 1 or 2 the node tiles
  * (which of their two cuts), on 16-byte aligned vectors; one_launch: 1 if solves

@@ -418,7 +418,10 @@ DevMat* clone_devmat(const DevMat& S, hipStream_t s) {
     if (S.tiling[i])
       build_tiling(*M, 1 << i, S.tiling[i]->cap, S.tiling[i]->rows_per_wave, S.tiling[i]->block, S.tiling[i]->wide);
   if (S.rgroups) build_row_groups(*M, S.rgroups->per_wave);
-  for (int i = 0; i < 2; ++i) M->tset[i].plan = S.tset[i].plan;  // in use once build_tiles has filled the values
+  // the tiles' pattern, in use once build_tiles has put the values in place
+  for (int i = 0; i < 2; ++i) M->tset[i].plan = S.tset[i].plan;
+  M->tile_state = S.tile_state;
+  M->tile_limit = S.tile_limit;
   return M.release();
 }
 
@@ -2339,11 +2342,18 @@ int nmg_csr_info(nmg_handle mat, int64_t* nrow, int64_t* ncol, int64_t* nnz, int
   });
 }
 
+// M as it is becomes an operator: the tiles that tuning laid out get their values
+static void use_plain(DevMat& M, hipStream_t s) {
+  M.plain = true;
+  if (M.tile_state == TILES_PLANNED) build_tiles(M, s);
+}
+
 int nmg_parcsr_matvec(const double* x, double* y, nmg_handle mat) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
     NMG_CHECK(x && y, NMG_EINVAL, "null vector");
     hipStream_t s = default_stream();
+    use_plain(*M, s);
     DVec dx, dy;
     dx.ensure(M->ncol);
     dy.ensure(M->nrow);
@@ -2393,6 +2403,7 @@ int nmg_set_amv_dad(nmg_handle h, nmg_handle matA, const double* d) {
     NMG_CHECK(d != nullptr, NMG_EINVAL, "null scaling vector");
     for (int64_t i = 0; i < S->n; ++i)
       NMG_CHECK(std::isfinite(d[i]) && d[i] > 0.0, NMG_EINVAL, "scaling vector must be positive");
+    plan_tiles(*M);  // once, for every copy of M
     std::unique_ptr<DevMat> C(clone_devmat(*M, S->s));
     DVec dd;
     dd.ensure(S->n);
@@ -2448,6 +2459,7 @@ int nmg_set_amv(nmg_handle h, nmg_handle mat) {
     Solver* S = get<Solver>(h, K_SOLVER);
     DevMat* M = get<DevMat>(mat, K_MAT);
     NMG_CHECK(S->n > 0 && M->nrow == S->n && M->ncol == S->n, NMG_EINVAL, "operator size mismatch");
+    use_plain(*M, S->s);
     S->amat = M;
     S->adad.reset();
     S->fs.reset();
@@ -2459,6 +2471,7 @@ int nmg_set_bmv(nmg_handle h, nmg_handle matB) {
     Solver* S = get<Solver>(h, K_SOLVER);
     DevMat* M = get<DevMat>(matB, K_MAT);
     NMG_CHECK(S->n > 0 && M->nrow == S->n && M->ncol == S->n, NMG_EINVAL, "B size mismatch");
+    use_plain(*M, S->s);
     S->bmat = M;
   });
 }
@@ -3249,6 +3262,9 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
     M.group = 0;
     build_row_groups(M, 0);
   }
+  // 3x3 blocks are mostly tuned for a scaled copy (nmg_set_amv_dad), which brings
+  // its own values: those made here go again, unless the matrix itself is in use
+  const bool keep = mass || M.plain || M.tset[0].use.load();
   build_tiles(M, s);
   // 7: no layout set -- the node tiles or, for small matrices, the row kernels
   const bool tiles = tiles_taken(M, K);
@@ -3347,6 +3363,7 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
     if (K == 1) M.single_blocked = true;
   }
   NMG_HIP(hipStreamSynchronize(s));
+  if (!keep) drop_tile_values(M);
   return best;
 }
 }  // namespace nmg
@@ -3502,6 +3519,17 @@ int nmg_small_layout_host(int64_t nb, const int64_t* rowptr, const int32_t* col,
   });
 }
 
+int nmg_set_tile_memory(nmg_handle mat, int64_t bytes) {
+  return guarded([&] {
+    DevMat* M = get<DevMat>(mat, K_MAT);
+    NMG_CHECK(bytes >= -1, NMG_EINVAL, "bytes must be >= 0, or -1 for no limit");
+    const bool had = M->tile_state == TILES_REFUSED || M->tset[0].use.load();
+    drop_tiles(*M, TILES_NONE);
+    M->tile_limit = bytes;
+    if (had) build_tiles(*M, default_stream());
+  });
+}
+
 int nmg_product_route(nmg_handle mat, int K, int fp32_vectors, int* tiles, int* one_launch) {
   return guarded([&] {
     DevMat* M = get<DevMat>(mat, K_MAT);
@@ -3591,6 +3619,7 @@ int nmg_bench_spmv(nmg_handle mat, int reps, int fp32, double* seconds, double* 
     NMG_CHECK(reps >= 1, NMG_EINVAL, "reps must be >= 1");
     hipStream_t s = default_stream();
     if (fp32 && !(M->val32 || M->bval32)) make_fp32(*M, s);
+    use_plain(*M, s);
     DVec dx, dy;
     dx.ensure(M->ncol);
     dy.ensure(M->nrow);

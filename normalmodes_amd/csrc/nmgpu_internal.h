@@ -115,8 +115,9 @@ struct TilePlan {
   ~TilePlan();
 };
 
+enum TileState { TILES_NONE = 0, TILES_PLANNED = 1, TILES_REFUSED = 2 };
 struct TileSet {
-  std::shared_ptr<const TilePlan> plan;        // the pattern, shared by copies of a matrix
+  std::shared_ptr<const TilePlan> plan;        // the pattern, shared with the copies of a matrix
   std::atomic<const TilePlan*> use{nullptr};   // set once the values are in place
   double* val = nullptr;                       // values in the tiles' order, and their FP32 copy
   float* val32 = nullptr;
@@ -195,6 +196,10 @@ struct DevMat {
   // node tiles (nmgpu_tiles.hip): [0] for up to 48 staged bytes per node, [1]
   // for more (unset when both are cut alike)
   TileSet tset[2];
+  int tile_state = TILES_NONE;
+  bool plain = false;         // an operator as it is (nmg_set_amv, nmg_set_bmv)
+  int64_t tile_limit = -1;    // device bytes the tiles may take (-1: no limit), and do
+  int64_t tile_bytes = 0;
   // whether K-column products take the node tiles: a layout set or tuned
   // explicitly for that width comes first
   bool tile_use(int K) const {
@@ -281,13 +286,17 @@ void make_fp32(DevMat& M, hipStream_t s);
 // return false when M takes another route
 bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int cap, int waves, int pack,
                  HostTiles& H);
-void build_tiles(DevMat& M, hipStream_t s);
+void plan_tiles(DevMat& M);                  // lays them out; nothing uses them yet
+void build_tiles(DevMat& M, hipStream_t s);  // and puts the values in place
+void drop_tile_values(DevMat& M);            // keeps the plan
+void drop_tiles(DevMat& M, int state);       // state: TILES_NONE or TILES_REFUSED
 // whether K-column FP64 products take them (no layout set for that width)
 bool tiles_taken(const DevMat& M, int K);
 // 0 none, else 1 + the tile set, for vectors of `size`-byte values
 int tile_route(const DevMat& M, int K, int size);
-// (re)writes the FP32 tile values, and with fp64 (or when new) the FP64 ones
-void fill_tile_values(DevMat& M, hipStream_t s, bool fp64);
+// rewrites the FP32 values of tiles in place (where M has FP32 values), and with
+// fp64 the FP64 ones
+void refresh_tile_values(DevMat& M, hipStream_t s, bool fp64);
 bool k_tile_spmv(int K, const DevMat& M, const double* x, double* y, hipStream_t s, bool fp32);
 bool k_tile_cheb_step(int K, const DevMat& M, const double* b, const double* xk, double* xm, double w, double ith,
                       hipStream_t s, bool fp32);

@@ -949,7 +949,7 @@ void scale_devmat(DevMat& M, const double* dl, const double* dr, double sign, hi
   }
   NMG_HIP(hipGetLastError());
   if (M.val32 || M.bval32) make_fp32(M, s);
-  fill_tile_values(M, s, true);
+  refresh_tile_values(M, s, true);
 }
 
 __global__ void csr_diag_k(int64_t nrow, const int64_t* rp, const int32_t* ci, const double* v, double* d) {
@@ -1013,7 +1013,7 @@ void make_fp32(DevMat& M, hipStream_t s) {
     hipLaunchKernelGGL(to_f32_k, dim3(grid_for(nv)), dim3(kBlock), 0, s, nv, M.bval, M.bval32);
   }
   NMG_HIP(hipGetLastError());
-  fill_tile_values(M, s, false);
+  refresh_tile_values(M, s, false);
 }
 
 }  // namespace nmg

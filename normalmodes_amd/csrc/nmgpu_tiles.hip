@@ -59,10 +59,22 @@ TilePlan::~TilePlan() {
     if (p) (void)hipFree(p);
 }
 
-template <class T, class A>
-static T* to_device(const std::vector<T, A>& v) {
+// Device memory of M's tiles, within its limit; throws NMG_ENOMEM.
+template <class T>
+static T* tile_alloc(DevMat& M, size_t count) {
   T* p = nullptr;
-  NMG_HIP(hipMalloc(&p, sizeof(T) * std::max<size_t>(v.size(), 1)));
+  const int64_t bytes = (int64_t)(sizeof(T) * std::max<size_t>(count, 1));
+  if ((M.tile_limit >= 0 && M.tile_bytes + bytes > M.tile_limit) || hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error{NMG_ENOMEM, "no memory for node tiles (" + std::to_string(bytes) + " bytes)"};
+  }
+  M.tile_bytes += bytes;
+  return p;
+}
+
+template <class T, class A>
+static T* to_device(DevMat& M, const std::vector<T, A>& v) {
+  T* p = tile_alloc<T>(M, v.size());
   const hipError_t e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     (void)hipFree(p);
@@ -257,25 +269,53 @@ __global__ void tile_values_k(int64_t nslot, int nv, int64_t nbnz, const int32_t
   }
 }
 
-void fill_tile_values(DevMat& M, hipStream_t s, bool fp64) {
-  const int nv = M.layout == L_BSR3 ? 9 : 1;
+template <class T>
+static void write_values(const DevMat& M, const TilePlan& P, T* out, hipStream_t s) {
+  const int64_t nslot = P.quads * 64;
+  const unsigned grid = (unsigned)std::min<int64_t>(std::max<int64_t>((nslot + 255) / 256, 1), 16384);
+  hipLaunchKernelGGL((tile_values_k<T>), dim3(grid), dim3(256), 0, s, nslot, M.layout == L_BSR3 ? 9 : 1, M.nbnz, P.perm,
+                     M.bval, out, kflags(M));
+  NMG_HIP(hipGetLastError());
+}
+static size_t value_slots(const DevMat& M, const TilePlan& P) {
+  return (size_t)P.quads * 64 * (M.layout == L_BSR3 ? 9 : 1);
+}
+
+void refresh_tile_values(DevMat& M, hipStream_t s, bool fp64) {
   for (TileSet& T : M.tset) {
-    if (!T.plan) continue;
-    const int64_t nslot = T.plan->quads * 64;
-    const size_t cnt = (size_t)std::max<int64_t>(nslot * nv, 1);
-    const unsigned grid = (unsigned)std::min<int64_t>(std::max<int64_t>((nslot + 255) / 256, 1), 16384);
-    if (fp64 || !T.val) {
-      if (!T.val) NMG_HIP(hipMalloc(&T.val, sizeof(double) * cnt));
-      hipLaunchKernelGGL((tile_values_k<double>), dim3(grid), dim3(256), 0, s, nslot, nv, M.nbnz, T.plan->perm, M.bval,
-                         T.val, kflags(M));
+    if (!T.val) continue;
+    if (fp64) write_values(M, *T.plan, T.val, s);
+    if (!M.bval32) continue;
+    if (!T.val32) {
+      try {
+        T.val32 = tile_alloc<float>(M, value_slots(M, *T.plan));
+      } catch (const Error& e) {
+        if (e.code != NMG_ENOMEM) throw;
+        continue;  // the FP64 values serve FP32 products too
+      }
     }
-    if (M.bval32) {
-      if (!T.val32) NMG_HIP(hipMalloc(&T.val32, sizeof(float) * cnt));
-      hipLaunchKernelGGL((tile_values_k<float>), dim3(grid), dim3(256), 0, s, nslot, nv, M.nbnz, T.plan->perm, M.bval,
-                         T.val32, kflags(M));
-    }
-    NMG_HIP(hipGetLastError());
+    write_values(M, *T.plan, T.val32, s);
   }
+}
+
+void drop_tile_values(DevMat& M) {
+  M.touch();
+  for (TileSet& T : M.tset) {
+    T.use.store(nullptr);
+    for (void* p : {(void*)T.val, (void*)T.val32})
+      if (p) (void)hipFree(p);
+    if (T.val) M.tile_bytes -= (int64_t)(sizeof(double) * value_slots(M, *T.plan));
+    if (T.val32) M.tile_bytes -= (int64_t)(sizeof(float) * value_slots(M, *T.plan));
+    T.val = nullptr;
+    T.val32 = nullptr;
+  }
+}
+
+void drop_tiles(DevMat& M, int state) {
+  drop_tile_values(M);
+  for (TileSet& T : M.tset) T.plan.reset();
+  M.tile_bytes = 0;
+  M.tile_state = state;
 }
 
 // Rows of a tile: as few as fill the rounds of 256 tiles, one to a CU, that
@@ -302,41 +342,81 @@ static int tile_rows(const DevMat& M, int most) {
 static int deep_rows(const DevMat& M) { return (int)((M.nb + 128 * kSliceRows - 1) / (128 * kSliceRows) * kSliceRows); }
 static bool deep_tiles(const DevMat& M) { return M.layout == L_MASS3 && M.nb <= 128 * 160; }
 
-void build_tiles(DevMat& M, hipStream_t s) {
-  static std::mutex mu;  // two solvers may set up on one matrix at once
-  std::lock_guard<std::mutex> lk(mu);
-  if (M.layout == L_CSR || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return;
-  if (M.tset[0].use.load()) return;
+// The smallest node count from which K-column products take the tiles (see
+// tile_set), and whether any width can: not with a layout set for each
+static int64_t least_rows(const DevMat& M, int K) {
+  return M.layout == L_BSR3 ? (K == 1 ? 65536 : 1024) : (K >= 8 ? 1 : 2048);
+}
+static bool any_width(const DevMat& M) {
+  for (int K = 1; K <= 64; K *= 2)
+    if (M.nb >= least_rows(M, K) && M.tile_use(K)) return true;
+  return false;
+}
+
+static void plan_tiles_locked(DevMat& M) {
+  if (M.tile_state != TILES_NONE || M.layout == L_CSR || M.nrow != M.ncol ||
+      (int64_t)M.h_browptr.size() != M.nb + 1 || !any_width(M))
+    return;
   const bool bsr = M.layout == L_BSR3;
   const int rows0 = tile_rows(M, bsr ? 96 : 224);
   const int rows1 = bsr ? rows0 : (deep_tiles(M) ? deep_rows(M) : tile_rows(M, M.nb <= 512 * 160 ? 160 : 128));
   const bool two = rows0 != rows1 || (!bsr && rows0 > 128);
   for (int i = 0; i < (two ? 2 : 1); ++i) {
-    TileSet& T = M.tset[i];
-    if (!T.plan) {  // else: the pattern of the matrix this one was copied from
-      HostTiles H;
-      const int cap = i == 0 && two && !deep_tiles(M) ? 1400 : 700;
-      if (!tile_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), i == 0 ? rows0 : rows1, cap, bsr ? 8 : 16,
-                       bsr ? 1 : 2, H))
-        break;
-      auto P = std::make_shared<TilePlan>();
-      P->ntiles = H.ntiles;
-      P->max_nodes = H.max_nodes;
-      P->max_extra = H.max_extra;
-      P->quads = H.quads;
-      P->un = to_device(H.un);
-      P->tcols = to_device(H.tcols);
-      P->lrow = to_device(H.lrow);
-      P->eidx = to_device(H.eidx);
-      P->perm = to_device(H.perm);
-      T.plan = P;
-    }
+    HostTiles H;
+    const int cap = i == 0 && two && !deep_tiles(M) ? 1400 : 700;
+    if (!tile_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), i == 0 ? rows0 : rows1, cap, bsr ? 8 : 16, bsr ? 1 : 2,
+                     H))
+      break;
+    auto P = std::make_shared<TilePlan>();
+    P->ntiles = H.ntiles;
+    P->max_nodes = H.max_nodes;
+    P->max_extra = H.max_extra;
+    P->quads = H.quads;
+    P->un = to_device(M, H.un);
+    P->tcols = to_device(M, H.tcols);
+    P->lrow = to_device(M, H.lrow);
+    P->eidx = to_device(M, H.eidx);
+    P->perm = to_device(M, H.perm);
+    M.tset[i].plan = P;
   }
-  M.touch();
-  fill_tile_values(M, s, false);
-  NMG_HIP(hipStreamSynchronize(s));
-  for (int i = 1; i >= 0; --i)
-    if (M.tset[i].plan) M.tset[i].use.store(M.tset[i].plan.get());
+  M.tile_state = M.tset[0].plan ? TILES_PLANNED : TILES_REFUSED;
+}
+
+// The tiles are an option: where their memory does not suffice the matrix keeps
+// the row kernels, as for patterns that no tile holds.
+template <class F>
+static void or_row_kernels(DevMat& M, F&& f) {
+  bool ok = false;
+  try {
+    f();
+    ok = true;
+  } catch (const std::bad_alloc&) {
+  } catch (const Error& e) {
+    if (e.code != NMG_ENOMEM) throw;
+  }
+  if (!ok) drop_tiles(M, TILES_REFUSED);
+}
+
+static std::mutex tiles_mu;  // two solvers may set up on one matrix at once
+
+void plan_tiles(DevMat& M) {
+  std::lock_guard<std::mutex> lk(tiles_mu);
+  or_row_kernels(M, [&] { plan_tiles_locked(M); });
+}
+
+void build_tiles(DevMat& M, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(tiles_mu);
+  or_row_kernels(M, [&] {
+    plan_tiles_locked(M);
+    if (M.tile_state != TILES_PLANNED || M.tset[0].val) return;
+    for (TileSet& T : M.tset)
+      if (T.plan) T.val = tile_alloc<double>(M, value_slots(M, *T.plan));
+    M.touch();
+    refresh_tile_values(M, s, true);
+    NMG_HIP(hipStreamSynchronize(s));
+    for (int i = 1; i >= 0; --i)
+      if (M.tset[i].plan) M.tset[i].use.store(M.tset[i].plan.get());
+  });
 }
 
 // The tiles for a K-column product on vectors of `size`-byte values, or null
@@ -348,8 +428,7 @@ void build_tiles(DevMat& M, hipStream_t s) {
 // 5.1 : 7.3).
 static const TileSet* tile_set(const DevMat& M, int K, int size) {
   if (M.layout == L_CSR || !M.tile_use(K)) return nullptr;
-  const int64_t least = M.layout == L_BSR3 ? (K == 1 ? 65536 : 1024) : (K >= 8 ? 1 : 2048);
-  if (M.nb < least) return nullptr;
+  if (M.nb < least_rows(M, K)) return nullptr;
   const int i = M.tset[1].use.load() && (deep_tiles(M) ? K >= 16 : std::min(K, 4) * size > 16) ? 1 : 0;
   return M.tset[i].use.load() ? &M.tset[i] : nullptr;
 }

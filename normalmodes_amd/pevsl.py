@@ -582,6 +582,11 @@ def set_row_groups(mat: Handle, per_wave: int):
     _check(_lib().nmg_set_row_groups(_i64(mat), ctypes.c_int(per_wave)))
 
 
+def set_tile_memory(mat: Handle, nbytes: int = -1):
+    """Device memory that the node tiles of mat may take (-1: no limit, 0: none)."""
+    _check(_lib().nmg_set_tile_memory(_i64(mat), ctypes.c_int64(nbytes)))
+
+
 def product_route(mat: Handle, K: int, fp32_vectors: bool = False):
     """(tiles, one_launch): the node tiles that K-column products take (0: row
     kernels or a layout set for K), and whether solves run in one launch."""

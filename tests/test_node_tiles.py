@@ -253,3 +253,88 @@ def test_chebyshev_steps(nb, long_row):
         if ch:
             pv.pevsl_chebiter_free(ch)
         pv.csr_free(m)
+
+
+def _solver(n, m, ch):
+    h = pv.pevsl_start(0)
+    pv.pevsl_setprobsizes(h, n, n, -1)
+    pv.pevsl_setbmv(h, m)
+    pv.pevsl_setbsol_chebiter(h, 2, ch)
+    pv.pevsl_setamv(h, m)
+    return h
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,nb", [("mass", 21000), ("bsr", 3000)])
+def test_tiles_that_do_not_fit(kind, nb):
+    """Where the tiles' memory does not suffice, set-up succeeds and products run
+    on the row kernels: no tiles, part of their tables, all but the last, and
+    room for the FP64 values but not for their FP32 copy."""
+    M = _pattern(nb, nb)
+    D, m = _handles(M, kind, 5)
+    n, K = D.shape[0], 4
+    h = ch = None
+    X = np.random.default_rng(2).standard_normal((K, n))
+    want, scale = (D @ X.T).T, (abs(D) @ abs(X).T).T
+    tol = 2 * (int(np.diff(D.indptr).max()) + 3) * np.finfo(float).eps * scale + 1e-300
+    try:
+        pv.set_tile_memory(m, 0)
+        ch = pv.pevsl_setup_chebiter(0.5, 1.5, 1, m)
+        h = _solver(n, m, ch)
+
+        def check(tiles):
+            assert (pv.product_route(m, K)[0] > 0) == tiles
+            assert (abs(pv.apply_block(h, 1, X) - want) <= tol).all()
+
+        check(False)
+        lo, hi = 0, 1 << 30
+        while hi - lo > 1:                                  # the least memory that holds them
+            mid = (lo + hi) // 2
+            pv.set_tile_memory(m, mid)
+            lo, hi = (lo, mid) if pv.product_route(m, K)[0] else (mid, hi)
+        for limit, tiles in ((hi, True), (hi - 1, False), (hi // 2, False), (1 << 12, False), (hi, True)):
+            pv.set_tile_memory(m, limit)
+            check(tiles)
+        pv.pevsl_set_precision(h, pv.FP32_FILTER)           # no room for FP32 values
+        got = pv.apply_block(h, 0, X)
+        assert (abs(got - want) <= tol + 2.0 ** -24 * scale).all()
+        pv.set_tile_memory(m, -1)
+        assert pv.product_route(m, K)[0] > 0
+    finally:
+        if h:
+            pv.pevsl_finish(h)
+        if ch:
+            pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@pytest.mark.gpu
+def test_tuned_source_of_a_scaled_copy():
+    """Tuning a 3x3-block matrix leaves it without tile values (a scaled copy
+    brings its own); they are there once the matrix itself is an operator.  The
+    copy's products see the scaling, and the source's do not."""
+    nb, K = 2000, 4
+    D, m = _handles(_pattern(nb, 4), "bsr", 6)
+    n = D.shape[0]
+    rng = np.random.default_rng(3)
+    d, X = rng.uniform(0.5, 2.0, n), rng.standard_normal((K, n))
+    h, g = pv.pevsl_start(0), pv.pevsl_start(0)
+    try:
+        for s in (h, g):
+            pv.pevsl_setprobsizes(s, n, n, -1)
+        pv.csr_autotune(m, 1, 2)
+        assert pv.product_route(m, K)[0] == 0
+        pv.pevsl_setamv_dad(h, m, d)
+        assert pv.product_route(m, K)[0] == 0
+        pv.pevsl_setamv(g, m)
+        assert pv.product_route(m, K)[0] > 0
+        eps = 2 * (int(np.diff(D.indptr).max()) + 5) * np.finfo(float).eps
+        for s, e in ((h, d), (g, np.ones(n))):
+            want, scale = e * (D @ (e * X).T).T, e * (abs(D) @ (e * abs(X)).T).T
+            assert (abs(pv.apply_block(s, 0, X) - want) <= eps * scale + 1e-300).all()
+        pv.csr_autotune(m, 2, 2)                            # in use: the values stay
+        assert pv.product_route(m, K)[0] > 0
+    finally:
+        pv.pevsl_finish(h)
+        pv.pevsl_finish(g)
+        pv.csr_free(m)
