@@ -142,7 +142,8 @@ void DevMat::release() {
     t.use.store(nullptr);
     t.plan.reset();
     dfree(t.val);
-    dfree(t.val32);
+    float* v32 = t.val32.exchange(nullptr);
+    dfree(v32);
   }
 }
 DevMat::~DevMat() { release(); }
@@ -381,6 +382,7 @@ void build_tiling(DevMat& M, int K, int max_nodes, int rows_per_wave, int block,
 }
 
 DevMat* clone_devmat(const DevMat& S, hipStream_t s) {
+  std::lock_guard<std::recursive_mutex> lk(S.mu);
   std::unique_ptr<DevMat> M(new DevMat());
   M->nrow = S.nrow;
   M->ncol = S.ncol;
@@ -2344,6 +2346,7 @@ int nmg_csr_info(nmg_handle mat, int64_t* nrow, int64_t* ncol, int64_t* nnz, int
 
 // M as it is becomes an operator: the tiles that tuning laid out get their values
 static void use_plain(DevMat& M, hipStream_t s) {
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
   M.plain = true;
   if (M.tile_state == TILES_PLANNED) build_tiles(M, s);
 }
@@ -2508,14 +2511,14 @@ int nmg_set_precision(nmg_handle h, int mode) {
       // B~ is well conditioned (kappa ~ 15 at P2): its FP32 values cost the
       // B-solve ~1e-7 relative.  FP32 stiffness values (NMG_FP32_FILTER_A)
       // perturb the low modes by ~eps32 lambda_max / lambda instead
-      make_fp32(*S->bsol->mat, S->s);
+      ensure_fp32(*S->bsol->mat, S->s);
       if (mode == NMG_FP32_FILTER_A) {
         if (S->fs) {
           for (DevMat* M : {S->fs->Ad, S->fs->E, S->fs->ET, S->fs->cp->mat})
-            if (!(M->val32 || M->bval32)) make_fp32(*M, S->s);
+            ensure_fp32(*M, S->s);
         } else {
           DevMat& A = const_cast<DevMat&>(S->A());
-          if (!(A.val32 || A.bval32)) make_fp32(A, S->s);
+          ensure_fp32(A, S->s);
         }
       }
       NMG_HIP(hipStreamSynchronize(S->s));
@@ -3386,7 +3389,7 @@ int nmg_csr_autotune(nmg_handle mat, int K, int reps, int fp32, double* seconds,
               "K must be 1, 2, 4, 8, 16, 32 or 64");
     NMG_CHECK(reps >= 1, NMG_EINVAL, "reps must be >= 1");
     hipStream_t s = default_stream();
-    if (fp32 && !M->bval32) make_fp32(*M, s);
+    if (fp32) ensure_fp32(*M, s);
     TuneResult r = tune_matrix(*M, K, reps, fp32 != 0, s);
     M->touch();
     if (seconds) *seconds = r.seconds;
@@ -3406,7 +3409,7 @@ int nmg_bench_block_chebstep(nmg_handle cheb, int K, int reps, int fp32, double*
     NMG_CHECK(fp32 >= 0 && fp32 <= 2, NMG_EINVAL, "fp32 must be 0 (FP64), 1 (FP32 values) or 2 (and FP32 vectors)");
     DevMat* M = C->mat;
     hipStream_t s = default_stream();
-    if (fp32 && !(M->val32 || M->bval32)) make_fp32(*M, s);
+    if (fp32) ensure_fp32(*M, s);
     const int64_t nk = M->nrow * K;
     const double th = 0.5 * (C->lmax + C->lmin);
     DVec b, xk, xm;
@@ -3618,7 +3621,7 @@ int nmg_bench_spmv(nmg_handle mat, int reps, int fp32, double* seconds, double* 
     DevMat* M = get<DevMat>(mat, K_MAT);
     NMG_CHECK(reps >= 1, NMG_EINVAL, "reps must be >= 1");
     hipStream_t s = default_stream();
-    if (fp32 && !(M->val32 || M->bval32)) make_fp32(*M, s);
+    if (fp32) ensure_fp32(*M, s);
     use_plain(*M, s);
     DVec dx, dy;
     dx.ensure(M->ncol);
@@ -3845,10 +3848,7 @@ int nmg_chebiter_set_refine(nmg_handle cheb, int passes, int inner_deg) {
     Cheb* C = get<Cheb>(cheb, K_CHEB);
     NMG_CHECK(passes == 0 || (passes >= 1 && passes <= 8 && inner_deg >= 1 && inner_deg <= 10000), NMG_EINVAL,
               "passes must be 0 (off) or 1..8 with an inner degree >= 1");
-    if (passes > 0 && !(C->mat->val32 || C->mat->bval32)) {
-      make_fp32(*C->mat, default_stream());
-      NMG_HIP(hipStreamSynchronize(default_stream()));
-    }
+    if (passes > 0) ensure_fp32(*C->mat, default_stream());
     C->gen = next_layout_gen();
     C->refine = passes;
     C->inner_deg = passes > 0 ? inner_deg : 0;
@@ -3861,7 +3861,7 @@ int nmg_chebiter_set_refine(nmg_handle cheb, int passes, int inner_deg) {
 int nmg_chebiter_info(nmg_handle cheb, int fp32, int* persistent, int* grid, int* lds_bytes) {
   return guarded([&] {
     Cheb* C = get<Cheb>(cheb, K_CHEB);
-    if (fp32 && !(C->mat->val32 || C->mat->bval32)) make_fp32(*C->mat, default_stream());
+    if (fp32) ensure_fp32(*C->mat, default_stream());
     const int saved = C->mode;
     C->mode = 1;
     const PersistPlan* P = C->persistent(fp32 != 0);
@@ -3878,7 +3878,7 @@ int nmg_bench_bsolve(nmg_handle cheb, int reps, int fp32, double* seconds, doubl
     NMG_CHECK(reps >= 1, NMG_EINVAL, "reps must be >= 1");
     DevMat* M = C->mat;
     hipStream_t s = default_stream();
-    if (fp32 && !(M->val32 || M->bval32)) make_fp32(*M, s);
+    if (fp32) ensure_fp32(*M, s);
     const int64_t n = M->nrow;
     DVec b, x, t;
     b.ensure(n);
@@ -3897,7 +3897,7 @@ int nmg_bench_chebstep(nmg_handle cheb, int reps, int fp32, double* seconds, dou
     NMG_CHECK(reps >= 1, NMG_EINVAL, "reps must be >= 1");
     DevMat* M = C->mat;
     hipStream_t s = default_stream();
-    if (fp32 && !(M->val32 || M->bval32)) make_fp32(*M, s);
+    if (fp32) ensure_fp32(*M, s);
     const int64_t n = M->nrow;
     DVec b, xk, xm;
     b.ensure(n);

@@ -6,6 +6,7 @@
 #include <atomic>
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -120,7 +121,7 @@ struct TileSet {
   std::shared_ptr<const TilePlan> plan;        // the pattern, shared with the copies of a matrix
   std::atomic<const TilePlan*> use{nullptr};   // set once the values are in place
   double* val = nullptr;                       // values in the tiles' order, and their FP32 copy
-  float* val32 = nullptr;
+  std::atomic<float*> val32{nullptr};
 };
 
 // One-launch Chebyshev solves of small scalar-mass systems (nmgpu_small.hip):
@@ -155,8 +156,13 @@ struct DevMat {
   // mapping below; captured HIP graphs of products on this matrix are keyed
   // on it, so a retuned or re-tiled matrix is never replayed with stale
   // kernels or freed buffers
-  uint64_t gen = next_layout_gen();
+  std::atomic<uint64_t> gen{next_layout_gen()};
   void touch() { gen = next_layout_gen(); }
+  // held by what solvers in several threads may do to a matrix they share:
+  // setting up solves, tiles and FP32 values.  Products take no lock: what they
+  // read is published once it is in place.  (Scaling and layout calls want the
+  // matrix to themselves.)
+  mutable std::recursive_mutex mu;
   int layout = L_CSR;
   // CSR (any matrix): rowptr[nrow+1], col[nnz], val[nnz]
   int64_t* rowptr = nullptr;
@@ -281,6 +287,8 @@ void scale_devmat(DevMat& M, const double* dl, const double* dr, double sign, hi
 void diag_devmat(const DevMat& M, double* d, hipStream_t s);
 // refresh float copies of the values
 void make_fp32(DevMat& M, hipStream_t s);
+// float copies in place, for whoever else reads M too
+void ensure_fp32(DevMat& M, hipStream_t s);
 
 // node tiles (nmgpu_tiles.hip): host layout, plan and values; the products
 // return false when M takes another route

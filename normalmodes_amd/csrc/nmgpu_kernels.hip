@@ -1003,6 +1003,7 @@ __global__ void to_f32_k(int64_t n, const double* __restrict__ x, float* __restr
 }
 
 void make_fp32(DevMat& M, hipStream_t s) {
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
   M.touch();
   if (M.layout == L_CSR) {
     if (!M.val32) NMG_HIP(hipMalloc(&M.val32, sizeof(float) * (M.nnz > 0 ? M.nnz : 1)));
@@ -1014,6 +1015,13 @@ void make_fp32(DevMat& M, hipStream_t s) {
   }
   NMG_HIP(hipGetLastError());
   refresh_tile_values(M, s, false);
+}
+
+void ensure_fp32(DevMat& M, hipStream_t s) {
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
+  if (M.val32 || M.bval32) return;
+  make_fp32(M, s);
+  NMG_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace nmg

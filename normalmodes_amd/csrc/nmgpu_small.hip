@@ -23,7 +23,6 @@
 #include <algorithm>
 #include <cmath>
 #include <memory>
-#include <mutex>
 #include <numeric>
 #include <vector>
 
@@ -133,8 +132,7 @@ static T* upload(const std::vector<T>& v) {
 }
 
 void build_small(DevMat& M) {
-  static std::mutex mu;  // two solves may be set up on one matrix at once
-  std::lock_guard<std::mutex> lk(mu);
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
   if (M.small || M.layout != L_MASS3 || M.nrow != M.ncol || (int64_t)M.h_browptr.size() != M.nb + 1) return;
   HostSmall H;
   if (!small_layout(M.nb, M.h_browptr.data(), M.h_bcol.data(), H)) return;

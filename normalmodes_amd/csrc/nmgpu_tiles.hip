@@ -39,7 +39,6 @@
 #include <algorithm>
 #include <initializer_list>
 #include <memory>
-#include <mutex>
 #include <numeric>
 #include <type_traits>
 #include <vector>
@@ -286,15 +285,20 @@ void refresh_tile_values(DevMat& M, hipStream_t s, bool fp64) {
     if (!T.val) continue;
     if (fp64) write_values(M, *T.plan, T.val, s);
     if (!M.bval32) continue;
-    if (!T.val32) {
+    float* v = T.val32;
+    if (!v) {
       try {
-        T.val32 = tile_alloc<float>(M, value_slots(M, *T.plan));
+        v = tile_alloc<float>(M, value_slots(M, *T.plan));
       } catch (const Error& e) {
         if (e.code != NMG_ENOMEM) throw;
         continue;  // the FP64 values serve FP32 products too
       }
     }
-    write_values(M, *T.plan, T.val32, s);
+    write_values(M, *T.plan, v, s);
+    if (!T.val32) {
+      NMG_HIP(hipStreamSynchronize(s));
+      T.val32 = v;
+    }
   }
 }
 
@@ -302,7 +306,7 @@ void drop_tile_values(DevMat& M) {
   M.touch();
   for (TileSet& T : M.tset) {
     T.use.store(nullptr);
-    for (void* p : {(void*)T.val, (void*)T.val32})
+    for (void* p : {(void*)T.val, (void*)T.val32.load()})
       if (p) (void)hipFree(p);
     if (T.val) M.tile_bytes -= (int64_t)(sizeof(double) * value_slots(M, *T.plan));
     if (T.val32) M.tile_bytes -= (int64_t)(sizeof(float) * value_slots(M, *T.plan));
@@ -397,15 +401,13 @@ static void or_row_kernels(DevMat& M, F&& f) {
   if (!ok) drop_tiles(M, TILES_REFUSED);
 }
 
-static std::mutex tiles_mu;  // two solvers may set up on one matrix at once
-
 void plan_tiles(DevMat& M) {
-  std::lock_guard<std::mutex> lk(tiles_mu);
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
   or_row_kernels(M, [&] { plan_tiles_locked(M); });
 }
 
 void build_tiles(DevMat& M, hipStream_t s) {
-  std::lock_guard<std::mutex> lk(tiles_mu);
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
   or_row_kernels(M, [&] {
     plan_tiles_locked(M);
     if (M.tile_state != TILES_PLANNED || M.tset[0].val) return;
@@ -774,7 +776,8 @@ static bool tile_product(const DevMat& M, const XT* x, int K, Epi epi, hipStream
     else if (K == 2) launch_tile<2, BSR>(M, *T->plan, v, x, K, epi, s);
     else launch_tile<4, BSR>(M, *T->plan, v, x, K, epi, s);
   };
-  if (fp32 && T->val32) go((const float*)T->val32);
+  const float* v32 = fp32 ? T->val32.load() : nullptr;
+  if (v32) go(v32);
   else go((const double*)T->val);
   return true;
 }

@@ -338,3 +338,61 @@ def test_tuned_source_of_a_scaled_copy():
         pv.pevsl_finish(h)
         pv.pevsl_finish(g)
         pv.csr_free(m)
+
+
+@pytest.mark.gpu
+def test_solvers_of_several_threads_share_a_matrix():
+    """Solvers in four threads set up solves, tiles and FP32 values of one matrix
+    at the same time and work with them at once."""
+    import threading
+    nb, deg, lo, hi = 6000, 6, 1.0, 3.0
+    M = (_pattern(nb, 8) * 0.02 + sp.identity(nb) * 2.0).tocsr()
+    M.sort_indices()
+    A, a = _handles(_pattern(1500, 9), "bsr", 5)
+    D, m = _handles(M, "mass", 5)
+    n, na = D.shape[0], A.shape[0]
+    th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
+    eps, go, failed = 2.0 ** -23, threading.Barrier(4), []
+
+    def ref(b):
+        xm, xk, w = np.zeros_like(b), b / th, 2.0
+        for _ in range(deg):
+            w = 1.0 / (1.0 - w / (4.0 * sg * sg))
+            xm, xk = xk, xm + w * (xk - xm + (b - D @ xk) / th)
+        return xk
+
+    def work(i):
+        try:
+            rng = np.random.default_rng(i)
+            X, Y, d = rng.standard_normal((4, n)), rng.standard_normal((4, na)), rng.uniform(0.5, 2.0, na)
+            want, wanta = ref(X.T).T, d * (A @ (d * Y).T).T
+            go.wait()
+            ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+            h, g = _solver(n, m, ch), pv.pevsl_start(0)
+            pv.pevsl_set_geneig(h)
+            pv.pevsl_setprobsizes(g, na, na, -1)
+            pv.pevsl_setamv_dad(g, a, d)
+            if i % 2:
+                pv.pevsl_set_precision(h, pv.FP32_FILTER)
+            for _ in range(3):
+                got, gota = pv.apply_block(h, 2, X), pv.apply_block(g, 0, Y)
+                # FP32 values: 2^-24 each, at most doubled by the recurrence
+                assert np.linalg.norm(got - want) <= (eps if i % 2 else 1e-13) * np.linalg.norm(want)
+                assert np.linalg.norm(gota - wanta) <= 1e-13 * np.linalg.norm(wanta)
+            pv.pevsl_finish(h)
+            pv.pevsl_finish(g)
+            pv.pevsl_chebiter_free(ch)
+        except BaseException as e:  # noqa: BLE001 - reported below
+            failed.append((i, e))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    try:
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert not failed, failed
+        assert pv.product_route(m, 4)[0] > 0 and pv.product_route(a, 4)[0] == 0
+    finally:
+        pv.csr_free(m)
+        pv.csr_free(a)
