@@ -3375,8 +3375,9 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
 static void check_pattern(int64_t nb, const int64_t* rp, const int32_t* ci) {
   NMG_CHECK(nb > 0 && rp && ci && rp[0] == 0, NMG_EINVAL, "null pattern");
   for (int64_t r = 0; r < nb; ++r) NMG_CHECK(rp[r + 1] >= rp[r], NMG_EINVAL, "row offsets must be non-decreasing");
-  for (int64_t k = 0; k < rp[nb]; ++k)
-    NMG_CHECK(ci[k] >= 0 && ci[k] < nb, NMG_EINVAL, "column index out of range");
+  int64_t bad = 0;
+  for (int64_t k = 0; k < rp[nb]; ++k) bad += ci[k] < 0 || ci[k] >= nb;
+  NMG_CHECK(bad == 0, NMG_EINVAL, "column index out of range");
 }
 
 extern "C" {

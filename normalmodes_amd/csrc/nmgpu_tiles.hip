@@ -36,9 +36,14 @@
 // counted: with 8 wavefronts or spills the same step took 2-4 times as long.  A
 // persistent form with the next tile's x in registers was no faster (137 us at
 // K = 4), nor was an epilogue through LDS with contiguous stores (143 us).
+#include <omp.h>
+
 #include <algorithm>
+#include <atomic>
+#include <cstdlib>
 #include <initializer_list>
 #include <memory>
+#include <new>
 #include <numeric>
 #include <type_traits>
 #include <vector>
@@ -82,6 +87,49 @@ static T* to_device(DevMat& M, const std::vector<T, A>& v) {
   return p;
 }
 
+// The nodes of one thread's current tile with their places.  calloc: of an array
+// over all nodes only the pages around a thread's tiles are ever backed by memory
+// (a hash table of the tile's size took 1.6 times as long to lay out 600k nodes).
+class NodeTable {
+ public:
+  explicit NodeTable(int64_t nb) : slot_((Slot*)std::calloc((size_t)nb, sizeof(Slot)), &std::free) {
+    if (!slot_) throw std::bad_alloc();
+  }
+  void clear() { ++now_; }  // at most a tile per node: never wraps
+  // whether node c is new, and takes `place`
+  bool add(int32_t c, int place) {
+    if (slot_.get()[c].epoch == now_) return false;
+    slot_.get()[c] = Slot{now_, place};
+    return true;
+  }
+  int operator[](int32_t c) const { return slot_.get()[c].place; }  // of a node that is there
+
+ private:
+  struct Slot {
+    uint32_t epoch;
+    int32_t place;
+  };
+  std::unique_ptr<Slot, void (*)(void*)> slot_;
+  uint32_t now_ = 0;
+};
+
+// f(i, thread) for i < n on all threads; std::bad_alloc passes to the caller
+// instead of ending the process at the end of the parallel region
+template <class F>
+static void parallel_for(int64_t n, F&& f) {
+  std::atomic<bool> failed{false};
+#pragma omp parallel for schedule(dynamic, 16)
+  for (int64_t i = 0; i < n; ++i) {
+    if (failed) continue;
+    try {
+      f(i, omp_get_thread_num());
+    } catch (const std::bad_alloc&) {
+      failed = true;
+    }
+  }
+  if (failed) throw std::bad_alloc();
+}
+
 bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int cap, int waves, int pack,
                  HostTiles& H) {
   const int spt = rows / kSliceRows;
@@ -96,40 +144,37 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
     std::vector<int32_t> nodes;
   };
   std::vector<std::vector<Cut>> blk(nblk);
-#pragma omp parallel
-  {
-    std::vector<int64_t> stamp(nb, -1);
+  std::vector<std::unique_ptr<NodeTable>> tables((size_t)omp_get_max_threads());
+  auto table = [&](int thread) -> NodeTable& {
+    if (!tables[thread]) tables[thread].reset(new NodeTable(nb));
+    return *tables[thread];
+  };
+  parallel_for(nblk, [&](int64_t b, int thread) {
+    NodeTable& seen = table(thread);
     std::vector<int32_t> fresh;
-    int64_t id = 0;
-#pragma omp for schedule(dynamic, 16)
-    for (int64_t b = 0; b < nblk; ++b) {
-      const int64_t end = std::min(nb, (b + 1) * rows);
-      Cut cur{b * rows, b * rows, {}};
-      for (int64_t r = b * rows; r < end;) {
-        fresh.clear();
-        auto see = [&](int32_t c) {
-          if (stamp[c] != id) {
-            stamp[c] = id;
-            fresh.push_back(c);
-          }
-        };
-        for (int64_t k = rp[r]; k < rp[r + 1]; ++k) see(ci[k]);
-        see((int32_t)r);  // the row's own x, for the epilogue
-        if ((int64_t)(cur.nodes.size() + fresh.size()) > cap) {
-          std::sort(cur.nodes.begin(), cur.nodes.end());
-          blk[b].push_back(std::move(cur));
-          cur = Cut{r, r, {}};
-          ++id;
-          continue;  // the row opens the next tile
-        }
-        cur.nodes.insert(cur.nodes.end(), fresh.begin(), fresh.end());
-        cur.r1 = ++r;
+    const int64_t end = std::min(nb, (b + 1) * rows);
+    Cut cur{b * rows, b * rows, {}};
+    seen.clear();
+    for (int64_t r = b * rows; r < end;) {
+      fresh.clear();
+      auto see = [&](int32_t c) {
+        if (seen.add(c, 0)) fresh.push_back(c);
+      };
+      for (int64_t k = rp[r]; k < rp[r + 1]; ++k) see(ci[k]);
+      see((int32_t)r);  // the row's own x, for the epilogue
+      if ((int64_t)(cur.nodes.size() + fresh.size()) > cap) {
+        std::sort(cur.nodes.begin(), cur.nodes.end());
+        blk[b].push_back(std::move(cur));
+        cur = Cut{r, r, {}};
+        seen.clear();
+        continue;  // the row opens the next tile
       }
-      std::sort(cur.nodes.begin(), cur.nodes.end());
-      blk[b].push_back(std::move(cur));
-      ++id;
+      cur.nodes.insert(cur.nodes.end(), fresh.begin(), fresh.end());
+      cur.r1 = ++r;
     }
-  }
+    std::sort(cur.nodes.begin(), cur.nodes.end());
+    blk[b].push_back(std::move(cur));
+  });
   std::vector<const Cut*> cut;
   for (auto& v : blk)
     for (auto& c : v) cut.push_back(&c);
@@ -146,8 +191,7 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
   H.tcols.resize(first[nt]);
   std::vector<int2> sd(nt * spt, int2{0, 0});  // per slice {first quad, quads}
   // rows of a tile in order of falling length, 16 to a slice
-#pragma omp parallel for schedule(dynamic, 16)
-  for (int64_t t = 0; t < nt; ++t) {
+  parallel_for(nt, [&](int64_t t, int) {
     const Cut& c = *cut[t];
     std::copy(c.nodes.begin(), c.nodes.end(), H.tcols.begin() + first[t]);
     std::vector<int32_t> ord(c.r1 - c.r0);
@@ -162,7 +206,7 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
         sd[s].y = (nq + pack - 1) / pack * pack;
       }
     }
-  }
+  });
   int64_t q = 0;
   for (auto& s : sd) {
     s.x = (int)q;
@@ -214,38 +258,41 @@ bool tile_layout(int64_t nb, const int64_t* rp, const int32_t* ci, int rows, int
   // Entries of a row in an order that spreads the simultaneous LDS reads of
   // four neighbouring rows over the banks: row i of a slice takes at place e
   // an entry whose node's place in the list is (e + i) mod 4, while it has one
-#pragma omp parallel
-  {
-    std::vector<uint16_t> local(nb, 0);
-    std::vector<int64_t> by[4];
-#pragma omp for schedule(dynamic, 16)
-    for (int64_t t = 0; t < nt; ++t) {
-      const Cut& c = *cut[t];
-      for (size_t i = 0; i < c.nodes.size(); ++i) local[c.nodes[i]] = (uint16_t)i;
-      for (int64_t s = t * spt; s < (t + 1) * spt; ++s) {
-        std::fill_n(H.eidx.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, kTileZero);
-        std::fill_n(H.perm.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, -1);
-        for (int j = 0; j < kSliceRows; ++j) {
-          if (H.lrow[s * kSliceRows + j] == 0xffff) continue;
-          const int64_t r = c.r0 + H.lrow[s * kSliceRows + j];
-          for (auto& b : by) b.clear();
-          for (int64_t k = rp[r + 1] - 1; k >= rp[r]; --k) by[local[ci[k]] & 3].push_back(k);
-          for (int64_t e = 0; e < rp[r + 1] - rp[r]; ++e) {
-            int cl = (int)((e + j) & 3);
-            if (by[cl].empty())
-              for (int b = 0; b < 4; ++b)
-                if (by[b].size() > by[cl].size()) cl = b;
-            const int64_t k = by[cl].back();
-            by[cl].pop_back();
-            const int64_t quad = sd[s].x + e / 4, l = j * 4 + e % 4;
-            // the two indices of a pair of quads side by side
-            H.eidx[pack == 2 ? quad / 2 * 128 + 2 * l + quad % 2 : quad * 64 + l] = (uint16_t)(local[ci[k]] + 1);
-            H.perm[quad * 64 + l] = (int32_t)k;
-          }
+  parallel_for(nt, [&](int64_t t, int thread) {
+    const Cut& c = *cut[t];
+    NodeTable& local = table(thread);
+    local.clear();
+    for (size_t i = 0; i < c.nodes.size(); ++i) local.add(c.nodes[i], (int)i);
+    struct Placed {
+      int32_t k, place;
+    };
+    std::vector<Placed> by[4];
+    for (int64_t s = t * spt; s < (t + 1) * spt; ++s) {
+      std::fill_n(H.eidx.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, kTileZero);
+      std::fill_n(H.perm.begin() + (int64_t)sd[s].x * 64, (int64_t)sd[s].y * 64, -1);
+      for (int j = 0; j < kSliceRows; ++j) {
+        if (H.lrow[s * kSliceRows + j] == 0xffff) continue;
+        const int64_t r = c.r0 + H.lrow[s * kSliceRows + j];
+        for (auto& b : by) b.clear();
+        for (int64_t k = rp[r + 1] - 1; k >= rp[r]; --k) {
+          const int place = local[ci[k]];
+          by[place & 3].push_back(Placed{(int32_t)k, place});
+        }
+        for (int64_t e = 0; e < rp[r + 1] - rp[r]; ++e) {
+          int cl = (int)((e + j) & 3);
+          if (by[cl].empty())
+            for (int b = 0; b < 4; ++b)
+              if (by[b].size() > by[cl].size()) cl = b;
+          const Placed v = by[cl].back();
+          by[cl].pop_back();
+          const int64_t quad = sd[s].x + e / 4, l = j * 4 + e % 4;
+          // the two indices of a pair of quads side by side
+          H.eidx[pack == 2 ? quad / 2 * 128 + 2 * l + quad % 2 : quad * 64 + l] = (uint16_t)(v.place + 1);
+          H.perm[quad * 64 + l] = v.k;
         }
       }
     }
-  }
+  });
   return true;
 }
 

@@ -119,6 +119,41 @@ def test_layout_refuses_what_a_tile_cannot_hold():
     assert _layout(M, 64, 160, 16, 2) is not None
 
 
+_LIMITED = '''
+import ctypes, resource
+import numpy as np
+from normalmodes_amd import pevsl as pv
+lib, p = pv._lib(), lambda a: a.ctypes.data_as(ctypes.c_void_p)
+
+def lay(nb, rp, ci, sz):
+    return lib.nmg_node_tiles_host(ctypes.c_int64(nb), p(rp), p(ci), 128, 700, 16, 2, p(sz), None, None, None, None, None)
+
+nb = 1 << 20
+rp, ci = np.arange(nb + 1, dtype=np.int64), np.arange(nb, dtype=np.int32)
+sz = np.zeros(6, dtype=np.int64)
+assert lay(4096, rp, ci, sz) == 0            # the threads and their heaps are there
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+seen = []
+for mb in list(range(1, 65, 3)) + [1024]:
+    resource.setrlimit(resource.RLIMIT_AS, (used + (mb << 20), resource.RLIM_INFINITY))
+    seen.append(lay(nb, rp, ci, sz))
+print(sorted(set(seen)), seen[0], seen[-1])
+'''
+
+
+def test_layout_without_memory_is_an_error():
+    """Host memory that runs out while tiles are laid out, in one of the threads
+    or outside, is an error of the call (NMG_ENOMEM), not the end of the process."""
+    import subprocess
+    import sys
+    from pathlib import Path
+    r = subprocess.run([sys.executable, "-c", _LIMITED], capture_output=True, text=True, timeout=120,
+                       cwd=Path(__file__).resolve().parent.parent)
+    assert r.returncode == 0, r.stderr[-800:]
+    kinds, first, last = r.stdout.strip().rsplit(" ", 2)
+    assert first != "0" and last == "0" and kinds == f"[{min(int(first), 0)}, {max(int(first), 0)}]", r.stdout
+
+
 def _handles(M, kind, seed):
     """The DoF matrix of a node pattern: mass (x) I3, or random 3x3 blocks."""
     if kind == "mass":
