@@ -393,6 +393,9 @@ int nmg_kernel_probe(nmg_handle h, int which, double *mean_seconds, int64_t *sam
 /* One application of the filter operator of the handle:
  * y = p((A B^-1 - cc)/dd) z (z-space of ChebLanNr) with pol; host vectors. */
 int nmg_filter_apply(nmg_handle h, nmg_handle pol, const double *z, double *y);
+/* The same on K columns at once (X, Y: K vectors of n, one after the other),
+ * column c with pols[c]; the filters share the spectrum's bounds. */
+int nmg_filter_apply_block(nmg_handle h, int K, const nmg_handle *pols, const double *X, double *Y);
 
 /* Mean seconds of one application of the filter to K device-resident
  * columns (K = 1, 2, 4, .., 64), with the solver's current precision, stream

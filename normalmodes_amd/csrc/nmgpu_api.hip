@@ -2971,6 +2971,40 @@ int nmg_filter_apply(nmg_handle h, nmg_handle pol, const double* z, double* y) {
   });
 }
 
+int nmg_filter_apply_block(nmg_handle h, int K, const nmg_handle* pols, const double* X, double* Y) {
+  return guarded([&] {
+    Solver* S = get<Solver>(h, K_SOLVER);
+    NMG_CHECK(pols && X && Y, NMG_EINVAL, "null argument");
+    NMG_CHECK(K == 1 || K == 2 || K == 4 || K == 8 || K == 16 || K == 32 || K == 64, NMG_EINVAL,
+              "K must be 1, 2, 4, 8, 16, 32 or 64");
+    S->check_A();
+    PolyFilter P = *get<PolyFilter>(pols[0], K_POL);
+    for (int c = 1; c < K; ++c) {
+      const PolyFilter* Q = get<PolyFilter>(pols[c], K_POL);
+      NMG_CHECK(Q->cc == P.cc && Q->dd == P.dd, NMG_EINVAL, "the filters of a block share the spectrum's bounds");
+      P.deg = std::max(P.deg, Q->deg);
+    }
+    std::vector<double> mu((size_t)(P.deg + 1) * K, 0.0);  // zero beyond a column's own degree
+    for (int c = 0; c < K; ++c) {
+      const PolyFilter* Q = get<PolyFilter>(pols[c], K_POL);
+      for (int k = 0; k <= Q->deg; ++k) mu[(size_t)k * K + c] = Q->mu[k];
+    }
+    const int64_t n = S->n;
+    setup_work(*S);
+    for (int i = 0; i < 6; ++i) S->bw[i].ensure(n * K);
+    DVec cm, dmu;
+    cm.ensure(n * K);
+    dmu.ensure((int64_t)mu.size());
+    NMG_HIP(hipMemcpyAsync(dmu.p, mu.data(), sizeof(double) * mu.size(), hipMemcpyHostToDevice, S->s));
+    NMG_HIP(hipMemcpyAsync(cm.p, X, sizeof(double) * n * K, hipMemcpyHostToDevice, S->s));
+    k_to_interleaved(n, K, cm.p, n, S->bw[4].p, S->s);
+    block_filter(*S, K, P, dmu.p, S->bw[4].p, S->bw[5].p);
+    k_from_interleaved(n, K, S->bw[5].p, cm.p, n, S->s);
+    NMG_HIP(hipMemcpyAsync(Y, cm.p, sizeof(double) * n * K, hipMemcpyDeviceToHost, S->s));
+    NMG_HIP(hipStreamSynchronize(S->s));
+  });
+}
+
 int nmg_bench_filter(nmg_handle h, nmg_handle pol, int K, int reps, double* seconds) {
   return guarded([&] {
     Solver* S = get<Solver>(h, K_SOLVER);

@@ -390,6 +390,15 @@ def filter_apply(h: Handle, pol: Handle, z):
     return y
 
 
+def filter_apply_block(h: Handle, pols, X):
+    """Column c of X (K x n) filtered with pols[c]."""
+    X = _f64(X)
+    Y = np.empty_like(X)
+    hs = (_i64 * len(pols))(*pols)
+    _check(_lib().nmg_filter_apply_block(_i64(h), ctypes.c_int(X.shape[0]), hs, _p(X, _f64p), _p(Y, _f64p)))
+    return Y
+
+
 def apply(h: Handle, which: int, x):
     """which: 0 A~ (DAD), 1 B~, 2 B-solve."""
     x = _f64(x)

@@ -12,6 +12,11 @@ from normalmodes_amd import pevsl as pv
 _i64p, _i32p, _u16p = (ctypes.POINTER(t) for t in (ctypes.c_int64, ctypes.c_int32, ctypes.c_uint16))
 
 
+# node counts from which K columns of 3x3 blocks, and of scalar masses, take the tiles
+def _on_tiles(kind, nb, K):
+    return nb >= ((65536 if K == 1 else 1024) if kind == "bsr" else (1 if K >= 8 else 2048))
+
+
 def _pattern(nb, seed, band=60, long_row=0):
     """A ragged node pattern: 0 to 30 local columns per row, some rows without
     a diagonal, a few far columns, optionally one row of `long_row` columns."""
@@ -173,8 +178,7 @@ def _handles(M, kind, seed):
     ("mass", 2048, 0), ("mass", 2049, 0), ("mass", 6000, 300), ("mass", 40000, 0), ("mass", 3000, 1500), ("mass", 40, 0),
     ("mass", 20480, 0), ("mass", 20481, 0), ("bsr", 1024, 0), ("bsr", 1025, 300), ("bsr", 30000, 0), ("bsr", 66000, 0)])
 def test_products(kind, nb, long_row):
-    """A x (or B x) on 1 to 64 columns, FP64 and FP32 values; the filter's fused
-    step through it on the same matrix as A~ of a diagonal-mass pencil."""
+    """A x (or B x) on 1 to 64 columns, FP64 and FP32 values."""
     M = _pattern(nb, nb, long_row=long_row)
     D, m = _handles(M, kind, 5)
     n = D.shape[0]
@@ -191,6 +195,8 @@ def test_products(kind, nb, long_row):
         most = int(np.diff(D.indptr).max())
         eps = np.finfo(float).eps
         for K in (1, 2, 4, 8, 16, 32, 64):
+            refused = long_row + 1 >= 1400 or (long_row >= 700 and K * 8 > 16)
+            assert (pv.product_route(m, K)[0] > 0) == (_on_tiles(kind, nb, K) and not refused)
             X = rng.standard_normal((K, n))
             tol = 2 * (most + 3) * eps * (aD @ abs(X).T).T + 1e-300
             assert (abs(pv.apply_block(h, 1, X) - (D @ X.T).T) <= tol).all(), K
@@ -431,3 +437,98 @@ def test_solvers_of_several_threads_share_a_matrix():
     finally:
         pv.csr_free(m)
         pv.csr_free(a)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nb,kind,band,long_row", [
+    (1024, "bsr", 60, 0), (3001, "bsr", 60, 300), (66000, "bsr", 60, 0)])
+def test_filter_steps(nb, kind, band, long_row):
+    """The fused filter step: whole filters of low degree on 1 to 16 columns with
+    a polynomial of its own each, FP64 and FP32 values, against the recurrence
+    in numpy; after non-finite columns, so that a first step that read the work
+    of the last call would show."""
+    M = _pattern(nb, nb + 2, band=band, long_row=long_row)
+    D, m = _handles(M, kind, 5)
+    pv.csr_free(m)
+    D = (D * (1.0 / abs(D).sum(1).max())).tocsr()           # the spectrum lies in [-1, 1]
+    D.sort_indices()
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    n, eps, most = D.shape[0], np.finfo(float).eps, int(np.diff(D.indptr).max())
+    ch = pv.pevsl_setup_chebiter(0.5, 1.5, 1, m)
+    h = _solver(n, m, ch)
+    pols = [pv.pevsl_findpol(np.array([lo, hi, -1.2, 1.1]), 0.8, 0.7)
+            for lo, hi in ((0.2, 1.0), (-0.3, 0.3), (-1.2, -0.4), (0.4, 1.0))]
+    info = [pv.pol_info(p) for p in pols]
+    assert [p.deg for p in info] == [3, 6, 2, 4]
+
+    def ref(p, v, absolute=False):
+        """p(D) v, or the sum of the absolute values that its rounding scales with."""
+        A, c, s = (abs(D), abs(p.cc), 1.0) if absolute else (D, p.cc, -1.0)
+        mu = abs(p.mu) if absolute else p.mu
+        vm, vk, y = np.zeros_like(v), v, mu[0] * v
+        for k in range(1, p.deg + 1):
+            vm, vk = vk, (1.0 if k == 1 else 2.0) / p.dd * (A @ vk + s * c * vk) + s * vm
+            y = y + mu[k] * vk
+        return y
+
+    try:
+        rng = np.random.default_rng(11)
+        for prec, unit in ((pv.FP64, 0.0), (pv.FP32_FILTER_A, 2.0 ** -24)):
+            pv.pevsl_set_precision(h, prec)
+            for K in (1, 2, 4, 8, 16):
+                assert (pv.product_route(m, K)[0] > 0) == _on_tiles(kind, nb, K)
+                X = rng.standard_normal((K, n))
+                mine = [c * 7 % 4 for c in range(K)]        # neighbours differ
+                pv.filter_apply_block(h, [pols[i] for i in mine], np.full((K, n), np.nan))
+                got = pv.filter_apply_block(h, [pols[i] for i in mine], X)
+                for c in range(K):
+                    p = info[mine[c]]
+                    tol = (p.deg + 1) * (2 * (most + 6) * eps + unit) * ref(p, abs(X[c]), True)
+                    assert (abs(got[c] - ref(p, X[c])) <= tol).all(), (prec, K, c)
+            if _on_tiles(kind, nb, 1):                      # the single-vector filter's scalar mu
+                pv.filter_apply(h, pols[0], np.full(n, np.nan))
+                for p, i in zip(pols, info):
+                    x = rng.standard_normal(n)
+                    tol = (i.deg + 1) * (2 * (most + 6) * eps + unit) * ref(i, abs(x), True)
+                    assert (abs(pv.filter_apply(h, p, x) - ref(i, x)) <= tol).all()
+    finally:
+        for p in pols:
+            pv.pevsl_freepol(p)
+        pv.pevsl_finish(h)
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("long_row", [0, 1000, 1398])
+def test_lists_near_the_largest(long_row):
+    """Node lists of up to 1400 nodes: more than 64 KB of LDS at two columns; with
+    a row of more than 700 nodes there is no second cut, and four columns take
+    the first, with up to 134 KB."""
+    nb = 36000
+    M = _pattern(nb, 5, band=1000, long_row=long_row)
+    M = M.tolil()
+    if long_row:                                            # exactly that many, and its own node
+        r = nb // 2
+        M[r, :] = 0.0
+        M[r, np.arange(r, r + long_row)] = 1.0
+    M = M.tocsr()
+    M.eliminate_zeros()
+    M.sort_indices()
+    assert _layout(M, 144, 1400, 16, 2)["max_nodes"] > 1390
+    assert (_layout(M, 144, 700, 16, 2) is None) == (long_row > 0)
+    D, m = _handles(M, "mass", 5)
+    n = D.shape[0]
+    ch = pv.pevsl_setup_chebiter(0.5, 1.5, 1, m)
+    h = _solver(n, m, ch)
+    rng, most = np.random.default_rng(2), int(np.diff(D.indptr).max())
+    try:
+        for K in (1, 2, 4, 8, 16):
+            assert pv.product_route(m, K)[0] == (2 if K >= 4 and not long_row else 1)
+            X = rng.standard_normal((K, n))
+            tol = 2 * (most + 3) * np.finfo(float).eps * (abs(D) @ abs(X).T).T + 1e-300
+            assert (abs(pv.apply_block(h, 1, X) - (D @ X.T).T) <= tol).all(), K
+    finally:
+        pv.pevsl_finish(h)
+        pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)

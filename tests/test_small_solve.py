@@ -83,7 +83,7 @@ def test_small_layout(nb, per_row, long_row, fits):
 
 
 # (nodes, entries per row): one slot per wavefront, a whole and a broken slice,
-# both sides of each register size (8, 16, 24, 32 quads) and sizes too large
+# both sides of each register size (8, 16, 24 quads) and sizes too large
 @gpu
 @pytest.mark.parametrize("nb,per_row,long_row", [
     (1, 1, 0), (15, 6, 0), (16, 6, 0), (17, 6, 0), (555, 28, 0), (614, 15, 0), (700, 40, 400), (1100, 28, 0),
@@ -119,6 +119,7 @@ def test_small_solve(nb, per_row, long_row):
             pv.pevsl_setamv(h, m)
             pv.pevsl_set_geneig(h)
             for K in (1, 2, 4, 16, 64):
+                assert pv.product_route(m, K)[1] == (_layout(M) is not None)
                 X = rng.standard_normal((K, n))
                 want = ref(X.T, deg).T
                 got = pv.apply_block(h, 2, X)
@@ -127,6 +128,7 @@ def test_small_solve(nb, per_row, long_row):
             one = pv.pevsl_chebiter(2, x, ch)
             assert np.linalg.norm(one - ref(x, deg)) <= 1e-13 * np.linalg.norm(one)
             pv.set_kernel_map(m, 32)                       # by hand: step by step
+            assert not pv.product_route(m, 1)[1]
             step = pv.pevsl_chebiter(2, x, ch)
             pv.set_kernel_map(m, 0)
             assert np.linalg.norm(one - step) <= 1e-14 * deg * np.linalg.norm(step)
