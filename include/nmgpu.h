@@ -545,10 +545,9 @@ int nmg_small_layout_host(int64_t nb, const int64_t *rowptr, const int32_t *col,
 /* Autotuner (no reference counterpart): times the layouts of mat for K columns
  * on the device, as the fused Chebyshev step of a scalar mass, the fused filter
  * step of 3x3 blocks or the product of a rectangular matrix, and keeps the
- * fastest: lanes per row, rows per wavefront, for K = 1 row groups and, from
- * 2048 rows and where no node tiles are, LDS tiles with capacities on a
- * geometric ladder up to 64 KB (workgroups of 1024 or 256 threads) and wide
- * rows.  kind: 0 lanes-per-row, 1 rows per wavefront, 2 tiled, 3 row groups, 4 wide,
+ * fastest: lanes per row, rows per wavefront, for K = 1 row groups, and where
+ * no node tiles are wide rows and (from 2048 rows) LDS tiles with capacities on
+ * a geometric ladder up to 64 KB (workgroups of 1024 or 256 threads).  kind: 0 lanes-per-row, 1 rows per wavefront, 2 tiled, 3 row groups, 4 wide,
  * 5 tiled wide (4 and 5: scalar mass, K >= 2), 6 pipelined lanes-per-row
  * (3x3 blocks, K = 1), 7 the default route (node tiles, or the row kernels
  * for small matrices); rows: lanes per row (kinds 0, 4, 5), rows per

@@ -3197,10 +3197,11 @@ int nmg_set_kernel_map(nmg_handle mat, int group, int K, int rows_per_wave) {
 namespace nmg {
 // ---------------------------------------------------------------------------
 // Autotuner of the sparse-product mapping of one matrix for K columns: times
-// the candidate lane layouts on the matrix itself (untiled rows-per-wavefront
-// 1..8; LDS-tiled at tile capacities on a geometric ladder x rows per
-// wavefront 1..8; for K = 1 also the lanes-per-row layout) and keeps the
-// fastest.
+// the default route (node tiles, or the row kernels of small matrices) and the
+// candidate layouts on the matrix itself (rows per wavefront 1..8; for K = 1 also
+// lanes per row, row groups and pipelined rows; without node tiles also the wide
+// layouts and, from 2048 rows, LDS tiles at capacities on a geometric ladder) and
+// keeps the fastest.
 template <class F>
 static double time_launches(hipStream_t s, int reps, F&& f) {
   f();  // warm-up
@@ -3218,8 +3219,9 @@ static double time_launches(hipStream_t s, int reps, F&& f) {
   return ms * 1e-3 / reps;
 }
 
-// the tuner's timing: at least `reps` launches and 0.3 ms of them, the better
-// of two runs (a run of 10 launches of a 3 us kernel mostly times its events)
+// the tuner's timing: `reps` launches, and where those take less than 0.3 ms the
+// better of two runs of 0.3 ms (at most 200 launches): a run of 10 launches of a
+// 3 us kernel mostly times its events
 template <class F>
 static double time_candidate(hipStream_t s, int reps, F&& f) {
   const double t = time_launches(s, reps, f);
@@ -3231,7 +3233,8 @@ struct TuneResult {
   double seconds = 1e30;
   int kind = 0;  // 0 lanes-per-row (K = 1), 1 untiled block, 2 tiled block, 3 row groups (K = 1),
                  // 4 wide (scalar mass, K >= 2), 5 tiled wide (scalar mass, K >= 2),
-                 // 6 pipelined lanes-per-row (BSR3, K = 1)
+                 // 6 pipelined lanes-per-row (BSR3, K = 1), 7 no layout set: the node tiles, or the
+                 // row kernels for small matrices
   int group = 0, rows = 1, cap = 0;
   int64_t ntiles = 0;
   int block = 1024;  // tile workgroup threads
@@ -3254,8 +3257,8 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   k_fill(nk, 0.0, w.p, s);
   k_fill(K, 0.1, mu.p, s);
   // What is timed is what the solver runs: the fused Chebyshev step of a scalar
-  // mass, the fused filter step of 3x3 blocks (the plain product only of
-  // rectangular matrices).  Plain products misjudge layouts whose epilogue
+  // mass, the fused filter step of 3x3 blocks (with its read of v_{k-1}, as all but
+  // a filter's first; the plain product only of rectangular matrices).  Plain products misjudge layouts whose epilogue
   // operands are loaded row by row: at 10.6k DoF one that won as a product took
   // 7.2 us as a Chebyshev step, against 4.0 for the row kernels.
   const bool square = M.nrow == M.ncol, mass = M.layout == L_MASS3;
@@ -3267,9 +3270,9 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
       K == 1 ? k_cheb_step(M, z.p, a, b, 1.0, 0.1, s, fp32) : k_block_cheb_step(K, M, z.p, a, b, 1.0, 0.1, s, fp32);
       std::swap(a, b);
     } else if (K == 1) {
-      k_filter_step(M, x.p, z.p, y.p, w.p, 1.0, 1.0, 0.1, true, s, fp32);
+      k_filter_step(M, x.p, z.p, y.p, w.p, 1.0, 1.0, 0.1, false, s, fp32);
     } else {
-      k_block_filter_step(K, M, x.p, z.p, y.p, w.p, mu.p, 1.0, 1.0, true, s, fp32);
+      k_block_filter_step(K, M, x.p, z.p, y.p, w.p, mu.p, 1.0, 1.0, false, s, fp32);
     }
   };
   // The wide layouts (kinds 4 and 5: one entry per lane, the K columns in
@@ -3346,10 +3349,11 @@ static TuneResult tune_matrix(DevMat& M, int K, int reps, bool fp32, hipStream_t
   }
   // Where the node tiles are the default the LDS tiles and the wide layouts are
   // not built: they lost by 10-70% at 51k to 1.9M DoF, and the ladder was most of
-  // the tuner's time (11 s at 1.9M DoF).  Nor are they below 2048 rows, where
-  // every layout takes the 3 us of a launch and the ladder took 0.1 s.  Else:
-  // tile capacities on a geometric ladder from the longest row (a tile must hold
-  // one row) up to 64 KB of LDS per workgroup
+  // the tuner's time (11 s at 1.9M DoF).  Nor are LDS tiles below 2048 rows, where
+  // every layout takes the 3 us of a launch and the ladder took 0.1 s.  What is
+  // left for them are matrices without node tiles: for want of memory, or with a
+  // row of 700 nodes and more (then K <= 2, since a tile must hold one row).  Tile
+  // capacities on a geometric ladder from the longest row up to 64 KB of LDS.
   int64_t longest = 0;
   for (int64_t r = 0; r < M.nb; ++r) longest = std::max(longest, M.h_browptr[r + 1] - M.h_browptr[r]);
   const int limit = K <= 16 && !tiles && blocked && M.nb >= 2048 ? std::min(65535, tile_cap_limit(K)) : 0;  // none beyond K = 16

@@ -8,12 +8,12 @@
 // communication between workgroups.
 //
 // The rows are sorted by length and cut into slices of 16 with four lanes per
-// row (long rows: four with 16 lanes), as in nmgpu_tiles.hip; the slices go to the 16 wavefronts longest first,
-// each to the least loaded.  A step reads x for all of a wavefront's quads
-// eight at a time, adds up each slice, closes it with two DPP additions and
-// updates its rows.  What bounds it is the LDS gather (8 bytes per entry, one
-// CU), so the entries of four neighbouring rows are ordered on the host such
-// that the 16 lanes read together touch different banks where possible.
+// row (long rows: four with 16 lanes), as in nmgpu_tiles.hip; the slices go to
+// the 16 wavefronts longest first, each to the least loaded.  A step reads x for
+// all of a wavefront's quads eight at a time, adds up each slice, closes it with
+// two DPP additions and updates its rows.  For the LDS gather (8 bytes per entry,
+// one CU) the entries of four neighbouring rows are ordered on the host such that
+// the 16 lanes read together touch different banks where possible.
 //
 // Measured, us per step of a 60-step solve (one launch per step in brackets):
 // 115 P2 nodes 0.46 (2.9), 614 P1 nodes 0.91 (2.9), 556 P2 nodes 1.26 (3.2), 1002

@@ -20,16 +20,20 @@
 //
 // Long slices (the vertex rows of P2 meshes hold 65 entries, edge rows 19-27)
 // are split over several wavefronts with partial sums in LDS added in a fixed
-// order, so that no wavefront carries more than about six quads: with one
-// wavefront per slice the longest one set the time of the tile.
+// order, as far as a tile has wavefronts beside one per slice: with one wavefront
+// per slice the longest one set the time of the tile.  On a P2 mesh of 60k nodes
+// the longest wavefront of a tile carries 6 quads at 128 rows, 8 at 160, 10
+// (median; at most 18) at 224, where two can share, and 7 (9) at the stiffness's
+// 96 rows of 8 wavefronts.
 //
-// Measured (FP64 fused Chebyshev step, us; row kernels as the autotuner left
-// them in brackets; one MI355X):
+// Measured (FP64 fused Chebyshev step, us; in brackets the fastest of the row
+// kernels, LDS tiles and wide layouts, as the autotuner picks it without node
+// tiles; one MI355X):
 //   DoF        K = 1         K = 2         K = 4         K = 8         K = 16
-//   51.5k    4.1 (4.6)     4.7 (5.7)     5.7 (8.2)     8.3 (12.5)   15.6 (21.9)
-//   439k    14.7 (19.8)   17.0 (24.5)   24.4 (39.5)   38.0 (84.5)   79.8 (161)
-//   1.90M   52.3 (65.5)   67.7 (276)     107 (184)     213 (541)     460 (956)
-// (the 1.9M-DoF figures in brackets at K = 2, 8, 16 are the untuned ones).  At
+//   51.5k    4.0 (5.2)     4.5 (6.1)     5.5 (9.2)     8.1 (14.3)   12.7 (26.7)
+//   439k    14.8 (20.8)   17.1 (26.0)   24.4 (49.0)   38.8 (91.9)   82.0 (177)
+//   1.90M   50.1 (72.0)   69.1 (109)     108 (229)     215 (486)     456 (954)
+// At
 // 1.9M DoF the step moves 487 MB at K = 4 (counted): 4.5 TB/s, against 5.6 TB/s
 // of a copy of that size.  Loads wider than 8 bytes, lists read once per
 // wavefront and 64 registers (two workgroups of 16 wavefronts per CU) each
@@ -470,11 +474,15 @@ void build_tiles(DevMat& M, hipStream_t s) {
 
 // The tiles for a K-column product on vectors of `size`-byte values, or null
 // for the row kernels: a layout set or tuned explicitly for that width, and
-// matrices too small to pay for the list -> x -> LDS chain of a tile (measured
-// against the row kernels, us: scalar mass 556 nodes K = 1 3.5 : 3.4, K = 4
-// 4.5 : 3.9, K = 8 4.6 : 5.0; 3545 nodes K = 1 3.1 : 4.0, K = 4 4.6 : 5.3;
-// stiffness K = 1 17 180 nodes 9.8 : 8.9, 146k nodes 65 : 73; K = 4 3545 nodes
-// 5.1 : 7.3).
+// matrices too small to pay for the list -> x -> LDS chain of a tile (least_rows).
+// Measured as the tuner does, tiles : row kernels, us.  Scalar mass, Chebyshev
+// step: 859 nodes K = 1 3.2 : 3.0, K = 2 3.4 : 3.4, K = 4 3.6 : 3.6; 2223 nodes
+// 3.3 : 3.6, 3.4 : 3.8, 4.1 : 4.2; K = 8 458 nodes 4.0 : 4.3.  Stiffness, filter
+// step: K = 2 859 nodes 3.6 : 3.6, 2223 4.2 : 4.4, 5235 4.5 : 6.4; K = 4 859 nodes
+// 4.5 : 4.5, 1421 5.1 : 5.4; K = 1 5235 nodes 4.1 : 4.5, 9971 5.1 : 6.0, 18 912
+// 9.9 : 10.0, 45 948 18.1 : 18.9, 67 539 25.7 : 25.6, 103 363 37.9 : 36.8, 146 293
+// 65 : 75.  (So the single column would gain from tiles below 18k nodes too; from
+// there to 100k nodes both are the same within 3%.)
 static const TileSet* tile_set(const DevMat& M, int K, int size) {
   if (M.layout == L_CSR || !M.tile_use(K)) return nullptr;
   if (M.nb < least_rows(M, K)) return nullptr;
