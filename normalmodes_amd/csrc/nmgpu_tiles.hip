@@ -475,14 +475,20 @@ void build_tiles(DevMat& M, hipStream_t s) {
 // The tiles for a K-column product on vectors of `size`-byte values, or null
 // for the row kernels: a layout set or tuned explicitly for that width, and
 // matrices too small to pay for the list -> x -> LDS chain of a tile (least_rows).
-// Measured as the tuner does, tiles : row kernels, us.  Scalar mass, Chebyshev
-// step: 859 nodes K = 1 3.2 : 3.0, K = 2 3.4 : 3.4, K = 4 3.6 : 3.6; 2223 nodes
-// 3.3 : 3.6, 3.4 : 3.8, 4.1 : 4.2; K = 8 458 nodes 4.0 : 4.3.  Stiffness, filter
-// step: K = 2 859 nodes 3.6 : 3.6, 2223 4.2 : 4.4, 5235 4.5 : 6.4; K = 4 859 nodes
-// 4.5 : 4.5, 1421 5.1 : 5.4; K = 1 5235 nodes 4.1 : 4.5, 9971 5.1 : 6.0, 18 912
-// 9.9 : 10.0, 45 948 18.1 : 18.9, 67 539 25.7 : 25.6, 103 363 37.9 : 36.8, 146 293
-// 65 : 75.  (So the single column would gain from tiles below 18k nodes too; from
-// there to 100k nodes both are the same within 3%.)
+// Measured as the tuner does, tiles : the fastest layout without them, us:
+//            stiffness, filter step               scalar mass, Chebyshev step
+//   nodes    K = 1        K = 2        K = 4         K = 1      K = 2      K = 4      K = 8
+//   458      3.6 : 3.3    4.0 : 3.6    5.0 : 4.3    3.1 : 2.9  3.4 : 3.4  3.9 : 3.5  4.0 : 4.3
+//   859      3.7 : 3.3    4.1 : 3.6    5.1 : 4.4    3.3 : 3.0  3.4 : 3.3  4.0 : 3.6  4.1 : 4.3
+//   1421     3.7 : 3.4    4.1 : 4.0    5.1 : 5.4    3.2 : 3.4  3.4 : 3.6  4.0 : 3.9  4.1 : 4.8
+//   2223     3.8 : 3.9    4.2 : 4.5    5.2 : 6.1    3.3 : 3.6  3.4 : 3.8  4.0 : 4.2  4.7 : 5.3
+//   9971     5.0 : 6.1    5.7 : 9.9    7.4 : 14.8   3.6 : 4.4  3.9 : 5.1  4.7 : 7.3  6.4 : 11.0
+//   31 016  14.2 : 14.4  14.9 : 23.4  17.2 : 37.8
+//   67 539  25.6 : 25.7  28.0 : 44.6  31.6 : 71.1
+//   103 363 40.0 : 36.8  43.5 : 66.3  50.6 : 112
+//   146 293 64.8 : 73.9  71.5 : 115   81.8 : 180
+// (So a single column of stiffness would gain from tiles between some 2 000 and
+// 17 000 nodes too; from there to 100 000 neither is ahead throughout.)
 static const TileSet* tile_set(const DevMat& M, int K, int size) {
   if (M.layout == L_CSR || !M.tile_use(K)) return nullptr;
   if (M.nb < least_rows(M, K)) return nullptr;
