@@ -471,6 +471,7 @@ struct Cheb {
   // Chebyshev solve of degree inner_deg with FP32 values and FP32 iterates
   // on the FP64 residual b - B~x of the sum so far, added in FP64
   int refine = 0, inner_deg = 0;
+  const double* wts = nullptr;  // step weights of one-launch solves, the matrix's
   FVec own32;           // inner work (3 n K floats) when the caller brings none
   PersistPlan plan[2];  // FP64 / FP32 values
   bool planned[2] = {false, false};
@@ -773,10 +774,10 @@ static Solver::GraphKey graph_key(const Solver& S, const Cheb& C, int K, int par
 // buffers of the matrix only, as the step launches do: a graph that captured it
 // stays valid while the matrix lives.
 static bool small_taken(const Cheb& C, int K) {
-  return C.mat->small_use(K) && small_steps(C.deg, C.lmin, C.lmax);
+  return C.wts && C.mat->small_use(K);
 }
 static void small_solve(const Cheb& C, int K, const double* b, double* out, hipStream_t s, bool fp32) {
-  k_cheb_small(*C.mat, K, C.deg, C.lmin, C.lmax, b, out, s, fp32);
+  k_cheb_small(*C.mat, K, C.deg, 2.0 / (C.lmax + C.lmin), C.wts, b, out, s, fp32);
 }
 
 // x ~ B~^{-1} b by the Chebyshev semi-iteration (x_0 = 0, deg products):
@@ -2555,6 +2556,7 @@ int nmg_setup_chebiter(double lmin, double lmax, int deg, nmg_handle mat, nmg_ha
     C->lmin = lmin;
     C->lmax = lmax;
     C->deg = deg;
+    C->wts = small_weights(*M, lmin, lmax, deg);
     *cheb = reg(C.release(), K_CHEB);
   });
 }

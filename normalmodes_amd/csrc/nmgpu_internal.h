@@ -142,6 +142,12 @@ struct SmallPlan {
   int32_t* perm = nullptr;
   ~SmallPlan();
 };
+struct SmallWeights {
+  double lmin = 0, lmax = 0;
+  int deg = 0;
+  double* w = nullptr;
+  ~SmallWeights();
+};
 
 // Process-wide source of layout generations (unique across matrices, so a
 // matrix freed and re-created at the same address never repeats one).
@@ -222,6 +228,7 @@ struct DevMat {
       if ((1 << i) == K) tuned[i] = false;
   }
   std::shared_ptr<const SmallPlan> small;  // one-launch solves (null: the matrix does not fit, or no solve was set up)
+  std::vector<std::unique_ptr<SmallWeights>> small_w;  // their step weights
   bool small_use(int K) const {
     if (!small) return false;
     for (int i = 0; i < 7; ++i)
@@ -313,14 +320,13 @@ bool k_tile_cheb_step32(int K, const DevMat& M, const float* b, const float* xk,
 bool k_tile_filter_step(int K, const DevMat& A, const double* x, const double* vk, double* vkm, double* y,
                         const double* mu, double mu0, double t, double cc, bool first, hipStream_t s, bool fp32);
 
-// one-launch solves of small systems: M.small is set when M fits; x ~ M^-1 b on
-// K interleaved columns by deg steps for the bounds lmin, lmax
+// one-launch solves of small systems: M.small is set when M fits; the step weights
+// w_1 .. w_deg of a solve on [lmin, lmax] (device; null: M does not fit or holds
+// too many, or they change beyond the 8192nd); x ~ M^-1 b on K interleaved columns, ith = 2/(lmax + lmin)
 bool small_layout(int64_t nb, const int64_t* rp, const int32_t* ci, HostSmall& H);
 void build_small(DevMat& M);
-// whether the weights of a solve of that many steps are held or have settled (to
-// rounding) before the last one held: deg <= 8192, or lmax/lmin below 8e5
-bool small_steps(int deg, double lmin, double lmax);
-void k_cheb_small(const DevMat& M, int K, int deg, double lmin, double lmax, const double* b, double* out,
+const double* small_weights(DevMat& M, double lmin, double lmax, int deg);
+void k_cheb_small(const DevMat& M, int K, int deg, double ith, const double* wts, const double* b, double* out,
                   hipStream_t s, bool fp32);
 
 // ---------------------------------------------------------------------------

@@ -21,7 +21,6 @@
 // and step at 614 nodes).  Reading each slice's rows and iterates from LDS at
 // its end took 1.06 us at 614 nodes; 32 quads per wavefront spill (2.7 us).
 #include <algorithm>
-#include <cmath>
 #include <memory>
 #include <numeric>
 #include <vector>
@@ -33,7 +32,7 @@ namespace nmg {
 
 constexpr int kSmallWaves = 16;
 constexpr int kSmallQuads = 24;  // quads per wavefront that the registers hold
-constexpr int kSmallWeights = 8192;  // step weights held in LDS; longer solves repeat the last
+constexpr int kSmallWeights = 8192;  // step weights held; longer solves repeat the last
 
 SmallPlan::~SmallPlan() {
   for (void* p : {(void*)ends, (void*)rows, (void*)eidx, (void*)perm})
@@ -146,6 +145,39 @@ void build_small(DevMat& M) {
   M.small = P;
 }
 
+SmallWeights::~SmallWeights() {
+  if (w) (void)hipFree(w);
+}
+
+// The weights live with the matrix, not with the solve: a graph that captured a
+// solve then holds buffers of its matrix only.  (In the kernel arguments they
+// cost 1.7 us of a 30 us solve; computed in the kernel from w_k = 2 s T_k(s) /
+// T_{k+1}(s) they cost nothing, but their rounding, other than the step kernels',
+// made a filtered Lanczos run whose residuals end just below its target stop
+// with eigenvalues that agree to 4e-12 instead of 1e-13.)
+const double* small_weights(DevMat& M, double lmin, double lmax, int deg) {
+  constexpr size_t kMost = 64;  // bounds and degrees of one matrix; further solves run step by step
+  std::lock_guard<std::recursive_mutex> lk(M.mu);
+  if (!M.small) return nullptr;
+  for (const auto& W : M.small_w)
+    if (W->lmin == lmin && W->lmax == lmax && W->deg == deg) return W->w;
+  if (M.small_w.size() >= kMost) return nullptr;
+  std::vector<double> w(deg);
+  const double sg = (lmax + lmin) / (lmax - lmin);
+  double wk = 2.0;
+  for (int k = 0; k < deg; ++k) w[k] = wk = 1.0 / (1.0 - wk / (4.0 * sg * sg));
+  for (int k = kSmallWeights; k < deg; ++k)
+    if (w[k] != w[kSmallWeights - 1]) return nullptr;  // not settled by then: step by step
+  w.resize(std::min(deg, kSmallWeights));
+  auto W = std::make_unique<SmallWeights>();
+  W->lmin = lmin;
+  W->lmax = lmax;
+  W->deg = deg;
+  W->w = upload(w);
+  M.small_w.push_back(std::move(W));
+  return M.small_w.back()->w;
+}
+
 struct SmallView {
   const uint32_t* ends;
   const uint16_t* rows;
@@ -154,41 +186,13 @@ struct SmallView {
   int slices;
 };
 
-// Step weights of the semi-iteration: the recurrence w_0 = 2, w_k = 1/(1 -
-// w_{k-1}/(4 s^2)), s = (lmax + lmin)/(lmax - lmin), is w_k = 2 s T_k(s)/T_{k+1}(s)
-// (T_k the Chebyshev polynomials), so with s = cosh a and r = e^-2a each weight
-// stands by itself: w_k = 2 s e^-a (1 + r^k)/(1 + r^{k+1}), and a launch needs no
-// buffer of them that would have to outlive it.
-struct SmallWeights {
-  static constexpr int kBits = 14;  // k <= kSmallWeights
-  double first;                     // 2 s e^-a
-  double power[kBits];              // r^(2^i)
-  __device__ __forceinline__ double operator()(int k) const {
-    double p = 1.0;
-#pragma unroll
-    for (int i = 0; i < kBits; ++i) p *= k >> i & 1 ? power[i] : 1.0;
-    return first * (1.0 + p) / (1.0 + p * power[0]);
-  }
-};
-static_assert(kSmallWeights < 1 << SmallWeights::kBits, "powers for every weight");
-
-// a above; cosh a = 1 + e, e small for ill-conditioned matrices
-static double small_arg(double lmin, double lmax) {
-  const double e = 2.0 * lmin / (lmax - lmin);
-  return std::log1p(e + std::sqrt(e * (2.0 + e)));
-}
-
-bool small_steps(int deg, double lmin, double lmax) {
-  return deg <= kSmallWeights || 2.0 * kSmallWeights * small_arg(lmin, lmax) > 37.5;
-}
-
 // Slice sl of a wavefront belongs to the lanes with (lane & 3) == sl & 3: after
 // a row's four lanes have its sum, that one keeps it, so the update of up to
 // four slices runs once, on all 64 lanes, with b and both iterates of a lane's
 // own rows in registers (NS rows for up to 4 NS slices).
 template <int QW, int NS, class VT>
 __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, const VT* __restrict__ val, int nb, int K,
-                                                                 int deg, double ith, SmallWeights wts,
+                                                                 int deg, double ith, const double* __restrict__ wts,
                                                                  const double* __restrict__ b,
                                                                  double* __restrict__ out) {
   // two iterates of nb values and a zero each, then the step weights
@@ -198,10 +202,6 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t o = (int64_t)(blockIdx.x % 3) * K + blockIdx.x / 3;  // component, column
-  // the step weights, all before the loop: a global load per step costs more
-  // than the step, and code in the loop that refills them 0.04 us of each
-  double* const ws = small_lds + 2 * ld;
-  for (int i = tid; i < min(deg, kSmallWeights); i += 64 * kSmallWaves) ws[i] = wts(i + 1);
   for (int i = tid; i < nb; i += 64 * kSmallWaves) small_lds[i] = b[3 * (int64_t)i * K + o] * ith;
   if (tid < 2) small_lds[tid * ld + nb] = 0.0;
   const uint32_t ends = P.ends[wave], wide = P.ends[kSmallWaves + wave];
@@ -226,6 +226,9 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
     xo[j] = bo[j] * ith;
     mo[j] = 0.0;
   }
+  // step weights in LDS: a global load per step costs more than the step
+  double* const ws = small_lds + 2 * ld;
+  for (int i = tid; i < min(deg, kSmallWeights); i += 64 * kSmallWaves) ws[i] = wts[i];
   __syncthreads();
   for (int k = 0; k < deg; ++k) {
     const double w = ws[min(k, kSmallWeights - 1)];
@@ -275,7 +278,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void cheb_small_k(SmallView P, co
 }
 
 template <int QW, class VT>
-static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const SmallWeights& wts,
+static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const double* wts,
                            const double* b, double* out, hipStream_t s) {
   const SmallView V{P.ends, P.rows, P.eidx, P.perm, P.slices};
   const size_t lds = (size_t)(nb + 1) * 16 + (size_t)std::min(deg, kSmallWeights) * 8;
@@ -290,7 +293,7 @@ static void launch_small_q(const SmallPlan& P, const VT* val, int nb, int K, int
 }
 
 template <class VT>
-static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const SmallWeights& wts,
+static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int deg, double ith, const double* wts,
                          const double* b, double* out, hipStream_t s) {
   switch (P.quads) {
     case 8: launch_small_q<8>(P, val, nb, K, deg, ith, wts, b, out, s); break;
@@ -299,15 +302,11 @@ static void launch_small(const SmallPlan& P, const VT* val, int nb, int K, int d
   }
 }
 
-void k_cheb_small(const DevMat& M, int K, int deg, double lmin, double lmax, const double* b, double* out,
+void k_cheb_small(const DevMat& M, int K, int deg, double ith, const double* wts, const double* b, double* out,
                   hipStream_t s, bool fp32) {
   const SmallPlan& P = *M.small;
-  const double a = small_arg(lmin, lmax), ith = 2.0 / (lmax + lmin);
-  SmallWeights w;
-  w.first = 2.0 * std::cosh(a) * std::exp(-a);
-  for (int i = 0; i < SmallWeights::kBits; ++i) w.power[i] = std::exp(-2.0 * a * (double)(1 << i));
-  if (fp32 && M.bval32) launch_small(P, (const float*)M.bval32, (int)M.nb, K, deg, ith, w, b, out, s);
-  else launch_small(P, (const double*)M.bval, (int)M.nb, K, deg, ith, w, b, out, s);
+  if (fp32 && M.bval32) launch_small(P, (const float*)M.bval32, (int)M.nb, K, deg, ith, wts, b, out, s);
+  else launch_small(P, (const double*)M.bval, (int)M.nb, K, deg, ith, wts, b, out, s);
 }
 
 }  // namespace nmg

@@ -263,11 +263,11 @@ def test_captured_solve_outlives_its_handle(nb):
     (1.0, 3.0, 1500), (1e-3, 1.0, 400), (1e-6, 1.0, 2500), (0.999, 1.0, 3), (1e-4, 1.0, 8192), (1e-4, 1.0, 8500),
     (1e-8, 1.0, 8500)])
 def test_small_solve_weights(lo, hi, deg):
-    """The one-launch solve's step weights from their closed form, up to and
-    beyond the 8192 held, from ill- to well-conditioned bounds (1e-8 with 8500
-    steps: not settled by then, so step by step), against the recurrence: diagonal systems, whose every entry is one polynomial of
+    """The one-launch solve's step weights, up to and beyond the 8192 held, from
+    ill- to well-conditioned bounds (1e-8 with 8500 steps: not settled by then, so
+    step by step), against the recurrence: diagonal systems, whose every entry is one polynomial of
     its eigenvalue."""
-    nb = 4096 if deg == 8500 else 48                       # 128 KB of LDS, and little
+    nb = 4096 if deg == 8500 else 48
     lam = np.linspace(lo, hi, nb)
     D = sp.kron(sp.diags(lam), sp.identity(3), format="csr")
     th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
@@ -370,4 +370,29 @@ def test_layouts_set_by_hand_come_first():
         assert routes() == [False, True, True]
     finally:
         pv.pevsl_chebiter_free(ch)
+        pv.csr_free(m)
+
+
+@gpu
+def test_many_bounds_on_one_matrix():
+    """A matrix keeps the weights of 64 different solves, those set up again
+    counting once; further ones run step by step.  All follow the recurrence."""
+    D = sp.kron(_mass(200, 10, 3), sp.identity(3), format="csr")
+    D.sort_indices()
+    m = pv.csr_create(D.indptr, D.indices, D.data)
+    b, lo, deg = np.random.default_rng(1).standard_normal(D.shape[0]), 1.0, 9
+    try:
+        for i in range(80):
+            hi = 3.0 + 1e-3 * i
+            th, sg = 0.5 * (lo + hi), (lo + hi) / (hi - lo)
+            xm, xk, w = np.zeros_like(b), b / th, 2.0
+            for _ in range(deg):
+                w = 1.0 / (1.0 - w / (4.0 * sg * sg))
+                xm, xk = xk, xm + w * (xk - xm + (b - D @ xk) / th)
+            for _ in range(2):
+                ch = pv.pevsl_setup_chebiter(lo, hi, deg, m)
+                x = pv.pevsl_chebiter(2, b, ch)
+                pv.pevsl_chebiter_free(ch)
+                assert np.linalg.norm(x - xk) <= 1e-13 * np.linalg.norm(xk), i
+    finally:
         pv.csr_free(m)
